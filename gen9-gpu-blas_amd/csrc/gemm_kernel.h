@@ -21,6 +21,7 @@
 //   each XCD a contiguous range, and tiles are ordered in groups of GM tile rows so an XCD's L2 shares A and B panels.
 #pragma once
 #include "internal.h"
+#include <type_traits>
 
 namespace g9 {
 
@@ -80,21 +81,29 @@ template <class S> struct GemmParams {
     const void *A, *B;
     void *C;
     long long lda, ldb, ldc, sA, sB, sC;
-    int M, N, K, tiles_m, tiles_n, vec_c;
+    int M, N, K, tiles_m, tiles_n;
     S alpha, beta;
     // split K (count = 1 only): slice z = blockIdx.y covers k = z·kper .. +kper and writes its unscaled partial sums
     // to P + z·M·N (row stride N, accumulator type S); a reduction kernel then forms alpha·Σ + beta·C
     S *P;
-    int kper, vec_p;
+    int kper;
     int kpair = 0;   // KLIM: the second half of the dispatch order reversed (see the tile mapping)
 };
 
+// 16 bytes at an address aligned to the element type only: one global_load_dwordx4 either way (the GPU serves it at
+// any element alignment, at the aligned rate when the address is aligned).
+template <class T> __device__ __forceinline__ u32x4 load16u(const T *p) {
+    typedef T TV __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+    const TV v = *reinterpret_cast<const TV *>(p);
+    return __builtin_bit_cast(u32x4, v);
+}
+
 // 16 bytes (V elements) of row r, columns c .. c+V-1 of a row-major matrix X (R valid rows, Cc valid columns, row
-// stride ld); zero outside the valid region. VEC: X and ld are 16-byte aligned, so whole chunks load as one vector.
-template <class T, bool VEC>
+// stride ld); zero outside the valid region.
+template <class T>
 __device__ __forceinline__ u32x4 load16(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
     constexpr int V = 16 / sizeof(T);
-    if (VEC && r < R && c + V <= Cc) return *reinterpret_cast<const u32x4 *>(X + (long long)r * ld + c);
+    if (r < R && c + V <= Cc) return load16u(X + (long long)r * ld + c);
     union { u32x4 v; T e[V]; } u;
 #pragma unroll
     for (int e = 0; e < V; e++) u.e[e] = (r < R && c + e < Cc) ? X[(long long)r * ld + c + e] : T(0);
@@ -127,7 +136,7 @@ template <> __device__ __forceinline__ void transpose<double>(const u32x4 *in, u
 // KC: the operand is stored k-contiguous (element (mn, k) at X[mn·ld + k]); otherwise mn-contiguous
 // (element (mn, k) at X[k·ld + mn]) and transposed in registers on the way to LDS.
 constexpr int ROWB = 144;   // LDS bytes per tile row: 128 of data + 16 of padding
-template <class T, int RT, int NT, bool KC, bool VEC>
+template <class T, int RT, int NT, bool KC>
 struct Stage {
     static constexpr int V = 16 / (int)sizeof(T);
     // k-contiguous: N16 chunks per thread. Transposed: NB V×V blocks per thread; when the tile has fewer blocks than
@@ -140,16 +149,48 @@ struct Stage {
     static_assert(KC || NBLK % NT == 0 || NT % NBLK == 0, "transposed blocks must divide over the threads");
     u32x4 r[N16];
 
-    // CHECK = false: the whole tile lies inside the matrix (interior tile, full k-step) and X is 16-byte aligned,
-    // so every chunk is one unconditional vector load.
-    template <bool CHECK>
-    __device__ __forceinline__ void load(const T *__restrict__ X, long long ld, int MN, int K, int mn0, int k0, int tid) {
+    // Unchecked loads of full k-steps. org: the tile's origin (wave-uniform), off: this thread's byte offsets from it,
+    // step: bytes per k-step of BK·KG. Rows (starts of chunks) past the matrix's end are moved back onto the last one,
+    // whose values no stored element uses; a chunk that straddles the end of an mn-contiguous row reads on into the
+    // next row, so a k-step loaded this way must not hold the last k unless the tile lies inside the matrix, and ld
+    // must be at least V - 1. The offsets are 32-bit: ok() bounds the row stride.
+    static constexpr int NOFF = KC ? N16 : NB;
+    const char *org;
+    unsigned off[NOFF];
+    long long step;
+    static __device__ __forceinline__ bool ok(long long ld) {
+        return (KC || ld >= V - 1) && (KC ? RT : 128 / (int)sizeof(T)) * ld * (long long)sizeof(T) < (1LL << 31);
+    }
+    __device__ __forceinline__ void init(const T *__restrict__ X, long long ld, int MN, int mn0, int k0, int kstep, int tid) {
+        org = reinterpret_cast<const char *>(KC ? X + (long long)mn0 * ld + k0 : X + (long long)k0 * ld + mn0);
+        step = (KC ? (long long)kstep : kstep * ld) * (long long)sizeof(T);
+#pragma unroll
+        for (int i = 0; i < NOFF; i++) {
+            const int id = i * NT + tid;
+            if constexpr (KC) {
+                off[i] = (unsigned)(min(id >> 3, MN - 1 - mn0) * (int)(ld * sizeof(T)) + (id & 7) * 16);
+            } else {
+                const int lo = id & 31, mb = (lo & 3) + 4 * (id >> 5), kb = lo >> 2;
+                off[i] = (unsigned)(kb * V * (int)(ld * sizeof(T)) + min(mb * V, (MN - 1 - mn0) / V * V) * (int)sizeof(T));
+            }
+        }
+    }
+    __device__ __forceinline__ void load(long long ld) {   // the next full k-step
+        if (PART && (int)threadIdx.x % NT >= NBLK) { org += step; return; }
+#pragma unroll
+        for (int i = 0; i < N16; i++) {
+            const char *o = KC ? org : org + (i % V) * ld * (long long)sizeof(T);
+            r[i] = load16u(reinterpret_cast<const T *>(o + off[KC ? i : i / V]));
+        }
+        org += step;
+    }
+    // Checked loads: any tile and k-step, element by element at the edges, zeros outside.
+    __device__ __forceinline__ void load_checked(const T *__restrict__ X, long long ld, int MN, int K, int mn0, int k0, int tid) {
         if constexpr (KC) {
 #pragma unroll
             for (int i = 0; i < N16; i++) {
-                const int id = i * NT + tid, row = mn0 + (id >> 3), col = k0 + (id & 7) * V;
-                if constexpr (CHECK) r[i] = load16<T, VEC>(X, ld, row, col, MN, K);
-                else r[i] = *reinterpret_cast<const u32x4 *>(X + (long long)row * ld + col);
+                const int id = i * NT + tid;
+                r[i] = load16<T>(X, ld, mn0 + (id >> 3), k0 + (id & 7) * V, MN, K);
             }
         } else {
             if (PART && tid >= NBLK) return;
@@ -158,11 +199,7 @@ struct Stage {
                 const int id = b * NT + tid, lo = id & 31;
                 const int mb = (lo & 3) + 4 * (id >> 5), kb = lo >> 2;
 #pragma unroll
-                for (int i = 0; i < V; i++) {
-                    const int row = k0 + kb * V + i, col = mn0 + mb * V;
-                    if constexpr (CHECK) r[b * V + i] = load16<T, VEC>(X, ld, row, col, K, MN);
-                    else r[b * V + i] = *reinterpret_cast<const u32x4 *>(X + (long long)row * ld + col);
-                }
+                for (int i = 0; i < V; i++) r[b * V + i] = load16<T>(X, ld, k0 + kb * V + i, mn0 + mb * V, K, MN);
             }
         }
     }
@@ -190,7 +227,7 @@ struct Stage {
 
 __device__ __forceinline__ float fma_s(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
-template <class T, class S> __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, bool vec, int valid);
+template <class T, class S> __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid);
 
 // Instruction-group masks of __builtin_amdgcn_sched_group_barrier.
 constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_WRITE = 0x200;
@@ -200,8 +237,8 @@ constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_W
 // KLIM: the k range of a tile is cut to where a triangular operand is non-zero (one product, no split):
 //   1: op(A) lower, k < m0 + BM; 2: op(A) upper, k ≥ m0; 3: op(B) lower, k ≥ n0; 4: op(B) upper, k < n0 + BN.
 //   Tiles are dispatched longest range first, spread over the XCDs.
-template <class T, int BM, int BN, int WM, int WN, bool AK, bool BKC, bool VEC, bool SCHED = true, bool SPLIT = false,
-          int TRI = 0, int KLIM = 0, int KG = 1>
+template <class T, int BM, int BN, int WM, int WN, bool AK, bool BKC, bool SPLIT = false, int TRI = 0, int KLIM = 0,
+          int KG = 1>
 __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typename Mma<T>::Sum> p) {
     using MM = Mma<T>;
     using S = typename MM::Sum;
@@ -297,8 +334,10 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         C += z * p.sC;
     }
 
-    Stage<T, BM, NT, AK, VEC> sa;
-    Stage<T, BN, NT, BKC, VEC> sb;
+    using SA = Stage<T, BM, NT, AK>;
+    using SB = Stage<T, BN, NT, BKC>;
+    SA sa;
+    SB sb;
     constexpr int TI = MM::SWAP ? TN : TM, TJ = MM::SWAP ? TM : TN;   // acc[i][j]: D tile of (first, second) operand
     typename MM::Acc acc[TI][TJ];
 #pragma unroll
@@ -353,68 +392,71 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     };
 
     // block tiles per k group (a group's tiles past K load as zeros)
-    const int nk = ((K + BK - 1) / BK + KG - 1) / KG;
+    const int nk = max(((K + BK - 1) / BK + KG - 1) / KG, 1);
     const int kofs = kh * BK;
     auto buf = [&](int b) { return lds[b * KG + kh]; };
-    // Interior tiles with whole k-steps load without bounds tests: the steady-state loop is then one basic block,
-    // whose instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between
-    // its MFMAs.
-    const bool fast = VEC && m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0;
-    if (fast) {
-        sa.template load<false>(A, p.lda, p.M, K, m0, kofs, tid);
-        sb.template load<false>(B, p.ldb, p.N, K, n0, kofs, tid);
-        sa.store(buf(0), tid);
-        sb.store(buf(0) + BM * ROWB, tid);
+    // Whole tiles and k-steps load without bounds tests. So do the other shapes, but for their last k-step, which the
+    // prologue takes first, with checked loads: the steady-state loop is then one basic block for every shape, whose
+    // instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between its
+    // MFMAs. Row strides below 16 bytes or beyond 32-bit offsets take the checked loads throughout. Before, a ragged
+    // tile took them in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9 µs, 64 × 250³
+    // (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096 140 → 112.
+    const auto load_checked = [&](int kt) {
+        sa.load_checked(A, p.lda, p.M, K, m0, kt * KG * BK + kofs, tid);
+        sb.load_checked(B, p.ldb, p.N, K, n0, kt * KG * BK + kofs, tid);
+    };
+    const auto store = [&](int b) {
+        sa.store(buf(b), tid);
+        sb.store(buf(b) + BM * ROWB, tid);
+    };
+    if (SA::ok(p.lda) && SB::ok(p.ldb)) {
+        sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
+        sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
+        if (m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {
+            sa.load(p.lda);
+            sb.load(p.ldb);
+        } else {
+            load_checked(nk - 1);
+        }
+        store(0);
         __syncthreads();
         for (int kt = 0; kt + 1 < nk; kt++) {
             const int cur = kt & 1;
-            sa.template load<false>(A, p.lda, p.M, K, m0, (kt + 1) * KG * BK + kofs, tid);
-            sb.template load<false>(B, p.ldb, p.N, K, n0, (kt + 1) * KG * BK + kofs, tid);
+            sa.load(p.lda);
+            sb.load(p.ldb);
             compute(cur);
-            sa.store(buf(cur ^ 1), tid);
-            sb.store(buf(cur ^ 1) + BM * ROWB, tid);
-            if constexpr (SCHED) {
-                constexpr int NRD = TM + TN;                         // LDS fragment reads per group
-                constexpr int NMF = SPG * TI * TJ;                   // MFMAs per group
-                constexpr int NVM = Stage<T, BM, NT, AK, VEC>::N16 + Stage<T, BN, NT, BKC, VEC>::N16;
-                constexpr int NWR = (AK ? Stage<T, BM, NT, AK, VEC>::N16 : Stage<T, BM, NT, AK, VEC>::NB * 8) +
-                                    (BKC ? Stage<T, BN, NT, BKC, VEC>::N16 : Stage<T, BN, NT, BKC, VEC>::NB * 8);
-                // global loads first, then group 0's fragments; each later group: its MFMAs interleaved with the next
-                // group's reads, and over the last two groups the LDS writes of the next tile
-                __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, NVM, 0);
-                __builtin_amdgcn_sched_group_barrier(SG_DS_READ, NRD, 0);
+            store(cur ^ 1);
+            constexpr int NRD = TM + TN;                         // LDS fragment reads per group
+            constexpr int NMF = SPG * TI * TJ;                   // MFMAs per group
+            constexpr int NVM = SA::N16 + SB::N16;
+            constexpr int NWR = (AK ? SA::N16 : SA::NB * 8) + (BKC ? SB::N16 : SB::NB * 8);
+            // global loads first, then group 0's fragments; each later group: its MFMAs interleaved with the next
+            // group's reads, and over the last two groups the LDS writes of the next tile
+            __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, NVM, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_DS_READ, NRD, 0);
 #pragma unroll
-                for (int q = 0; q < QG; q++) {
-                    const int nrd = q + 1 < QG ? NRD : 0;
-                    const int nwr = q >= QG - 2 ? (q == QG - 1 ? NWR - NWR / 2 : NWR / 2) : 0;
+            for (int q = 0; q < QG; q++) {
+                const int nrd = q + 1 < QG ? NRD : 0;
+                const int nwr = q >= QG - 2 ? (q == QG - 1 ? NWR - NWR / 2 : NWR / 2) : 0;
 #pragma unroll
-                    for (int t = 0; t < NMF; t++) {
-                        __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                        if (t < nrd) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
-                        else if (t - nrd < nwr) __builtin_amdgcn_sched_group_barrier(SG_DS_WRITE, 1, 0);
-                    }
+                for (int t = 0; t < NMF; t++) {
+                    __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                    if (t < nrd) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
+                    else if (t - nrd < nwr) __builtin_amdgcn_sched_group_barrier(SG_DS_WRITE, 1, 0);
                 }
             }
             __syncthreads();
         }
         compute((nk - 1) & 1);
     } else {
-        auto load_tile = [&](int k0) {
-            sa.template load<true>(A, p.lda, p.M, K, m0, k0, tid);
-            sb.template load<true>(B, p.ldb, p.N, K, n0, k0, tid);
-        };
-        load_tile(kofs);
-        sa.store(buf(0), tid);
-        sb.store(buf(0) + BM * ROWB, tid);
+        load_checked(0);
+        store(0);
         __syncthreads();
         for (int kt = 0; kt < nk; kt++) {
             const int cur = kt & 1;
-            if (kt + 1 < nk) load_tile((kt + 1) * KG * BK + kofs);
+            if (kt + 1 < nk) load_checked(kt + 1);
             compute(cur);
-            if (kt + 1 < nk) {
-                sa.store(buf(cur ^ 1), tid);
-                sb.store(buf(cur ^ 1) + BM * ROWB, tid);
-            }
+            if (kt + 1 < nk) store(cur ^ 1);
             __syncthreads();
         }
     }
@@ -473,9 +515,9 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
                         continue;
                     }
                     if constexpr (SPLIT)
-                        store4<S, S>(p.P + z * p.M * (long long)p.N + (long long)m * p.N + n, v, S(1), S(0), p.vec_p, p.N - n);
+                        store4<S, S>(p.P + z * p.M * (long long)p.N + (long long)m * p.N + n, v, S(1), S(0), p.N - n);
                     else
-                        store4<T, S>(C + (long long)m * p.ldc + n, v, p.alpha, p.beta, p.vec_c, p.N - n);
+                        store4<T, S>(C + (long long)m * p.ldc + n, v, p.alpha, p.beta, p.N - n);
                 }
             }
     } else {
@@ -505,28 +547,16 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
 
 // C[0..3] = alpha·v + beta·C (C not read when beta = 0), rounded once to T; `valid` elements are inside C.
 template <class T, class S>
-__device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, bool vec, int valid) {
-    if (vec && valid >= 4) {
-        if constexpr (sizeof(T) == 2) {
-            u32x2 old = beta != S(0) ? *reinterpret_cast<const u32x2 *>(c) : u32x2{0, 0};
-            union { u32x2 w; T e[4]; } o, n;
-            o.w = old;
+__device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid) {
+    if (valid >= 4) {
+        // one vector store at element alignment (as load16u)
+        typedef T T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+        T4 *p = reinterpret_cast<T4 *>(c);
+        T4 o = {}, n;
+        if (beta != S(0)) o = *p;
 #pragma unroll
-            for (int e = 0; e < 4; e++) n.e[e] = (T)(beta != S(0) ? __builtin_fmaf(beta, (S)o.e[e], alpha * v[e]) : alpha * v[e]);
-            *reinterpret_cast<u32x2 *>(c) = n.w;
-        } else if constexpr (sizeof(T) == 4) {
-            f32x4 o = beta != S(0) ? *reinterpret_cast<const f32x4 *>(c) : f32x4{0, 0, 0, 0};
-            f32x4 n;
-#pragma unroll
-            for (int e = 0; e < 4; e++) n[e] = beta != S(0) ? __builtin_fmaf(beta, o[e], alpha * v[e]) : alpha * v[e];
-            *reinterpret_cast<f32x4 *>(c) = n;
-        } else {
-            f64x4 o = beta != S(0) ? *reinterpret_cast<const f64x4 *>(c) : f64x4{0, 0, 0, 0};
-            f64x4 n;
-#pragma unroll
-            for (int e = 0; e < 4; e++) n[e] = beta != S(0) ? __builtin_fma(beta, o[e], alpha * v[e]) : alpha * v[e];
-            *reinterpret_cast<f64x4 *>(c) = n;
-        }
+        for (int e = 0; e < 4; e++) n[e] = (T)(beta != S(0) ? fma_s(beta, (S)o[e], alpha * v[e]) : alpha * v[e]);
+        *p = n;
         return;
     }
 #pragma unroll
@@ -553,7 +583,7 @@ __global__ void __launch_bounds__(256) splitk_reduce(const S *__restrict__ P, T 
             for (int sp = 0; sp < splits; sp++)
 #pragma unroll
                 for (int t = 0; t < 4; t++) v[t] += P[sp * mn + e + t];
-            store4<T, S>(C + (long long)m * ldc + n, v, alpha, beta, true, 4);
+            store4<T, S>(C + (long long)m * ldc + n, v, alpha, beta, 4);
         }
     } else {
         for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < mn; e += stride) {

@@ -23,22 +23,22 @@ namespace g9 {
 //   Small at n = 1024 (NN): FP32 64×64 (256 tiles, no split) 69 TFLOP/s against 62 for 128×128 split four ways;
 //   FP64 64×128 split two ways 43, 64×64 41. Both are beaten by 64×64 tiles with two k groups (launch_layout).
 struct TileCfg { int BM, BN, WM, WN; };
-// Layouts whose staging needs more registers than a wave has at 2 waves per SIMD (transposed A, unaligned
-// operands) keep FP16 at 4 waves (512 registers per wave), which compiles without spills.
-template <class T, bool AK, bool BKC, bool VEC> struct Cfg;
+// Transposed A, whose staging needs more registers than a wave has at 2 waves per SIMD, keeps FP16 at 4 waves (512
+// registers per wave), which compiles without spills.
+template <class T, bool AK, bool BKC> struct Cfg;
 // small_div: the small tile is taken when the big tiles times small_div are fewer than the CUs.
-template <bool AK, bool BKC, bool VEC> struct Cfg<f16, AK, BKC, VEC> {
-    static constexpr TileCfg big = (AK && VEC) ? TileCfg{256, 256, 4, 2} : TileCfg{256, 256, 2, 2};
+template <bool AK, bool BKC> struct Cfg<f16, AK, BKC> {
+    static constexpr TileCfg big = AK ? TileCfg{256, 256, 4, 2} : TileCfg{256, 256, 2, 2};
     static constexpr TileCfg small{128, 128, 2, 2};
     static constexpr int small_div = 2;
 };
-template <bool AK, bool BKC, bool VEC> struct Cfg<float, AK, BKC, VEC> {
+template <bool AK, bool BKC> struct Cfg<float, AK, BKC> {
     static constexpr TileCfg big = !AK ? (BKC ? TileCfg{128, 64, 2, 2} : TileCfg{128, 128, 2, 2})
                                        : (BKC ? TileCfg{64, 64, 2, 2} : TileCfg{64, 128, 2, 2});
     static constexpr TileCfg small{64, 64, 2, 2};
     static constexpr int small_div = 1;
 };
-template <bool AK, bool BKC, bool VEC> struct Cfg<double, AK, BKC, VEC> {
+template <bool AK, bool BKC> struct Cfg<double, AK, BKC> {
     static constexpr TileCfg big{256, 128, 4, 2}, small{64, 128, 2, 2};
     static constexpr int small_div = 2;
 };
@@ -67,7 +67,7 @@ static int splitk_slices(long long tiles, int K, int BK, int count) {
     return s;
 }
 
-template <class T, TileCfg C, bool AK, bool BKC, bool VEC, int KG = 1>
+template <class T, TileCfg C, bool AK, bool BKC, int KG = 1>
 static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     using S = typename Mma<T>::Sum;
     constexpr int BK = 128 / (int)sizeof(T);
@@ -85,12 +85,11 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
         void *P;
         G9_TRY(scratch(SLOT_P, (size_t)ns * p.M * p.N * sizeof(S), &P));
         p.P = reinterpret_cast<S *>(P);
-        p.vec_p = p.N % 4 == 0;
-        hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, VEC, true, true>), dim3((unsigned)tiles, (unsigned)ns),
+        hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, true>), dim3((unsigned)tiles, (unsigned)ns),
                            block, 0, stream, p);
         G9_HIP(hipGetLastError());
         const long long mn = (long long)p.M * p.N;
-        const bool v4 = p.vec_c && p.N % 4 == 0;
+        const bool v4 = p.N % 4 == 0;
         const long long work = v4 ? mn / 4 : mn;
         const unsigned blocks = (unsigned)std::min<long long>((work + 255) / 256, (long long)num_cus * 8);
         T *Cp = reinterpret_cast<T *>(p.C);
@@ -100,14 +99,14 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
         return 0;
     }
     const dim3 grid((unsigned)tiles, (unsigned)count);
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, VEC, true, false, 0, 0, KG>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, 0, 0, KG>), grid, block, 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
 }
 
-template <class T, bool AK, bool BKC, bool VEC>
+template <class T, bool AK, bool BKC>
 static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
-    using CF = Cfg<T, AK, BKC, VEC>;
+    using CF = Cfg<T, AK, BKC>;
     const long long big_tiles = (long long)((p.M + CF::big.BM - 1) / CF::big.BM) * ((p.N + CF::big.BN - 1) / CF::big.BN) * count;
     if (big_tiles * CF::small_div < num_cus) {
         // 64×64 tiles with two k groups of 4 waves (8 waves per workgroup, the groups' sums added through LDS), when
@@ -124,9 +123,9 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
             const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
             const long long need = count > 1 ? (num_cus + 3) / 4 : (num_cus + 1) / 2;
             if (splitk_forced() < 0 && t64 >= need && (sizeof(T) == 8 || t64 <= num_cus))
-                return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, VEC, 2>(p, count);
+                return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 2>(p, count);
         }
-        return launch_t<T, CF::small, AK, BKC, VEC>(p, count);
+        return launch_t<T, CF::small, AK, BKC>(p, count);
     }
     // FP64 whose big tiles are exactly half the CUs (K would be split in two, with a reduction pass after): the small
     // tiles instead, when they fill the CUs. MI355X, µs (TFLOP/s): 1024×4096×1024 with beta = 1 (the triangular
@@ -136,14 +135,14 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
         const long long ts = (long long)((p.M + CF::small.BM - 1) / CF::small.BM) *
                              ((p.N + CF::small.BN - 1) / CF::small.BN) * count;
         if (splitk_forced() < 0 && count == 1 && big_tiles * 2 == num_cus && ts >= num_cus)
-            return launch_t<T, CF::small, AK, BKC, VEC>(p, count);
+            return launch_t<T, CF::small, AK, BKC>(p, count);
     }
     // FP32 with B k-contiguous has 64×64 big tiles, so a product of exactly num_cus of them lands here: the same
     // two-k-group tiles (NT n = 1024)
     if constexpr (sizeof(T) == 4) {
         const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
         if (splitk_forced() < 0 && t64 * 2 >= num_cus && t64 <= num_cus)
-            return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, VEC, 2>(p, count);
+            return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 2>(p, count);
     }
     // FP32: 128×128 tiles with two k groups of 2×2 waves (64×64 per wave, 147 KiB of LDS: one workgroup per CU) when
     // their count fills whole rounds of num_cus workgroups (the last round at least 95 % full). Measured (TFLOP/s,
@@ -153,9 +152,9 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
         const long long t128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * count;
         const long long rounds = (t128 + num_cus - 1) / num_cus;
         if (splitk_forced() < 0 && t128 >= num_cus && t128 * 20 >= rounds * num_cus * 19)
-            return launch_t<T, TileCfg{128, 128, 2, 2}, AK, BKC, VEC, 2>(p, count);
+            return launch_t<T, TileCfg{128, 128, 2, 2}, AK, BKC, 2>(p, count);
     }
-    return launch_t<T, CF::big, AK, BKC, VEC>(p, count);
+    return launch_t<T, CF::big, AK, BKC>(p, count);
 }
 
 // ---------------- FP16 whole-tile kernel ----------------
@@ -453,24 +452,10 @@ static int launch_typed(const GemmCall &c) {
     p.beta = (S)c.beta;
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
-    p.kper = p.vec_p = 0;
-    const long long es = sizeof(T);
-    const long long cal = es * 4 < 16 ? es * 4 : 16;   // alignment of a 4-element group of C
-    p.vec_c = ((uintptr_t)c.C % cal == 0) && (c.ldc * es) % cal == 0 && (c.count == 1 || (c.sC * es) % cal == 0);
-    const bool vec = ((uintptr_t)c.A % 16 == 0) && ((uintptr_t)c.B % 16 == 0) && (c.lda * es) % 16 == 0 &&
-                     (c.ldb * es) % 16 == 0 && (c.count == 1 || ((c.sA * es) % 16 == 0 && (c.sB * es) % 16 == 0));
+    p.kper = 0;
     const bool ak = !c.tA, bk = c.tB;   // k-contiguous A: not transposed; k-contiguous B: transposed (stored N×K)
-    const int sel = (ak ? 4 : 0) | (bk ? 2 : 0) | (vec ? 1 : 0);
-    switch (sel) {
-    case 0: return launch_layout<T, false, false, false>(p, c.count);
-    case 1: return launch_layout<T, false, false, true>(p, c.count);
-    case 2: return launch_layout<T, false, true, false>(p, c.count);
-    case 3: return launch_layout<T, false, true, true>(p, c.count);
-    case 4: return launch_layout<T, true, false, false>(p, c.count);
-    case 5: return launch_layout<T, true, false, true>(p, c.count);
-    case 6: return launch_layout<T, true, true, false>(p, c.count);
-    default: return launch_layout<T, true, true, true>(p, c.count);
-    }
+    if (ak) return bk ? launch_layout<T, true, true>(p, c.count) : launch_layout<T, true, false>(p, c.count);
+    return bk ? launch_layout<T, false, true>(p, c.count) : launch_layout<T, false, false>(p, c.count);
 }
 
 // Triangle of a square product (SYRK, SYR2K): alpha·op(A)·op(B) + beta·C written on the lower (upper) triangle of C
@@ -478,21 +463,20 @@ static int launch_typed(const GemmCall &c) {
 // element, each C element rounded once; the two layouts those routines use: A and B both k-contiguous, or both
 // mn-contiguous. FP32 and FP64 take 64×64 tiles: at n = 4096 their 2080 tiles keep every CU busy to the end (FP32
 // SYRK 0.71 ms, FP64 1.21), where 128×128 tiles (528) left a nearly empty last round (1.02, 1.58).
-template <class T, int TRI, bool AK, bool BKC, bool VEC>
+template <class T, int TRI, bool AK, bool BKC>
 static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
     constexpr TileCfg C = sizeof(T) == 2 ? TileCfg{128, 128, 2, 2} : TileCfg{64, 64, 2, 2};
     p.tiles_m = p.tiles_n = (p.M + C.BM - 1) / C.BM;
     const long long tiles = (long long)p.tiles_m * (p.tiles_m + 1) / 2;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product too large (%d tiles per side)", p.tiles_m);
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, VEC, true, false, TRI>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI>), dim3((unsigned)tiles),
                        dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
 }
 template <class T, bool AK, bool BKC>
-static int launch_tri_layout(const GemmParams<typename Mma<T>::Sum> &p, bool vec, bool lower) {
-    if (vec) return lower ? launch_tri_t<T, 1, AK, BKC, true>(p) : launch_tri_t<T, 2, AK, BKC, true>(p);
-    return lower ? launch_tri_t<T, 1, AK, BKC, false>(p) : launch_tri_t<T, 2, AK, BKC, false>(p);
+static int launch_tri_layout(const GemmParams<typename Mma<T>::Sum> &p, bool lower) {
+    return lower ? launch_tri_t<T, 1, AK, BKC>(p) : launch_tri_t<T, 2, AK, BKC>(p);
 }
 template <class T>
 static int launch_tri_typed(const GemmCall &c, bool lower) {
@@ -507,14 +491,9 @@ static int launch_tri_typed(const GemmCall &c, bool lower) {
     p.beta = (S)c.beta;
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
-    p.kper = p.vec_p = 0;
-    const long long es = sizeof(T);
-    const long long cal = es * 4 < 16 ? es * 4 : 16;
-    p.vec_c = ((uintptr_t)c.C % cal == 0) && (c.ldc * es) % cal == 0 && (p.sC * es) % cal == 0;
-    const bool vec = ((uintptr_t)c.A % 16 == 0) && ((uintptr_t)c.B % 16 == 0) && (c.lda * es) % 16 == 0 && (c.ldb * es) % 16 == 0 &&
-                     (p.sA * es) % 16 == 0 && (p.sB * es) % 16 == 0;
-    if (!c.tA && c.tB) return launch_tri_layout<T, true, true>(p, vec, lower);
-    if (c.tA && !c.tB) return launch_tri_layout<T, false, false>(p, vec, lower);
+    p.kper = 0;
+    if (!c.tA && c.tB) return launch_tri_layout<T, true, true>(p, lower);
+    if (c.tA && !c.tB) return launch_tri_layout<T, false, false>(p, lower);
     G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product: layout tA=%d tB=%d", c.tA, c.tB);
 }
 int launch_gemm_tri(const GemmCall &c, bool lower) {
@@ -535,13 +514,13 @@ int launch_gemm_tri(const GemmCall &c, bool lower) {
 // range is cut to where the triangle is non-zero (klim as gemm_kernel's KLIM), one launch over every tile of C,
 // longest ranges dispatched first; the small tiles when the big ones are fewer than the CUs. Layout NN only (both
 // operands as stored), one product.
-template <class T, TileCfg C, int KLIM, bool VEC>
+template <class T, TileCfg C, int KLIM>
 static int launch_klim_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     p.tiles_m = (p.M + C.BM - 1) / C.BM;
     p.tiles_n = (p.N + C.BN - 1) / C.BN;
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles)", p.tiles_m, p.tiles_n);
-    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, VEC, true, false, 0, KLIM>;
+    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM>;
     p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(C.WM * C.WN * 64));
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
@@ -560,41 +539,32 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     p.beta = (S)c.beta;
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
-    p.kper = p.vec_p = 0;
-    const long long es = sizeof(T);
-    const long long cal = es * 4 < 16 ? es * 4 : 16;
-    p.vec_c = ((uintptr_t)c.C % cal == 0) && (c.ldc * es) % cal == 0 && (p.sC * es) % cal == 0;
-    const bool vec = ((uintptr_t)c.A % 16 == 0) && ((uintptr_t)c.B % 16 == 0) && (c.lda * es) % 16 == 0 && (c.ldb * es) % 16 == 0 &&
-                     (p.sA * es) % 16 == 0 && (p.sB * es) % 16 == 0;
+    p.kper = 0;
     // tile class: FP16 the big tiles when they are at least the CUs; FP32 / FP64 the first of big, small and (FP64)
     // 64×64 that makes two workgroups per CU or more, so that long and short k ranges can share the CUs
-    const auto by_cfg = [&](auto vc) -> int {
-        constexpr bool V = decltype(vc)::value;
-        using CF = Cfg<T, true, false, V>;
-        constexpr TileCfg tiny{64, 64, 2, 2};
-        const auto ntiles = [&](TileCfg t) {
-            return (long long)((c.M + t.BM - 1) / t.BM) * ((c.N + t.BN - 1) / t.BN) * c.count;
-        };
-        constexpr bool half = sizeof(T) == 2, dbl = sizeof(T) == 8;
-        const long long want = half ? num_cus : 2LL * num_cus;
-        const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
-        const auto go = [&](auto kc) -> int {
-            constexpr int K = decltype(kc)::value;
-            if (cls == 0) return launch_klim_t<T, CF::big, K, V>(p, c.count);
-            if constexpr (dbl) {
-                if (cls == 2) return launch_klim_t<T, tiny, K, V>(p, c.count);
-            }
-            return launch_klim_t<T, CF::small, K, V>(p, c.count);
-        };
-        switch (klim) {
-        case 1: return go(std::integral_constant<int, 1>());
-        case 2: return go(std::integral_constant<int, 2>());
-        case 3: return go(std::integral_constant<int, 3>());
-        case 4: return go(std::integral_constant<int, 4>());
-        }
-        G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "k-limited product: mode %d", klim);
+    using CF = Cfg<T, true, false>;
+    constexpr TileCfg tiny{64, 64, 2, 2};
+    const auto ntiles = [&](TileCfg t) {
+        return (long long)((c.M + t.BM - 1) / t.BM) * ((c.N + t.BN - 1) / t.BN) * c.count;
     };
-    return vec ? by_cfg(std::true_type()) : by_cfg(std::false_type());
+    constexpr bool half = sizeof(T) == 2, dbl = sizeof(T) == 8;
+    const long long want = half ? num_cus : 2LL * num_cus;
+    const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
+    const auto go = [&](auto kc) -> int {
+        constexpr int K = decltype(kc)::value;
+        if (cls == 0) return launch_klim_t<T, CF::big, K>(p, c.count);
+        if constexpr (dbl) {
+            if (cls == 2) return launch_klim_t<T, tiny, K>(p, c.count);
+        }
+        return launch_klim_t<T, CF::small, K>(p, c.count);
+    };
+    switch (klim) {
+    case 1: return go(std::integral_constant<int, 1>());
+    case 2: return go(std::integral_constant<int, 2>());
+    case 3: return go(std::integral_constant<int, 3>());
+    case 4: return go(std::integral_constant<int, 4>());
+    }
+    G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "k-limited product: mode %d", klim);
 }
 int launch_gemm_klim(const GemmCall &c, int klim) {
     if (c.tA || c.tB || c.count < 1) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "k-limited product: layout tA=%d tB=%d, batch %d", c.tA, c.tB, c.count);

@@ -1,0 +1,70 @@
+"""Matrix products of ragged and unaligned shapes on the GPU, bit-exact on small integers.
+
+Operands are views into NaN-filled device buffers, at an element offset and with a row stride of their own, so that a
+value read from outside an operand that reaches a result shows as NaN; C lies in a buffer of a sentinel value that must
+survive around it. The integers are small enough that every product and sum is exact in each type.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DT = {"H": "float16", "S": "float32", "D": "float64"}
+
+
+def _view(torch, rng, dt, shape, pad, off, count=1, fill=float("nan")):
+    """(count, rows, cols) small integers in a `fill` buffer: row stride cols + pad, first element at `off`."""
+    rows, cols = shape
+    ld = cols + pad
+    span = rows * ld + 3
+    buf = torch.full((off + count * span + 64,), fill, dtype=getattr(torch, dt), device="cuda")
+    v = torch.as_strided(buf, (count, rows, cols), (span, ld, 1), off)
+    v.copy_(torch.from_numpy(rng.integers(-2, 3, (count, rows, cols)).astype(np.float64)).cuda())
+    return buf, v, ld, span
+
+
+def check(g9, torch, kind, M, N, K, ta, tb, pad=0, off=0, beta=0.0, count=1, seed=0):
+    """One gemm / gemm_batched call against the same product in float64."""
+    rng, dt = np.random.default_rng(seed), DT[kind]
+    _, a, lda, sa = _view(torch, rng, dt, (K, M) if ta else (M, K), pad, off, count)
+    _, b, ldb, sb = _view(torch, rng, dt, (N, K) if tb else (K, N), pad, off, count)
+    cb, c, ldc, sc = _view(torch, rng, dt, (M, N), pad, off, count, fill=77.0)
+    opa, opb = (x.double().transpose(1, 2) if t else x.double() for x, t in ((a, ta), (b, tb)))
+    want = torch.stack([torch.mm(x.contiguous(), y.contiguous()) for x, y in zip(opa, opb)]) * 2.0
+    if beta:
+        want += beta * c.double()
+    else:
+        c.fill_(float("nan"))   # beta = 0: C is not read
+    keep = cb.clone()
+    torch.as_strided(keep, c.shape, c.stride(), off).copy_(want)
+    code = {"H": 0, "S": 1, "D": 3}[kind]
+    g9._call("gemm_batched", code, ta, tb, M, N, K, 2.0, a.data_ptr(), lda, sa, b.data_ptr(), ldb, sb, beta, c.data_ptr(),
+             ldc, sc, count)
+    torch.cuda.synchronize()
+    bad = (cb != keep).nonzero()
+    assert bad.numel() == 0, f"{kind} {M}x{N}x{K} tA={ta} tB={tb} pad={pad} off={off} beta={beta} count={count}: " \
+                             f"{bad.shape[0]} wrong elements, first at {bad[0].item() - off}, row stride {ldc}"
+
+
+# tile edges (one past, one short, a remainder of one element) and k remainders around the k-step of each type (64
+# FP16, 32 FP32, 16 FP64; twice that for tiles with two k groups)
+RAGGED = [(129, 127, 65), (65, 255, 31), (257, 130, 129), (320, 192, 97), (200, 1000, 17), (19, 24, 200), (513, 512, 33),
+          (1000, 1001, 111)]
+
+
+@pytest.mark.parametrize("kind", ["H", "S", "D"])
+@pytest.mark.parametrize("M,N,K", RAGGED)
+def test_gemm_ragged_steps(g9, torch_dev, kind, M, N, K):
+    """Tiles that cross the matrix's edges load full k-steps unchecked and their last k-step with checks."""
+    for ta, tb in [(0, 0), (1, 0), (0, 1), (1, 1)]:
+        for pad, off, beta in [(0, 0, 0.0), (1, 1, -1.0), (3, 2, 0.0), (8, 0, 0.5)]:
+            check(g9, torch_dev, kind, M, N, K, ta, tb, pad, off, beta, seed=M + N + K)
+
+
+@pytest.mark.parametrize("kind", ["H", "S", "D"])
+def test_gemm_ragged_batch_and_tiny_strides(g9, torch_dev, kind):
+    """Batches of unaligned matrices, and operands whose rows are shorter than one 16-byte load (N or M of 1-3)."""
+    for ta, tb in [(0, 0), (1, 0), (0, 1), (1, 1)]:
+        check(g9, torch_dev, kind, 70, 90, 75, ta, tb, 1, 1, 0.0, count=5, seed=5)
+        for M, N in [(200, 1), (2, 300), (3, 5)]:
+            check(g9, torch_dev, kind, M, N, 150, ta, tb, 0, 0, 0.0, count=3, seed=M + N)
