@@ -21,6 +21,7 @@
 //   each XCD a contiguous range, and tiles are ordered in groups of GM tile rows so an XCD's L2 shares A and B panels.
 #pragma once
 #include "internal.h"
+#include "lds_dma.h"
 #include <type_traits>
 
 namespace g9 {
@@ -90,26 +91,6 @@ template <class S> struct GemmParams {
     int kpair = 0;   // KLIM: the second half of the dispatch order reversed (see the tile mapping)
 };
 
-// 16 bytes at an address aligned to the element type only: one global_load_dwordx4 either way (the GPU serves it at
-// any element alignment, at the aligned rate when the address is aligned).
-template <class T> __device__ __forceinline__ u32x4 load16u(const T *p) {
-    typedef T TV __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
-    const TV v = *reinterpret_cast<const TV *>(p);
-    return __builtin_bit_cast(u32x4, v);
-}
-
-// 16 bytes (V elements) of row r, columns c .. c+V-1 of a row-major matrix X (R valid rows, Cc valid columns, row
-// stride ld); zero outside the valid region.
-template <class T>
-__device__ __forceinline__ u32x4 load16(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
-    constexpr int V = 16 / sizeof(T);
-    if (r < R && c + V <= Cc) return load16u(X + (long long)r * ld + c);
-    union { u32x4 v; T e[V]; } u;
-#pragma unroll
-    for (int e = 0; e < V; e++) u.e[e] = (r < R && c + e < Cc) ? X[(long long)r * ld + c + e] : T(0);
-    return u.v;
-}
-
 // Transpose of a V×V block held as V rows of 16 bytes: out[j] element i = in[i] element j.
 template <class T> __device__ __forceinline__ void transpose(const u32x4 *in, u32x4 *out);
 template <> __device__ __forceinline__ void transpose<f16>(const u32x4 *in, u32x4 *out) {
@@ -136,7 +117,8 @@ template <> __device__ __forceinline__ void transpose<double>(const u32x4 *in, u
 // KC: the operand is stored k-contiguous (element (mn, k) at X[mn·ld + k]); otherwise mn-contiguous
 // (element (mn, k) at X[k·ld + mn]) and transposed in registers on the way to LDS.
 constexpr int ROWB = 144;   // LDS bytes per tile row: 128 of data + 16 of padding
-template <class T, int RT, int NT, bool KC>
+// SHIFT: as load16 (the 256-row tiles have no registers left for it).
+template <class T, int RT, int NT, bool KC, bool SHIFT>
 struct Stage {
     static constexpr int V = 16 / (int)sizeof(T);
     // k-contiguous: N16 chunks per thread. Transposed: NB V×V blocks per thread; when the tile has fewer blocks than
@@ -153,14 +135,11 @@ struct Stage {
     // step: bytes per k-step of BK·KG. Rows (starts of chunks) past the matrix's end are moved back onto the last one,
     // whose values no stored element uses; a chunk that straddles the end of an mn-contiguous row reads on into the
     // next row, so a k-step loaded this way must not hold the last k unless the tile lies inside the matrix, and ld
-    // must be at least V - 1. The offsets are 32-bit: ok() bounds the row stride.
+    // must be at least V - 1. The offsets are 32-bit, which bounds the row stride (unchecked_ok).
     static constexpr int NOFF = KC ? N16 : NB;
     const char *org;
     unsigned off[NOFF];
     long long step;
-    static __device__ __forceinline__ bool ok(long long ld) {
-        return (KC || ld >= V - 1) && (KC ? RT : 128 / (int)sizeof(T)) * ld * (long long)sizeof(T) < (1LL << 31);
-    }
     __device__ __forceinline__ void init(const T *__restrict__ X, long long ld, int MN, int mn0, int k0, int kstep, int tid) {
         org = reinterpret_cast<const char *>(KC ? X + (long long)mn0 * ld + k0 : X + (long long)k0 * ld + mn0);
         step = (KC ? (long long)kstep : kstep * ld) * (long long)sizeof(T);
@@ -190,7 +169,7 @@ struct Stage {
 #pragma unroll
             for (int i = 0; i < N16; i++) {
                 const int id = i * NT + tid;
-                r[i] = load16<T>(X, ld, mn0 + (id >> 3), k0 + (id & 7) * V, MN, K);
+                r[i] = load16<T, SHIFT>(X, ld, mn0 + (id >> 3), k0 + (id & 7) * V, MN, K);
             }
         } else {
             if (PART && tid >= NBLK) return;
@@ -199,7 +178,7 @@ struct Stage {
                 const int id = b * NT + tid, lo = id & 31;
                 const int mb = (lo & 3) + 4 * (id >> 5), kb = lo >> 2;
 #pragma unroll
-                for (int i = 0; i < V; i++) r[b * V + i] = load16<T>(X, ld, k0 + kb * V + i, mn0 + mb * V, K, MN);
+                for (int i = 0; i < V; i++) r[b * V + i] = load16<T, SHIFT>(X, ld, k0 + kb * V + i, mn0 + mb * V, K, MN);
             }
         }
     }
@@ -229,6 +208,12 @@ __device__ __forceinline__ float fma_s(float a, float b, float c) { return __bui
 __device__ __forceinline__ double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
 template <class T, class S> __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid);
 
+// Whether the unchecked loads take an operand of this row stride: at least one element short of 16 bytes where chunks run
+// along mn, and offsets inside a tile (at most 256 rows) below 2^31 bytes.
+template <class T> inline bool unchecked_ok(bool kc, long long ld) {
+    return (kc || ld >= 16 / (int)sizeof(T) - 1) && ld * 256 * (long long)sizeof(T) < (1LL << 31);
+}
+
 // Instruction-group masks of __builtin_amdgcn_sched_group_barrier.
 constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_WRITE = 0x200;
 
@@ -237,8 +222,9 @@ constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_W
 // KLIM: the k range of a tile is cut to where a triangular operand is non-zero (one product, no split):
 //   1: op(A) lower, k < m0 + BM; 2: op(A) upper, k ≥ m0; 3: op(B) lower, k ≥ n0; 4: op(B) upper, k < n0 + BN.
 //   Tiles are dispatched longest range first, spread over the XCDs.
+// CHECKED: every k-step takes the checked loads (row strides that the unchecked ones do not take).
 template <class T, int BM, int BN, int WM, int WN, bool AK, bool BKC, bool SPLIT = false, int TRI = 0, int KLIM = 0,
-          int KG = 1>
+          int KG = 1, bool CHECKED = false>
 __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typename Mma<T>::Sum> p) {
     using MM = Mma<T>;
     using S = typename MM::Sum;
@@ -334,8 +320,8 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         C += z * p.sC;
     }
 
-    using SA = Stage<T, BM, NT, AK>;
-    using SB = Stage<T, BN, NT, BKC>;
+    using SA = Stage<T, BM, NT, AK, (BM < 256)>;
+    using SB = Stage<T, BN, NT, BKC, (BM < 256)>;
     SA sa;
     SB sb;
     constexpr int TI = MM::SWAP ? TN : TM, TJ = MM::SWAP ? TM : TN;   // acc[i][j]: D tile of (first, second) operand
@@ -398,8 +384,8 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     // Whole tiles and k-steps load without bounds tests. So do the other shapes, but for their last k-step, which the
     // prologue takes first, with checked loads: the steady-state loop is then one basic block for every shape, whose
     // instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between its
-    // MFMAs. Row strides below 16 bytes or beyond 32-bit offsets take the checked loads throughout. Before, a ragged
-    // tile took them in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9 µs, 64 × 250³
+    // MFMAs. (The checked loop is a variant of its own: beside it, the compiler copies the accumulators in every k-step
+    // of the steady loop.) Before, a ragged tile took the checked loads in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9 µs, 64 × 250³
     // (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096 140 → 112.
     const auto load_checked = [&](int kt) {
         sa.load_checked(A, p.lda, p.M, K, m0, kt * KG * BK + kofs, tid);
@@ -409,7 +395,7 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         sa.store(buf(b), tid);
         sb.store(buf(b) + BM * ROWB, tid);
     };
-    if (SA::ok(p.lda) && SB::ok(p.ldb)) {
+    if constexpr (!CHECKED) {
         sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
         sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
         if (m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {
@@ -420,6 +406,16 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         }
         store(0);
         __syncthreads();
+        // what the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes the compiler wait for
+        // every LDS read of a k-step at once (scalar loads and LDS reads share a counter)
+        asm volatile("" : "+s"(C), "+s"(p.P), "+s"(p.ldc), "+s"(p.M), "+s"(p.N));
+        wait_lgkm0();
+        // the accumulators' zeros are hidden from the compiler: as one shared constant they cost FP64 tiles 16-64 register
+        // copies per k-step (the loop's values then rotate through the accumulation registers)
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) asm volatile("" : "+v"(acc[i][j]));
         for (int kt = 0; kt + 1 < nk; kt++) {
             const int cur = kt & 1;
             sa.load(p.lda);
@@ -549,7 +545,7 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
 template <class T, class S>
 __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid) {
     if (valid >= 4) {
-        // one vector store at element alignment (as load16u)
+        // one vector store at element alignment (as load16u's loads)
         typedef T T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
         T4 *p = reinterpret_cast<T4 *>(c);
         T4 o = {}, n;

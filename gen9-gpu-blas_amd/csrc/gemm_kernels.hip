@@ -1,8 +1,7 @@
 // Host side of the MFMA GEMM: tile configuration per type and dispatch over the transpose layouts.
-// The kernel templates and their design notes are in gemm_kernel.h (every shape and type), hgemm_kernel.h (FP16,
-// whole tiles, direct global→LDS loads) and sgemm_kernel.h (FP32, whole tiles, direct global→LDS loads).
+// The kernel templates and their design notes are in gemm_kernel.h (every shape and type) and sgemm_kernel.h (FP32,
+// whole tiles, direct global→LDS loads); hgemm_launch.h holds the FP16 products on direct global→LDS loads.
 #include "gemm_kernel.h"
-#include "hgemm_kernel.h"
 #include "sgemm_kernel.h"
 #include <stdlib.h>
 #include <string.h>
@@ -67,7 +66,7 @@ static int splitk_slices(long long tiles, int K, int BK, int count) {
     return s;
 }
 
-template <class T, TileCfg C, bool AK, bool BKC, int KG = 1>
+template <class T, TileCfg C, bool AK, bool BKC, int KG = 1, bool CHECKED = false>
 static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     using S = typename Mma<T>::Sum;
     constexpr int BK = 128 / (int)sizeof(T);
@@ -76,9 +75,9 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     if ((long long)p.tiles_m * p.tiles_n > 0x7fffffffLL || count > 65535)
         G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles, batch %d)", p.tiles_m, p.tiles_n, count);
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
-    const int split = KG > 1 ? 1 : splitk_slices(tiles, p.K, BK, count);
+    const int split = KG > 1 || CHECKED ? 1 : splitk_slices(tiles, p.K, BK, count);
     const dim3 block(C.WM * C.WN * 64 * KG);
-    if (split > 1) {
+    if constexpr (!CHECKED) if (split > 1) {
         static_assert((size_t)C.BM * C.BN * sizeof(S) <= SPLITK_TILE_BYTES_MAX, "split tile beyond the work-space bound");
         p.kper = ((p.K + split - 1) / split + BK - 1) / BK * BK;
         const int ns = (p.K + p.kper - 1) / p.kper;
@@ -99,7 +98,7 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
         return 0;
     }
     const dim3 grid((unsigned)tiles, (unsigned)count);
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, 0, 0, KG>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, 0, 0, KG, CHECKED>), grid, block, 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
 }
@@ -107,6 +106,7 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
 template <class T, bool AK, bool BKC>
 static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     using CF = Cfg<T, AK, BKC>;
+    if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 1, true>(p, count);
     const long long big_tiles = (long long)((p.M + CF::big.BM - 1) / CF::big.BM) * ((p.N + CF::big.BN - 1) / CF::big.BN) * count;
     if (big_tiles * CF::small_div < num_cus) {
         // 64×64 tiles with two k groups of 4 waves (8 waves per workgroup, the groups' sums added through LDS), when
@@ -157,80 +157,9 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     return launch_t<T, CF::big, AK, BKC>(p, count);
 }
 
-// ---------------- FP16 whole-tile kernel ----------------
-// Configurations from sweeps on MI355X with N(0,1) FP16 inputs, timed after 1.5 s of the same load (the clock
-// settles under the board's power limit; shorter runs see its ramp), every variant bit-exact on small integers:
-// - products with at least one 256×256 tile per CU: 256×256 tiles, 8 waves of 128×64 (2×4), two stages of KB = 64.
-//   n = 4096 NN 1314-1324 TFLOP/s (8 waves of 64×128: 1276-1286; 4 waves of 128×128: 1243-1246, at 2.03 GHz against
-//   1.79-1.81; the same 8 waves on 32x32x16 MFMAs: 1166-1176); TN 1249, NT 1339, TT 1267 (32x32x16: 1180-1188);
-// - at least one 128×128 tile per CU: 128×128, 8 waves of 64×32 (2×4), three stages. n = 2048 NN 835 (4 waves of
-//   64×64 with 3 or 4 stages: 798-807; 32x32x16 tiles: 795), NT 845 (767), TN and TT 800-804 (800-802);
-// - fewer 128×128 tiles than CUs, with A k-contiguous: 64×64 tiles (below); before them 32×128 tiles, 4 waves of
-//   32×32, three stages, fragments read one k-step ahead: n = 1024 NN 385-386, NT 385 (reading inside the k-step:
-//   369-371 and 363; four stages 359-370,
-//   two 288-312; two k groups of 4 waves on separate rings, their sums added through LDS: 335-340; 32x32x16: 346).
-//   Time per call against K at M = N = 1024 is about 2-3 µs plus 0.26 µs per k-step of 64 (8 MFMAs per wave), so
-//   the k-step's latency chain (LDS reads, barrier), not its MFMAs, sets the rate; the read-ahead takes the LDS
-//   reads off that chain.
-//   At n = 2048 (128×128 tiles) the read-ahead gives nothing (841-849 against 849-853): that size runs at the power
-//   limit (1.8-2.0 GHz).
-// - the same small products on 64×64 tiles, 4 waves of 32×32, three stages, read-ahead: NT n = 1024 399.9 against
-//   385.9 for 32×128 (four stages 390.6, two 303.6, no read-ahead 378.1); NN 400.7 against 382.8 (four stages 394.2),
-//   its 64-wide mn-contiguous B rows swizzled by mnswz (hgemm_kernel.h). Per k-step a CU moves 16 KiB from L2 into
-//   LDS instead of 20 KiB for the same flops; at n = 1024 the 256 CUs together pull about 20 TB/s.
-template <int BM, int BN, int WM, int WN, int KB, int NS, bool AK, bool BKC, bool RA = false>
-static int launch_hg(const hg::Params &p0, int count) {
-    hg::Params p = p0;
-    p.tiles_m = p.M / BM;
-    p.tiles_n = p.N / BN;
-    const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)count), block(WM * WN * 64);
-    hipLaunchKernelGGL((hg::hgemm_kernel<BM, BN, WM, WN, KB, NS, AK, BKC, RA>), grid, block, 0, stream, p);
-    G9_HIP(hipGetLastError());
-    return 0;
-}
-template <bool AK, bool BKC>
-static int launch_hg_layout(const hg::Params &p, int count) {
-    if ((long long)(p.M / 256) * (p.N / 256) * count >= num_cus && p.M % 256 == 0 && p.N % 256 == 0)
-        return launch_hg<256, 256, 2, 4, 64, 2, AK, BKC>(p, count);
-    // below one 128×128 tile per CU: 64×64 tiles, every layout. With A k-contiguous they move 20 % fewer L2 → LDS bytes
-    // per flop than the 32×128 tiles of the same count (n = 1024 NN 382.8 → 400.7, NT 386 → 400 TFLOP/s); with A
-    // transposed they replace 128×128 tiles, 64 of them for 256 CUs at n = 1024 (TN 212.6 → 365.5, TT 215.3 → 393.1)
-    if ((long long)(p.M / 128) * (p.N / 128) * count < num_cus) return launch_hg<64, 64, 2, 2, 64, 3, AK, BKC, true>(p, count);
-    return launch_hg<128, 128, 2, 4, 64, 3, AK, BKC>(p, count);
-}
-// The whole-tile FP16 kernel applies when every operand is 16-byte aligned with 16-byte row strides, M and N are
-// multiples of 128, K of 64 (the k-step of every tile configuration), and the grid fits. GEN9BLAS_HGEMM=generic forces the general kernel.
-static bool hgemm_tiles_apply(const GemmCall &c) {
-    static int generic = -1;
-    if (generic < 0) {
-        const char *e = getenv("GEN9BLAS_HGEMM");
-        generic = e && !strcmp(e, "generic");
-    }
-    if (generic || c.M % 128 || c.N % 128 || c.K % 64 || c.count > 65535) return false;
-    const long long es = 2;
-    // each lane's byte offset inside a 256-row (or 64-k-row) tile is 32-bit: rows of up to 8 Mi elements
-    if (c.lda * es * 256 >= (1LL << 32) || c.ldb * es * 256 >= (1LL << 32)) return false;
-    return (uintptr_t)c.A % 16 == 0 && (uintptr_t)c.B % 16 == 0 && (uintptr_t)c.C % 16 == 0 && (c.lda * es) % 16 == 0 &&
-           (c.ldb * es) % 16 == 0 && (c.ldc * es) % 16 == 0 &&
-           (c.count == 1 || ((c.sA * es) % 16 == 0 && (c.sB * es) % 16 == 0 && (c.sC * es) % 16 == 0));
-}
-static int launch_hgemm_tiles(const GemmCall &c) {
-    hg::Params p;
-    p.A = reinterpret_cast<const hg::f16 *>(c.A);
-    p.B = reinterpret_cast<const hg::f16 *>(c.B);
-    p.C = reinterpret_cast<hg::f16 *>(c.C);
-    p.lda = c.lda; p.ldb = c.ldb; p.ldc = c.ldc;
-    p.sA = c.sA; p.sB = c.sB; p.sC = c.sC;
-    p.M = c.M; p.N = c.N; p.K = c.K;
-    p.tiles_m = p.tiles_n = 0;
-    p.alpha = (float)c.alpha;
-    p.beta = (float)c.beta;
-    const bool ak = !c.tA, bk = c.tB;
-    if (ak && bk) return launch_hg_layout<true, true>(p, c.count);
-    if (ak) return launch_hg_layout<true, false>(p, c.count);
-    if (bk) return launch_hg_layout<false, true>(p, c.count);
-    return launch_hg_layout<false, false>(p, c.count);
-}
+}  // namespace g9
+#include "hgemm_launch.h"
+namespace g9 {
 
 // ---------------- FP32 whole-tile kernel ----------------
 // Classes, largest tile first; a product takes the first class whose whole tiles fill the CUs (128×128: twice over,
@@ -463,13 +392,16 @@ static int launch_typed(const GemmCall &c) {
 // element, each C element rounded once; the two layouts those routines use: A and B both k-contiguous, or both
 // mn-contiguous. FP32 and FP64 take 64×64 tiles: at n = 4096 their 2080 tiles keep every CU busy to the end (FP32
 // SYRK 0.71 ms, FP64 1.21), where 128×128 tiles (528) left a nearly empty last round (1.02, 1.58).
-template <class T, int TRI, bool AK, bool BKC>
+template <class T, int TRI, bool AK, bool BKC, bool CHECKED = false>
 static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
-    constexpr TileCfg C = sizeof(T) == 2 ? TileCfg{128, 128, 2, 2} : TileCfg{64, 64, 2, 2};
+    constexpr TileCfg C = sizeof(T) == 2 && !CHECKED ? TileCfg{128, 128, 2, 2} : TileCfg{64, 64, 2, 2};
+    if constexpr (!CHECKED) {
+        if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_tri_t<T, TRI, AK, BKC, true>(p);
+    }
     p.tiles_m = p.tiles_n = (p.M + C.BM - 1) / C.BM;
     const long long tiles = (long long)p.tiles_m * (p.tiles_m + 1) / 2;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product too large (%d tiles per side)", p.tiles_m);
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI, 0, 1, CHECKED>), dim3((unsigned)tiles),
                        dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
@@ -514,13 +446,13 @@ int launch_gemm_tri(const GemmCall &c, bool lower) {
 // range is cut to where the triangle is non-zero (klim as gemm_kernel's KLIM), one launch over every tile of C,
 // longest ranges dispatched first; the small tiles when the big ones are fewer than the CUs. Layout NN only (both
 // operands as stored), one product.
-template <class T, TileCfg C, int KLIM>
+template <class T, TileCfg C, int KLIM, bool CHECKED = false>
 static int launch_klim_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     p.tiles_m = (p.M + C.BM - 1) / C.BM;
     p.tiles_n = (p.N + C.BN - 1) / C.BN;
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles)", p.tiles_m, p.tiles_n);
-    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM>;
+    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM, 1, CHECKED>;
     p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(C.WM * C.WN * 64));
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
@@ -552,6 +484,7 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
     const auto go = [&](auto kc) -> int {
         constexpr int K = decltype(kc)::value;
+        if (!unchecked_ok<T>(true, p.lda) || !unchecked_ok<T>(false, p.ldb)) return launch_klim_t<T, tiny, K, true>(p, c.count);
         if (cls == 0) return launch_klim_t<T, CF::big, K>(p, c.count);
         if constexpr (dbl) {
             if (cls == 2) return launch_klim_t<T, tiny, K>(p, c.count);
@@ -583,7 +516,10 @@ int launch_gemm_klim(const GemmCall &c, int klim) {
 int launch_gemm(const GemmCall &c) {
     switch (c.type) {
     case GEN9BLAS_H:
-    case GEN9BLAS_HS: return hgemm_tiles_apply(c) ? launch_hgemm_tiles(c) : launch_typed<f16>(c);
+    case GEN9BLAS_HS: {
+        int rc = 0;
+        return launch_hgemm_tiles(c, &rc) ? rc : launch_typed<f16>(c);
+    }
     case GEN9BLAS_S: return launch_sgemm(c);
     case GEN9BLAS_D: return launch_typed<double>(c);
     }

@@ -67,6 +67,8 @@ struct Params {
     long long lda, ldb, ldc, sA, sB, sC;
     int M, N, K, tiles_m, tiles_n;
     float alpha, beta;
+    float *P = nullptr;   // SPLIT: partial sums, kper of k per slice (a multiple of KB, at least two of them)
+    int kper = 0;
 };
 
 // Global → LDS loads of one operand tile: RT rows (m or n) × KB k, RT·KB·2 bytes, issued by NW waves (counted in FP16
@@ -85,7 +87,11 @@ template <int RT, bool X3 = false> __device__ __forceinline__ int mnswz(int k) {
     static_assert(RT >= 64, "an mn-contiguous row holds at least 8 chunks");
     return (RT >= 128 ? 4 * (k & 3) : 4 * ((k >> 1) & 1)) ^ (X3 ? 2 * ((k >> 3) & 1) : 0);
 }
-template <int RT, int KB, int NW, bool KC, int MS = 0>
+// EDGE: the tile may cross the matrix's last row or column: rows (starts of 16-byte chunks) past the end are moved back
+// onto the last one, whose values no stored element uses. A chunk that straddles the end of an mn-contiguous row reads
+// on into the next row, so a k-step that holds the matrix's last k is not loaded this way then: checked() takes it
+// through registers, with zeros outside the matrix (also for a k-step that K does not fill). T: the element type.
+template <int RT, int KB, int NW, bool KC, int MS = 0, bool EDGE = false, class T = f16>
 struct Loader {
     static constexpr int NINST = RT * KB * 2 / 1024;       // 1 KiB instructions per tile
     static constexpr int NI = NINST / NW;                  // per wave
@@ -93,32 +99,44 @@ struct Loader {
                                                                           // instruction, rows per 256 bytes
     static constexpr int CPR = RT / 8, RPI = 512 / RT;                    // mn-contiguous: chunks per row, rows per
                                                                           // instruction
+    static constexpr int V = 16 / (int)sizeof(T);
     static_assert(NINST % NW == 0, "tile instructions must divide over the waves");
     static_assert(!KC || (RPIK * NW) % 32 == 0, "k-contiguous swizzle must repeat over a wave's instructions");
     static_assert(KC || ((RT >= 128 || (RT == 64 && MS != 1)) && (RPI * NW) % (MS == 2 ? 16 : MS ? 8 : 4) == 0),
                   "mn-contiguous swizzle must repeat over a wave's instructions");
+    static constexpr int NV = EDGE && KC ? NI : 1;
     const char *org;      // wave-uniform: tile origin at the next k-step to load
-    unsigned voff;        // this lane's byte offset for instruction 0
+    unsigned voff[NV];    // this lane's byte offset for instruction 0 (EDGE, k-contiguous: for each instruction)
     long long step_i;     // bytes between consecutive instructions of this wave
     long long step_k;     // bytes per k-step
 
-    __device__ __forceinline__ void init(const f16 *X, long long ld, int mn0, int wave, int lane) {
+    // This lane's row and logical chunk of instruction i: k-contiguous, row of the tile and chunk of k; mn-contiguous,
+    // k-row and chunk of mn.
+    static __device__ __forceinline__ int row(int i, int wave, int lane) {
+        return KC ? RPIK * (wave + NW * i) + lane / CPRK : RPI * (wave + NW * i) + lane / CPR;
+    }
+    static __device__ __forceinline__ int chunk(int wave, int lane) {
+        const int r = row(0, wave, lane);   // the swizzle repeats over a wave's instructions
+        if constexpr (KC) return (lane % CPRK) ^ kswz<KB>(r);
+        else return (lane % CPR) ^ (MS == 1 ? 8 * ((r >> 2) & 1) : mnswz<RT, MS == 2>(r));
+    }
+    // ld and mn0 in FP16 elements; MN (EDGE): rows or columns of the matrix in elements T from the tile's origin on.
+    __device__ __forceinline__ void init(const f16 *X, long long ld, int mn0, int wave, int lane, int MN = 0) {
+        const int r = row(0, wave, lane), c = chunk(wave, lane);
         if constexpr (KC) {
             // instruction j = wave + NW·i covers rows RPIK·j ..; lane L: row RPIK·j + L / CPRK, physical chunk L % CPRK
-            const int r = RPIK * wave + lane / CPRK;
-            const int c = (lane % CPRK) ^ kswz<KB>(r);
             org = reinterpret_cast<const char *>(X + (long long)mn0 * ld);
-            voff = (unsigned)(((long long)r * ld + 8 * c) * 2);
-            step_i = (long long)RPIK * NW * ld * 2;
+            step_i = EDGE ? 0 : (long long)RPIK * NW * ld * 2;
             step_k = KB * 2;
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                voff[i] = (unsigned)(((long long)(EDGE ? min(row(i, wave, lane), MN - 1) : r) * ld + 8 * c) * 2);
         } else {
             // instruction j covers k rows RPI·j ..; lane L: row RPI·j + L / CPR, physical chunk L % CPR
-            const int k = RPI * wave + lane / CPR;
-            const int c = (lane % CPR) ^ (MS == 1 ? 8 * ((k >> 2) & 1) : mnswz<RT, MS == 2>(k));
             org = reinterpret_cast<const char *>(X + mn0);
-            voff = (unsigned)(((long long)k * ld + 8 * c) * 2);
             step_i = (long long)RPI * NW * ld * 2;
             step_k = (long long)KB * ld * 2;
+            voff[0] = (unsigned)((long long)r * ld * 2 + (EDGE ? min(16 * c, (MN - 1) / V * 16) : 16 * c));
         }
     }
     // Issues this wave's loads of the next k-step into the tile at LDS address `dst`, then advances.
@@ -129,9 +147,21 @@ struct Loader {
     }
     // Instruction i of this wave's loads of the current k-step; advance() moves to the next k-step.
     __device__ __forceinline__ void one(int i, unsigned dst, int wave) const {
-        lds_dma16(org + i * step_i, voff, dst + 1024 * (wave + NW * i));
+        lds_dma16(org + (EDGE && KC ? 0 : i * step_i), voff[EDGE && KC ? i : 0], dst + 1024 * (wave + NW * i));
     }
     __device__ __forceinline__ void advance(bool more) { if (more) org += step_k; }
+    // EDGE: the k-step from k0 on of the matrix whose tile starts at X (MN rows or columns, K of k from there on, row
+    // stride ld, in elements T), loaded through registers into the tile at `dst`.
+    static __device__ __forceinline__ void checked(const T *X, long long ld, int MN, int K, int k0, G9_LDS unsigned char *dst,
+                                                   int wave, int lane) {
+        const int c = chunk(wave, lane);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int r = row(i, wave, lane);
+            const dma_u32x4 v = KC ? load16<T>(X, ld, r, k0 + V * c, MN, K) : load16<T>(X, ld, k0 + r, V * c, K, MN);
+            *reinterpret_cast<G9_LDS dma_u32x4 *>(dst + 1024 * (wave + NW * i) + 16 * lane) = v;
+        }
+    }
 };
 
 // Fragment reads of one operand for a wave's TT MFMA tiles (16 rows of m or n each, starting at wave row w0): per
@@ -183,17 +213,47 @@ __device__ __forceinline__ f32x4 mma(u32x4 b, u32x4 a, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
 }
 
+// C[0 .. 7] = alpha·(lo, hi) + beta·C (C not read when beta = 0), rounded once, for the first `valid` of them; one
+// 16-byte access at element alignment when all eight are inside C.
+__device__ __forceinline__ void store8(f16 *c, f32x4 lo, f32x4 hi, float alpha, float beta, int valid) {
+    typedef f16 f16x8u __attribute__((ext_vector_type(8), aligned(2)));
+    if (valid >= 8) {
+        f16x8u o = {}, v;
+        if (beta != 0.f) o = *reinterpret_cast<const f16x8u *>(c);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x = alpha * (e < 4 ? lo[e & 3] : hi[e & 3]);
+            v[e] = (f16)(beta != 0.f ? __builtin_fmaf(beta, (float)o[e], x) : x);
+        }
+        __builtin_nontemporal_store(v, reinterpret_cast<f16x8u *>(c));
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        if (e < valid) {
+            const float x = alpha * (e < 4 ? lo[e & 3] : hi[e & 3]);
+            c[e] = (f16)(beta != 0.f ? __builtin_fmaf(beta, (float)c[e], x) : x);
+        }
+}
+
 // RA (read-ahead): the main loop reads each k-step's fragments one k-step early (for small wave tiles, whose few
 // MFMAs per k-step cannot cover the LDS read latency inside the k-step).
-template <int BM, int BN, int WM, int WN, int KB, int NS, bool AK, bool BKC, bool RA = false>
+// EDGE: tiles may cross the last row or column of C, and K need not be whole k-steps (at least two of them, counting
+// the last); operands at 4-byte, C at element alignment. All k-steps run the same pipeline; the one the loaders cannot
+// copy directly (EDGE in Loader) is taken first, through registers.
+// SPLIT: blockIdx.y is a slice of K (count 1); each workgroup leaves its unscaled FP32 sums in P, accumulator by
+// accumulator (64 lanes × 16 bytes), for split_sum.
+template <int BM, int BN, int WM, int WN, int KB, int NS, bool AK, bool BKC, bool RA = false, bool EDGE = false,
+          bool SPLIT = false>
 __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
     constexpr int NW = WM * WN;
     constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16;
     constexpr int ABYTES = BM * KB * 2, BBYTES = BN * KB * 2, SBYTES = ABYTES + BBYTES;
     constexpr int NSUB = KB / 32;
     constexpr bool AX3 = !AK && !BKC;   // TN: A's transposing reads take the bit-3 swizzle term
-    using LA = Loader<BM, KB, NW, AK, AX3 ? 2 : 0>;
-    using LB = Loader<BN, KB, NW, BKC>;
+    using LA = Loader<BM, KB, NW, AK, AX3 ? 2 : 0, EDGE>;
+    using LB = Loader<BN, KB, NW, BKC, 0, EDGE>;
+    static_assert(EDGE || !SPLIT, "split K: edge-capable tiles");
     constexpr int LPS = LA::NI + LB::NI;   // loads per stage per wave
     static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32 (n tiles come in pairs)");
     static_assert(NSUB % 2 == 0, "fragment double buffer alternates over an even number of substeps");
@@ -217,14 +277,24 @@ __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
     const int m0 = (first_m + in_group % gsz) * BM, n0 = (in_group / gsz) * BN;
 
     const long long z = blockIdx.y;
-    const f16 *A = p.A + z * p.sA;
-    const f16 *B = p.B + z * p.sB;
-    f16 *C = p.C + z * p.sC;
+    int K = p.K;
+    const f16 *A = p.A, *B = p.B;
+    f16 *C = p.C;
+    if constexpr (SPLIT) {
+        const long long k0 = z * p.kper;
+        K = min(p.kper, p.K - (int)k0);
+        A += AK ? k0 : k0 * p.lda;
+        B += BKC ? k0 : k0 * p.ldb;
+    } else {
+        A += z * p.sA;
+        B += z * p.sB;
+        C += z * p.sC;
+    }
 
     LA la;
     LB lb;
-    la.init(A, p.lda, m0, wave, lane);
-    lb.init(B, p.ldb, n0, wave, lane);
+    la.init(A, p.lda, m0, wave, lane, p.M - m0);
+    lb.init(B, p.ldb, n0, wave, lane, p.N - n0);
     Frags<BM, KB, TM, AK, false, AX3> fa;
     Frags<BN, KB, TN, BKC, true> fb;
     fa.init(wm * WTM, lane);
@@ -236,17 +306,42 @@ __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
 #pragma unroll
         for (int j = 0; j < TM; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nk = p.K / KB;
+    // EDGE: the checked k-step first (when there is one), then the direct ones
+    const int tail = !EDGE ? 0 : K % KB ? K % KB : (!AK && p.M % 8 && m0 + BM > p.M) || (!BKC && p.N % 8 && n0 + BN > p.N) ? KB : 0;
+    const int nk = EDGE ? (K + KB - 1) / KB : K / KB;
+    if constexpr (SPLIT) {
+        // a last slice that is one checked k-step: the ring's copies, whose values nobody uses, read the k-step before
+        // it (of the slice before: the first slice is longer)
+        if (tail && nk == 1) { la.org -= la.step_k; lb.org -= lb.step_k; }
+    }
     // prologue: k-steps 0 .. NS-1 into stages 0 .. NS-1 (past the last k-step, the last one is loaded again into a
     // stage nobody reads, so every k-step issues the same number of loads), then wait for k-step 0
 #pragma unroll
     for (int s = 0; s < NS; s++) {
+        if (EDGE && s == 0 && tail) continue;
         la.issue(lds_addr + s * SBYTES, wave);
         lb.issue(lds_addr + s * SBYTES + ABYTES, wave);
         if (s + 1 >= nk) { la.org -= la.step_k; lb.org -= lb.step_k; }
     }
+    if constexpr (EDGE) {
+        if (tail) {
+            LA::checked(AK ? A + (long long)m0 * p.lda : A + m0, p.lda, p.M - m0, K, K - tail, lds, wave, lane);
+            LB::checked(BKC ? B + (long long)n0 * p.ldb : B + n0, p.ldb, p.N - n0, K, K - tail, lds + ABYTES, wave, lane);
+        }
+    }
     wait_vm<(NS - 1) * LPS>();
     __syncthreads();
+    if constexpr (EDGE) {
+        // What the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes
+        // the compiler wait for all LDS reads of a substep at once (scalar loads and LDS reads share a counter). The
+        // accumulators' zeros are hidden from the compiler: as one shared constant they cost register copies per k-step.
+        asm volatile("" : "+s"(C), "+s"(p.P), "+s"(p.ldc), "+s"(p.M), "+s"(p.N));
+        wait_lgkm0();
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int j = 0; j < TM; j++) asm volatile("" : "+v"(acc[i][j]));
+    }
 
     if constexpr (RA) {
         // Read-ahead: the fragments of a whole k-step are read one k-step before its MFMAs use them (two register
@@ -385,6 +480,17 @@ __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
     // workgroup stores its tile at about the same time at the end (n = 2048: 832 → 856 TFLOP/s, n = 4096:
     // 1330 → 1350, in alternating runs of both builds; the FP32 kernel's stores lose with it, 87.5 → 84.3 at
     // n = 1024).
+    if constexpr (SPLIT) {
+        f32x4 *P = reinterpret_cast<f32x4 *>(p.P) +
+                   (((z * (p.tiles_m * p.tiles_n) + (m0 / BM) * p.tiles_n + n0 / BN) * NW + wave) * (TM * TN)) * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+            if (m0 + wm * WTM + j * 16 + (lane & 15) < p.M) {
+#pragma unroll
+                for (int i = 0; i < TN; i++) P[(j * TN + i) * 64] = acc[i][j];
+            }
+        return;
+    }
     const float alpha = p.alpha, beta = p.beta;
     const int g = lane >> 4;
 #pragma unroll
@@ -392,7 +498,12 @@ __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
 #pragma unroll
         for (int j = 0; j < TM; j++) {
             const int m = m0 + wm * WTM + j * 16 + (lane & 15);
-            f16 *cp = C + (long long)m * p.ldc + n0 + wn * WTN + 32 * pp + 8 * g;
+            const int n = n0 + wn * WTN + 32 * pp + 8 * g;
+            f16 *cp = C + (long long)m * p.ldc + n;
+            if constexpr (EDGE) {
+                if (m < p.M) store8(cp, acc[2 * pp][j], acc[2 * pp + 1][j], alpha, beta, p.N - n);
+                continue;
+            }
             union { u32x4 w; f16 e[8]; } o, v;
             if (beta != 0.f) o.w = *reinterpret_cast<const u32x4 *>(cp);
 #pragma unroll
@@ -402,6 +513,30 @@ __global__ void __launch_bounds__(WM *WN * 64) hgemm_kernel(Params p) {
             }
             __builtin_nontemporal_store(v.w, reinterpret_cast<u32x4 *>(cp));
         }
+}
+
+// Finish of a SPLIT product on BM × BN tiles of WM × WN waves: the slices' sums added in slice order, then alpha / beta and
+// one rounding. A workgroup of 256 takes four (wave tile, pair of n tiles, m tile) groups of 64 lanes, each lane the 8
+// consecutive n of one row that it held in the product.
+template <int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(256) split_sum(Params p, int slices) {
+    constexpr int NW = WM * WN, WTM = BM / WM, WTN = BN / WN, TM = WTM / 16, TN = WTN / 16, PER = NW * TM * (TN / 2);
+    const int lane = threadIdx.x & 63;
+    const long long q = (long long)blockIdx.x * 4 + (threadIdx.x >> 6), tiles = (long long)p.tiles_m * p.tiles_n;
+    const long long tile = q / PER;
+    if (tile >= tiles) return;
+    const int u = (int)(q % PER), wave = u / (TM * (TN / 2)), j = u / (TN / 2) % TM, pp = u % (TN / 2);
+    const int m = (int)(tile / p.tiles_n) * BM + (wave % WM) * WTM + j * 16 + (lane & 15);
+    const int n = (int)(tile % p.tiles_n) * BN + (wave / WM) * WTN + 32 * pp + 8 * (lane >> 4);
+    if (m >= p.M || n >= p.N) return;
+    const f32x4 *P = reinterpret_cast<const f32x4 *>(p.P) + ((tile * NW + wave) * (TM * TN) + j * TN + 2 * pp) * 64 + lane;
+    const long long slice = tiles * NW * (TM * TN) * 64;
+    f32x4 lo = P[0], hi = P[64];
+    for (int s = 1; s < slices; s++) {
+        lo += P[s * slice];
+        hi += P[s * slice + 64];
+    }
+    store8(p.C + (long long)m * p.ldc + n, lo, hi, p.alpha, p.beta, p.N - n);
 }
 
 }  // namespace hg

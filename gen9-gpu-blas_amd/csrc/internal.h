@@ -50,6 +50,9 @@ G9_HIDDEN void set_fixed_workspace(void *base, size_t bytes, const char *who);
 // A split of s > 1 slices is chosen only while tiles · s ≤ CUs, so the slices of one product never exceed
 // CUs × this many bytes (the launch asserts every split tile against it).
 constexpr size_t SPLITK_TILE_BYTES_MAX = 256 * 256 * 4;
+// The split-K work space (SLOT_P) at its bound of num_cus × SPLITK_TILE_BYTES_MAX bytes, or null (with no error set) when
+// there is no memory for it.
+G9_HIDDEN void *splitk_workspace();
 // Set-up of the no-allocation entry point on `dev` (called by init with `dev` current): finds the device address of
 // its static work space. A failure is kept and reported by that entry point only.
 G9_HIDDEN void noalloc_setup(int dev);

@@ -1,5 +1,6 @@
-// Direct global→LDS copies (global_load_lds_dwordx4) and the waits that go with them, shared by the FP16 GEMM and
-// the skinny kernels.
+// Direct global→LDS copies (global_load_lds_dwordx4) and the waits that go with them, shared by the FP16 and FP32 GEMM
+// and the skinny kernels, and 16-byte loads at element alignment. The copies' global addresses need 4-byte alignment
+// (a streaming probe on MI355X reads 1 GiB at 6.3-6.4 TB/s at 4-, 8-, 12- and 16-byte alignment alike).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -30,6 +31,41 @@ template <int MAXS, int LPS> __device__ __forceinline__ void wait_vm_stages(int 
     } else {
         wait_vm<0>();
     }
+}
+
+typedef unsigned int dma_u32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes at an address aligned to the element type only: one global_load_dwordx4 either way (the GPU serves it at
+// any element alignment, at the aligned rate when the address is aligned).
+template <class T> __device__ __forceinline__ dma_u32x4 load16u(const T *p) {
+    typedef T TV __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+    const TV v = *reinterpret_cast<const TV *>(p);
+    return __builtin_bit_cast(dma_u32x4, v);
+}
+
+// 16 bytes (V elements) of row r, columns c .. c+V-1 of a row-major matrix X (R valid rows, Cc valid columns, row
+// stride ld); zero outside the valid region. A chunk that crosses the last column is the row's last 16 bytes, shifted:
+// one load as for any other chunk (a load per element there waits for each of them: FP16 1000³, whose K leaves every
+// tile such a k-step, took 9.8 µs against 6.7 for 1024³). SHIFT false: element by element, in fewer registers.
+template <class T, bool SHIFT = true>
+__device__ __forceinline__ dma_u32x4 load16(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
+    constexpr int V = 16 / sizeof(T);
+    if (r >= R || c >= Cc) return dma_u32x4{0, 0, 0, 0};
+    const T *row = X + (long long)r * ld;
+    if (SHIFT && Cc >= V) {
+        const int cc = min(c, Cc - V), bytes = (c - cc) * (int)sizeof(T);
+        dma_u32x4 v = load16u(row + cc);
+        if (bytes & 8) v = dma_u32x4{v[2], v[3], 0, 0};
+        if (sizeof(T) < 8 && (bytes & 4)) v = dma_u32x4{v[1], v[2], v[3], 0};
+        if (sizeof(T) < 4 && (bytes & 2))
+            v = dma_u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+        return v;
+    }
+    if (!SHIFT && c + V <= Cc) return load16u(row + c);
+    union { dma_u32x4 v; T e[V]; } u;
+#pragma unroll
+    for (int e = 0; e < V; e++) u.e[e] = c + e < Cc ? row[c + e] : T(0);
+    return u.v;
 }
 
 }  // namespace g9

@@ -172,6 +172,15 @@ int scratch(int slot, size_t bytes, void **p) {
     return 0;
 }
 
+void *splitk_workspace() {
+    void *p = nullptr;
+    if (scratch(SLOT_P, (size_t)num_cus * SPLITK_TILE_BYTES_MAX, &p)) {
+        gst = 0;
+        return nullptr;
+    }
+    return p;
+}
+
 // ---------------- operand resolution ----------------
 int mem_kind(const void *p, size_t bytes) {
     if (!p) return MEM_HOST;
