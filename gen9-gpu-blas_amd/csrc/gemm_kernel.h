@@ -427,13 +427,14 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
             constexpr int NVM = SA::N16 + SB::N16;
             constexpr int NWR = (AK ? SA::N16 : SA::NB * 8) + (BKC ? SB::N16 : SB::NB * 8);
             // global loads first, then group 0's fragments; each later group: its MFMAs interleaved with the next
-            // group's reads, and over the last two groups the LDS writes of the next tile
+            // group's reads, and in the last group the LDS writes of the next tile (FP64 n = 4096 NN 70.8 TFLOP/s; over
+            // the last two groups 69.7; without the pinned order 62.8)
             __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, NVM, 0);
             __builtin_amdgcn_sched_group_barrier(SG_DS_READ, NRD, 0);
 #pragma unroll
             for (int q = 0; q < QG; q++) {
                 const int nrd = q + 1 < QG ? NRD : 0;
-                const int nwr = q >= QG - 2 ? (q == QG - 1 ? NWR - NWR / 2 : NWR / 2) : 0;
+                const int nwr = q == QG - 1 ? NWR : 0;
 #pragma unroll
                 for (int t = 0; t < NMF; t++) {
                     __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);

@@ -1,8 +1,7 @@
 // Host side of the MFMA GEMM: tile configuration per type and dispatch over the transpose layouts.
-// The kernel templates and their design notes are in gemm_kernel.h (every shape and type) and sgemm_kernel.h (FP32,
-// whole tiles, direct global→LDS loads); hgemm_launch.h holds the FP16 products on direct global→LDS loads.
+// The kernel templates and their design notes are in gemm_kernel.h (every shape and type); hgemm_launch.h and
+// sgemm_launch.h hold the FP16 and FP32 products on direct global→LDS loads.
 #include "gemm_kernel.h"
-#include "sgemm_kernel.h"
 #include <stdlib.h>
 #include <string.h>
 #include <algorithm>
@@ -161,57 +160,7 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
 #include "hgemm_launch.h"
 namespace g9 {
 
-// ---------------- FP32 whole-tile kernel ----------------
-// Classes, largest tile first; a product takes the first class whose whole tiles fill the CUs (128×128: twice over,
-// else the 64×64 tiles of several rounds finish sooner: 2048³ 129 → 125 µs, 2048×2048×1024 68 → 66, the triangular
-// solve's 1024×4096×1024 with beta = 1 70.3 → 67.1) and cover at least 90 % of C. Measured on MI355X (TFLOP/s,
-// sustained, against the general kernel of gemm_kernel.h in the same runs):
-// - 128×256 tiles, 8 waves of 64×64, two stages, sums blocked per 128 k: n = 4096 NN 144.9 (124.6), NT 144.3
-//   (130.8); 8192×8192×2048 144.1 (123.4); 2944×11008×4096 NT β = 0.5 140.0 (127.9). Three stages 142.6, blocks of
-//   32 k 134.3, of 64 k 140.3, of 256 k 142.6; 256×128 tiles 142.7;
-// - 128×128 tiles, 8 waves of 64×32, three stages, 128-k blocks: n = 2048 134.4 (121.4; 4 waves of 64×64: 129.7;
-//   64×64 tiles: 132.4; a later build read 133.0 against 137.2 for the 64×64 tiles, which n = 2048 now takes);
-// - 64×64 tiles, 4 waves of 32×32, four stages, 256-k blocks: n = 1024 102.6 (87.7; 128-k blocks 101.9, 32-k blocks
-//   90.9; three stages 94.0, six 93.0, eight 92.2).
-// The rows and columns beyond the whole tiles (an M or N that is not a multiple of the tile) go to the general
-// kernel, each C element still computed by exactly one of the launches; a bottom strip of r rows over a width that is
-// a multiple of 64 instead takes 64×64 whole tiles on the last ⌈r/64⌉·64 rows, storing only its own r rows
-// (3000×11008×4096 NT β = 0.5: 2.04 → 1.99 ms, the 56-row strip about 146 → 99 µs).
-template <class T> static int launch_typed(const GemmCall &c);
-struct SgClass { int BM, BN; };
-static constexpr SgClass SG_CLASSES[] = {{128, 256}, {128, 128}, {64, 64}};
-template <int BM, int BN, int WM, int WN, int NS, int BLK, bool AK, bool BKC>
-static int launch_sg(const sg::Params &p0, int count) {
-    sg::Params p = p0;
-    p.tiles_m = p.M / BM;
-    p.tiles_n = p.N / BN;
-    const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)count), block(WM * WN * 64);
-    hipLaunchKernelGGL((sg::sgemm_kernel<BM, BN, WM, WN, NS, AK, BKC, BLK>), grid, block, 0, stream, p);
-    G9_HIP(hipGetLastError());
-    return 0;
-}
-template <bool AK, bool BKC>
-static int launch_sg_layout(const sg::Params &p, int count, int cls) {
-    if (cls == 0) return launch_sg<128, 256, 2, 4, 2, 4, AK, BKC>(p, count);
-    if (cls == 1) return launch_sg<128, 128, 2, 4, 3, 4, AK, BKC>(p, count);
-    return launch_sg<64, 64, 2, 2, 4, 8, AK, BKC>(p, count);
-}
-// The FP32 whole-tile kernel applies to 16-byte aligned operands with 16-byte row strides and K a multiple of 32,
-// unless GEN9BLAS_SGEMM=generic or a forced split-K (GEN9BLAS_SPLITK) asks for the general kernel.
-static bool sgemm_tiles_ok(const GemmCall &c) {
-    static int generic = -1;
-    if (generic < 0) {
-        const char *e = getenv("GEN9BLAS_SGEMM");
-        generic = e && !strcmp(e, "generic");
-    }
-    if (generic || splitk_forced() >= 0 || c.K % 32 || c.count > 65535) return false;
-    const long long es = 4;
-    // each lane's byte offset inside a tile is 32-bit
-    if (c.lda * es * 256 >= (1LL << 32) || c.ldb * es * 256 >= (1LL << 32)) return false;
-    return (uintptr_t)c.A % 16 == 0 && (uintptr_t)c.B % 16 == 0 && (uintptr_t)c.C % 16 == 0 && (c.lda * es) % 16 == 0 &&
-           (c.ldb * es) % 16 == 0 && (c.ldc * es) % 16 == 0 &&
-           (c.count == 1 || ((c.sA * es) % 16 == 0 && (c.sB * es) % 16 == 0 && (c.sC * es) % 16 == 0));
-}
+// ---------------- FP32 on direct global→LDS loads ----------------
 // Workgroups of KERN (threads each) that one CU holds at once, from the runtime's occupancy query (1 if it fails).
 template <auto KERN> static int wgs_per_cu(int threads) {
     static const int occ = [threads] {
@@ -225,149 +174,9 @@ template <auto KERN> static int wgs_per_cu(int threads) {
 // the later half starts as CUs free up, and the longest-first order balances better.
 static int klim_pair(long long tiles, int per_cu) { return tiles > num_cus && tiles <= 2LL * num_cus && per_cu >= 2; }
 
-// Triangle (TRI) and k-limited (KLIM) modes of the FP32 whole-tile kernel for SYRK / SYR2K / TRMM: one product,
-// whole tiles (the callers check), `tiles` workgroups.
-template <int BM, int BN, int WM, int WN, int NS, int BLK, bool AK, bool BKC, int TRI, int KLIM>
-static int launch_sg_mode(const sg::Params &p0, long long tiles, int count = 1) {
-    constexpr auto kern = sg::sgemm_kernel<BM, BN, WM, WN, NS, AK, BKC, BLK, TRI, KLIM>;
-    sg::Params p = p0;
-    p.tiles_m = p.M / BM;
-    p.tiles_n = p.N / BN;
-    if constexpr (KLIM != 0) p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(WM * WN * 64));
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(WM * WN * 64), 0, stream, p);
-    G9_HIP(hipGetLastError());
-    return 0;
-}
-static sg::Params sg_params(const GemmCall &c) {
-    sg::Params p;
-    p.A = reinterpret_cast<const float *>(c.A);
-    p.B = reinterpret_cast<const float *>(c.B);
-    p.C = reinterpret_cast<float *>(c.C);
-    p.lda = c.lda; p.ldb = c.ldb; p.ldc = c.ldc;
-    p.sA = c.sA; p.sB = c.sB; p.sC = c.sC;
-    p.M = c.M; p.N = c.N; p.K = c.K;
-    p.tiles_m = p.tiles_n = 0;
-    p.alpha = (float)c.alpha;
-    p.beta = (float)c.beta;
-    return p;
-}
-// Triangle of an FP32 square product on the whole-tile kernel (NT or TN): 128×128 or 64×64 tiles, whichever fills
-// its last round of one workgroup per CU better (n = 4096: 528 tiles of 128×128 are 2.06 rounds, SYRK 90 TFLOP/s;
-// 2080 of 64×64 fill 90 % of 9 rounds), when the triangle has at least one such tile per CU. Returns false (nothing
-// launched) when neither applies; *rc is the launch's status otherwise.
-template <int TRI, bool AK, bool BKC>
-static bool sg_tri_layout(const GemmCall &c, int *rc) {
-    const sg::Params p = sg_params(c);
-    const long long t128 = (long long)(c.M / 128) * (c.M / 128 + 1) / 2, t64 = (long long)(c.M / 64) * (c.M / 64 + 1) / 2;
-    const auto fill = [](long long t) { return (double)t / (double)(((t + num_cus - 1) / num_cus) * num_cus); };
-    const bool ok128 = c.M % 128 == 0 && t128 >= num_cus, ok64 = c.M % 64 == 0 && t64 >= num_cus;
-    if (ok128 && (!ok64 || fill(t128) >= fill(t64))) *rc = launch_sg_mode<128, 128, 2, 4, 3, 4, AK, BKC, TRI, 0>(p, t128);
-    else if (ok64) *rc = launch_sg_mode<64, 64, 2, 2, 4, 8, AK, BKC, TRI, 0>(p, t64);
-    else return false;
-    return true;
-}
-static bool sg_tri(const GemmCall &c, bool lower, int *rc) {
-    if (c.M != c.N || c.count != 1 || !sgemm_tiles_ok(c)) return false;
-    if (!c.tA && c.tB) return lower ? sg_tri_layout<1, true, true>(c, rc) : sg_tri_layout<2, true, true>(c, rc);
-    if (c.tA && !c.tB) return lower ? sg_tri_layout<1, false, false>(c, rc) : sg_tri_layout<2, false, false>(c, rc);
-    return false;
-}
-// k-limited FP32 NN product (or strided batch of them) on the whole-tile kernel (TRMM, the triangular solves): the
-// plain products' classes, whole tiles only. A batch takes the big classes only with two tiles per CU or more, so
-// that tiles of long and short k ranges share the CUs (TRSV's E_q = inv(D_q)·C_q, 512³ × 31: 128×128 tiles 80 µs
-// in a kernel trace; on 64×64 tiles the n = 16384 solve takes 385 against 400 µs).
-template <int KLIM>
-static bool sg_klim_mode(const GemmCall &c, int *rc) {
-    const sg::Params p = sg_params(c);
-    const long long t0 = (long long)(c.M / 128) * (c.N / 256), t1 = (long long)(c.M / 128) * (c.N / 128),
-                    t2 = (long long)(c.M / 64) * (c.N / 64), nb = c.count;
-    const long long want = nb > 1 ? 2LL * num_cus : num_cus;
-    if (c.M % 128 == 0 && c.N % 256 == 0 && t0 * nb >= want)
-        *rc = launch_sg_mode<128, 256, 2, 4, 2, 4, true, false, 0, KLIM>(p, t0, c.count);
-    else if (c.M % 128 == 0 && c.N % 128 == 0 && t1 * nb >= want)
-        *rc = launch_sg_mode<128, 128, 2, 4, 3, 4, true, false, 0, KLIM>(p, t1, c.count);
-    else if (c.M % 64 == 0 && c.N % 64 == 0 && t2 * nb >= num_cus)
-        *rc = launch_sg_mode<64, 64, 2, 2, 4, 8, true, false, 0, KLIM>(p, t2, c.count);
-    else return false;
-    return true;
-}
-static bool sg_klim(const GemmCall &c, int klim, int *rc) {
-    // the k range of every tile is non-empty only when K spans the triangular operand's order
-    if (c.count < 1 || c.tA || c.tB || !sgemm_tiles_ok(c) || (klim <= 2 ? c.K != c.M : c.K != c.N)) return false;
-    switch (klim) {
-    case 1: return sg_klim_mode<1>(c, rc);
-    case 2: return sg_klim_mode<2>(c, rc);
-    case 3: return sg_klim_mode<3>(c, rc);
-    case 4: return sg_klim_mode<4>(c, rc);
-    }
-    return false;
-}
-
-// The part of an FP32 product in rows [m0, m0 + M) and columns [n0, n0 + N) of C, as a product of its own.
-static GemmCall sub_call(const GemmCall &c, int m0, int M, int n0, int N) {
-    GemmCall s = c;
-    const float *A = reinterpret_cast<const float *>(c.A), *B = reinterpret_cast<const float *>(c.B);
-    s.A = A + (c.tA ? (long long)m0 : (long long)m0 * c.lda);
-    s.B = B + (c.tB ? (long long)n0 * c.ldb : (long long)n0);
-    s.C = reinterpret_cast<float *>(c.C) + (long long)m0 * c.ldc + n0;
-    s.M = M;
-    s.N = N;
-    return s;
-}
-static int launch_sgemm(const GemmCall &c) {
-    if (!sgemm_tiles_ok(c)) return launch_typed<float>(c);
-    int cls = -1, Mi = 0, Ni = 0;
-    for (int k = 0; k < 3 && cls < 0; k++) {
-        const int mi = c.M / SG_CLASSES[k].BM * SG_CLASSES[k].BM, ni = c.N / SG_CLASSES[k].BN * SG_CLASSES[k].BN;
-        const long long tiles = (long long)(mi / SG_CLASSES[k].BM) * (ni / SG_CLASSES[k].BN) * c.count;
-        if (tiles >= (k == 1 ? 2LL : 1LL) * num_cus && tiles <= 0x7fffffffLL && (double)mi * ni >= 0.9 * (double)c.M * c.N) {
-            cls = k;
-            Mi = mi;
-            Ni = ni;
-        }
-    }
-    if (cls < 0) return launch_typed<float>(c);
-    sg::Params p;
-    p.A = reinterpret_cast<const float *>(c.A);
-    p.B = reinterpret_cast<const float *>(c.B);
-    p.C = reinterpret_cast<float *>(c.C);
-    p.lda = c.lda; p.ldb = c.ldb; p.ldc = c.ldc;
-    p.sA = c.sA; p.sB = c.sB; p.sC = c.sC;
-    p.M = Mi; p.N = Ni; p.K = c.K;
-    p.tiles_m = p.tiles_n = 0;
-    p.alpha = (float)c.alpha;
-    p.beta = (float)c.beta;
-    const bool ak = !c.tA, bk = c.tB;
-    if (ak && bk) G9_TRY((launch_sg_layout<true, true>(p, c.count, cls)));
-    else if (ak) G9_TRY((launch_sg_layout<true, false>(p, c.count, cls)));
-    else if (bk) G9_TRY((launch_sg_layout<false, true>(p, c.count, cls)));
-    else G9_TRY((launch_sg_layout<false, false>(p, c.count, cls)));
-    if (Ni < c.N) G9_TRY(launch_typed<float>(sub_call(c, 0, Mi, Ni, c.N - Ni)));   // right strip
-    if (Mi < c.M) {   // bottom strip, full width
-        const int r = c.M - Mi, Ms = (r + 63) / 64 * 64;
-        // shifted 64×64 whole tiles when the width is whole 64-column tiles and the shift keeps A 16-byte aligned
-        if (Ni == c.N && c.N % 64 == 0 && Ms <= c.M && (!c.tA || (c.M - Ms) % 4 == 0)) {
-            const GemmCall sc = sub_call(c, c.M - Ms, Ms, 0, c.N);
-            sg::Params ps = p;
-            ps.A = reinterpret_cast<const float *>(sc.A);
-            ps.C = reinterpret_cast<float *>(sc.C);
-            ps.M = Ms;
-            ps.N = c.N;
-            ps.m_skip = Ms - r;
-            ps.tiles_m = Ms / 64;
-            ps.tiles_n = c.N / 64;
-            const dim3 grid((unsigned)(ps.tiles_m * ps.tiles_n), (unsigned)c.count), block(256);
-            if (ak && bk) hipLaunchKernelGGL((sg::sgemm_kernel<64, 64, 2, 2, 4, true, true, 8, 0, 0, true>), grid, block, 0, stream, ps);
-            else if (ak) hipLaunchKernelGGL((sg::sgemm_kernel<64, 64, 2, 2, 4, true, false, 8, 0, 0, true>), grid, block, 0, stream, ps);
-            else if (bk) hipLaunchKernelGGL((sg::sgemm_kernel<64, 64, 2, 2, 4, false, true, 8, 0, 0, true>), grid, block, 0, stream, ps);
-            else hipLaunchKernelGGL((sg::sgemm_kernel<64, 64, 2, 2, 4, false, false, 8, 0, 0, true>), grid, block, 0, stream, ps);
-            G9_HIP(hipGetLastError());
-        } else {
-            G9_TRY(launch_typed<float>(sub_call(c, Mi, r, 0, c.N)));
-        }
-    }
-    return 0;
-}
+}  // namespace g9
+#include "sgemm_launch.h"
+namespace g9 {
 
 template <class T>
 static int launch_typed(const GemmCall &c) {
@@ -520,7 +329,10 @@ int launch_gemm(const GemmCall &c) {
         int rc = 0;
         return launch_hgemm_tiles(c, &rc) ? rc : launch_typed<f16>(c);
     }
-    case GEN9BLAS_S: return launch_sgemm(c);
+    case GEN9BLAS_S: {
+        int rc = 0;
+        return launch_sgemm_direct(c, &rc) ? rc : launch_typed<float>(c);
+    }
     case GEN9BLAS_D: return launch_typed<double>(c);
     }
     G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "type %d unavailable", c.type);

@@ -68,3 +68,38 @@ def test_gemm_ragged_batch_and_tiny_strides(g9, torch_dev, kind):
         check(g9, torch_dev, kind, 70, 90, 75, ta, tb, 1, 1, 0.0, count=5, seed=5)
         for M, N in [(200, 1), (2, 300), (3, 5)]:
             check(g9, torch_dev, kind, M, N, 150, ta, tb, 0, 0, 0.0, count=3, seed=M + N)
+
+
+# few tiles and a long k: K split into slices whose sums a second kernel adds (K = 3841: with 12 or 16 slices of FP16, 24
+# of FP32, the last slice is one k; K = 4160: whole k-steps, the last slice one of them with 8 slices of 9)
+@pytest.mark.parametrize("kind", ["H", "S", "D"])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 3841), (100, 60, 3841), (48, 300, 4160), (130, 129, 3009), (20, 700, 2050)])
+def test_gemm_slices_of_k(g9, torch_dev, kind, M, N, K):
+    for ta, tb in [(0, 0), (1, 0), (0, 1), (1, 1)]:
+        for pad, off, beta in [(0, 0, 0.0), (1, 1, -1.0), (2, 2, 0.5)]:
+            check(g9, torch_dev, kind, M, N, K, ta, tb, pad, off, beta, seed=M + K)
+
+
+@pytest.mark.parametrize("kind", ["H", "S", "D"])
+@pytest.mark.parametrize("N,K", [(70, 3841), (129, 2000), (64, 65), (333, 700), (1, 50), (3, 130)])
+def test_syrk_ragged_and_long(g9, torch_dev, kind, N, K):
+    """The triangle of X·Xᵀ and Xᵀ·X on unaligned views: edge tiles, slices of K, the other triangle left alone."""
+    torch, dt = torch_dev, DT[kind]
+    code = {"H": 0, "S": 1, "D": 3}[kind]
+    for trans in (0, 1):
+        for uplo in (0, 1):
+            for pad, off, beta in [(0, 0, 0.0), (1, 1, -1.0)]:
+                rng = np.random.default_rng(N + K + trans)
+                _, x, ldx, _ = _view(torch, rng, dt, (K, N) if trans else (N, K), pad, off)
+                cb, c, ldc, _ = _view(torch, rng, dt, (N, N), pad, off, fill=77.0)
+                xd = x[0].double()
+                full = (torch.mm(xd.t().contiguous(), xd) if trans else torch.mm(xd, xd.t().contiguous())) * 2.0 + beta * c[0].double()
+                mask = torch.ones(N, N, dtype=torch.bool, device="cuda")
+                mask = torch.triu(mask) if uplo else torch.tril(mask)
+                keep = cb.clone()
+                torch.as_strided(keep, (N, N), (ldc, 1), off)[mask] = full[mask].to(keep.dtype)
+                if not beta:
+                    c[0][mask] = float("nan")
+                g9._call("syrk", code, uplo, trans, N, K, 2.0, x.data_ptr(), ldx, beta, c.data_ptr(), ldc)
+                torch.cuda.synchronize()
+                assert torch.equal(cb, keep), f"{kind} N={N} K={K} trans={trans} uplo={uplo} pad={pad} beta={beta}"
