@@ -119,6 +119,8 @@ __device__ __forceinline__ double block_sum(double s) {
 // Two kernels: every block writes its FP64 partial, then reduce_final adds the partials in index order, so the
 // result does not depend on block scheduling. (Finishing in the last block instead needs a device-scope fence per
 // block, which writes back and invalidates the L2 of the XCD: about 35 % of the HBM rate at 1 GiB on gfx950.)
+// A single block's partial is the result itself (square root taken for nrm2) and goes to `part` without the second
+// kernel.
 template <class T, int MODE>
 __global__ void __launch_bounds__(NT) reduce_kernel(int n, const T *x, ll ix, const T *y, ll iy, int vec, double *part) {
     constexpr int V = VW<T>;
@@ -165,7 +167,7 @@ __global__ void __launch_bounds__(NT) reduce_kernel(int n, const T *x, ll ix, co
     for (ll i = tail + (ll)blockIdx.x * NT + threadIdx.x; i < n; i += stride)
         acc(s0, (double)x[i * ix], MODE == 0 ? (double)y[i * iy] : 0.0);
     const double t = block_sum(s0 + s1);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+    if (threadIdx.x == 0) part[blockIdx.x] = MODE == 2 && gridDim.x == 1 ? __builtin_sqrt(t) : t;
 }
 
 // Sum of np ≤ FIN·NT partials (more are handled by the plain loop): all loads are issued before the first add, so
@@ -230,100 +232,160 @@ __global__ void __launch_bounds__(NT) iamax_final(int np, const double *pv, cons
     if (threadIdx.x == 0) *out = b.i == 0x7fffffffffffffffLL ? 0 : b.i;
 }
 
-// ---------------- GEMV no-trans: y = alpha·A·x + beta·y ----------------
-// A wave owns RWN consecutive rows; its lanes stream 16 bytes of each row per step (1 KiB per row per wave-step) and
-// reuse each x chunk for the RWN rows. The RWN sums are reduced across the wave by the transposing butterfly.
+// ---------------- GEMV ----------------
+// Both directions read A once, 16 bytes per lane, at whatever alignment its rows have (an odd row length or a
+// submatrix leaves rows aligned to their elements only; the GPU serves such loads), and are bound by the bytes they
+// keep in flight: every batch of loads, the last partial one included, is issued before its first product.
+template <int ES> struct Unaligned;
+template <> struct Unaligned<2> { typedef u32x4 type __attribute__((aligned(2))); };
+template <> struct Unaligned<4> { typedef u32x4 type __attribute__((aligned(4))); };
+template <> struct Unaligned<8> { typedef u32x4 type __attribute__((aligned(8))); };
+// NTL: nontemporal, for an A too large to be found in the last-level cache by the next product with it.
+template <bool NTL, class T> __device__ __forceinline__ Vec<T> vload_a(const T *p) {
+    Vec<T> v;
+    const auto *q = reinterpret_cast<const typename Unaligned<(int)sizeof(T)>::type *>(p);
+    if constexpr (NTL) v.u = __builtin_nontemporal_load(q);
+    else v.u = *q;
+    return v;
+}
+// Elements j .. j + V - 1 of x; XC: contiguous.
+template <class T, bool XC> __device__ __forceinline__ Vec<T> vload_x(const T *x, ll j, ll ix) {
+    Vec<T> v;
+    if constexpr (XC) {
+        v.u = *reinterpret_cast<const typename Unaligned<(int)sizeof(T)>::type *>(x + j);
+    } else {
+#pragma unroll
+        for (int e = 0; e < VW<T>; e++) v.e[e] = x[(j + e) * ix];
+    }
+    return v;
+}
+
+// No-trans, y = alpha·A·x + beta·y: RWN rows per group of KS waves, whose lanes stream 16 bytes of each row per step
+// (1 KiB per row and wave, steps dealt to the waves in turn) and reuse each chunk of x for the RWN rows. The RWN sums
+// are reduced across the wave by the transposing butterfly, the KS waves' sums added in LDS in wave order. Two steps
+// per batch: 4 take 101 registers and halve the waves of a SIMD (40000×200 FP32 7.8 µs against 5.6), 1 leaves too few
+// bytes in flight on long rows (1000×8192 7.5 against 5.8).
+// MI355X, µs per call, FP32 unless said, before (element-wise loads for rows not 16-byte aligned, a block of 16 rows
+// throughout) -> now: 6000×1501 10.3 -> 5.8, 6000×1500 6.5 -> 5.8, 1000×8192 13.5 -> 5.3, 300×40000 75 -> 12,
+// 16384×16383 188 -> 168, FP16 8191×4097 23.2 -> 11.3.
 constexpr int RWN = 4;
-template <class T, bool VEC>
+template <class T, bool XC, bool NTL, int KS>
 __global__ void __launch_bounds__(NT) gemv_n_kernel(int M, int N, typename Comp<T>::R alpha, const T *A, ll lda, const T *x,
                                                     ll ix, typename Comp<T>::R beta, T *y, ll iy) {
+    static_assert(KS == 1 || KS == NT / 64, "rows of a wave, or of a block");
     using R = typename Comp<T>::R;
-    constexpr int V = VW<T>;
-    const int lane = threadIdx.x & 63;
-    const int r0 = (blockIdx.x * (NT / 64) + (threadIdx.x >> 6)) * RWN;
-    if (r0 >= M) return;
+    constexpr int V = VW<T>, U = 2, SW = KS * 64 * V;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = (KS == 1 ? (int)blockIdx.x * (NT / 64) + w : (int)blockIdx.x) * RWN, kw = KS == 1 ? 0 : w;
+    if (KS == 1 && r0 >= M) return;
     const T *ar[RWN];
 #pragma unroll
     for (int r = 0; r < RWN; r++) ar[r] = A + (ll)min(r0 + r, M - 1) * lda;
     R s[RWN];
 #pragma unroll
     for (int r = 0; r < RWN; r++) s[r] = 0;
-    int j = lane * V;
-    if (VEC) {
-        const int nvec = N - N % V;
-        // U steps per batch: all U·RWN loads of A (nontemporal: A is read once) are issued before the first product
-        constexpr int U = 4;
-        for (; j + (U - 1) * 64 * V < nvec; j += U * 64 * V) {
-            Vec<T> xv[U], av[U][RWN];
+    const int nvec = N - N % V;
+    // US steps from column j0 of this wave; LAST: columns past nvec count as zeros (both factors, so that an infinity
+    // beside them stays out)
+    auto batch = [&](int j0, auto us, auto last) {
+        constexpr int US = decltype(us)::value;
+        constexpr bool LAST = decltype(last)::value;
+        Vec<T> xv[US], av[US][RWN];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                xv[u] = vload(x + j + u * 64 * V);
+        for (int u = 0; u < US; u++) {
+            const unsigned j = (unsigned)j0 + u * SW + lane * V, jc = LAST ? min(j, (unsigned)(nvec - V)) : j;
+            xv[u] = vload_x<T, XC>(x, jc, ix);
 #pragma unroll
-                for (int r = 0; r < RWN; r++) av[u][r] = vload_nt(ar[r] + j + u * 64 * V);
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int r = 0; r < RWN; r++)
-#pragma unroll
-                    for (int e = 0; e < V; e++) s[r] = fma_r((R)av[u][r].e[e], (R)xv[u].e[e], s[r]);
+            for (int r = 0; r < RWN; r++) av[u][r] = vload_a<NTL>(ar[r] + jc);
         }
-        for (; j < nvec; j += 64 * V) {
-            const Vec<T> xv = vload(x + j);
+        if constexpr (LAST) {
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            if ((unsigned)j0 + (US - 1) * SW + lane * V >= (unsigned)nvec) {   // only the last step can be partial
+                xv[US - 1].u = z;
 #pragma unroll
-            for (int r = 0; r < RWN; r++) {
-                const Vec<T> av = vload_nt(ar[r] + j);
-#pragma unroll
-                for (int e = 0; e < V; e++) s[r] = fma_r((R)av.e[e], (R)xv.e[e], s[r]);
+                for (int r = 0; r < RWN; r++) av[US - 1][r].u = z;
             }
         }
-        for (int jt = nvec + lane; jt < N; jt += 64)
 #pragma unroll
-            for (int r = 0; r < RWN; r++) s[r] = fma_r((R)ar[r][jt], (R)x[jt], s[r]);
-    } else {
-        for (int jt = lane; jt < N; jt += 64) {
-            const R xj = (R)x[(ll)jt * ix];
+        for (int u = 0; u < US; u++)
 #pragma unroll
-            for (int r = 0; r < RWN; r++) s[r] = fma_r((R)ar[r][jt], xj, s[r]);
-        }
+            for (int r = 0; r < RWN; r++)
+#pragma unroll
+                for (int e = 0; e < V; e++) s[r] = fma_r((R)av[u][r].e[e], (R)xv[u].e[e], s[r]);
+    };
+    using No = std::false_type;
+    using Yes = std::true_type;
+    int j0 = kw * 64 * V;
+    for (; nvec - j0 >= U * SW; j0 += U * SW) batch(j0, std::integral_constant<int, U>(), No());
+    // the columns past the last whole 16 bytes, one per lane of the first wave, loaded ahead of the last batch
+    const bool tail = kw == 0 && nvec < N;
+    R at[RWN], xt = 0;
+    if (tail) {
+        const int jt = min(nvec + lane, N - 1);
+        xt = (R)x[(ll)jt * ix];
+#pragma unroll
+        for (int r = 0; r < RWN; r++) at[r] = (R)ar[r][jt];
     }
+    const int left = j0 < nvec ? (nvec - j0 + SW - 1) / SW : 0;   // steps of this wave still to do, 0 .. U
+    if (left == 2) batch(j0, std::integral_constant<int, 2>(), Yes());
+    else if (left == 1) batch(j0, std::integral_constant<int, 1>(), Yes());
+    if (tail && nvec + lane < N)
+#pragma unroll
+        for (int r = 0; r < RWN; r++) s[r] = fma_r(at[r], xt, s[r]);
     // butterfly over the RWN row sums: two halving exchanges, then plain sums
     int base = 0;
     butterfly<0, RWN>(s, lane, base);
-    if ((lane & (64 / RWN - 1)) == 0) {
-        const int row = r0 + base;
-        if (row < M) {
-            T *yp = y + (ll)row * iy;
-            *yp = (T)(beta == R(0) ? alpha * s[0] : fma_r(alpha, s[0], beta * (R)*yp));
+    R sum = s[0];
+    int row = r0 + base;
+    bool writer = (lane & (64 / RWN - 1)) == 0;
+    if constexpr (KS > 1) {
+        __shared__ R red[KS][RWN];
+        if (writer) red[w][base] = sum;
+        __syncthreads();
+        writer = threadIdx.x < RWN;
+        if (writer) {
+            row = r0 + (int)threadIdx.x;
+            sum = red[0][threadIdx.x];
+#pragma unroll
+            for (int q = 1; q < KS; q++) sum += red[q][threadIdx.x];
         }
+    }
+    if (writer && row < M) {
+        T *yp = y + (ll)row * iy;
+        *yp = (T)(beta == R(0) ? alpha * sum : fma_r(alpha, sum, beta * (R)*yp));
     }
 }
 
-// ---------------- GEMV trans: y = alpha·Aᵀ·x + beta·y ----------------
-// Stage 1: a thread owns V consecutive columns (16 bytes) and a band of rpp rows, partial sums to P[part][col].
-// Stage 2: y[col] = alpha·Σ_part P[part][col] + beta·y[col] in a fixed order. With one part stage 1 writes y.
-template <class T, bool VEC>
+// Trans, y = alpha·Aᵀ·x + beta·y. Stage 1: a block owns 64·V columns (16 bytes per lane) and a band of rpp rows, a
+// quarter of it per wave; the waves' sums are added in LDS in wave order and go to P[part][col]. Stage 2: y[col] =
+// alpha·Σ_part P[part][col] + beta·y[col] in a fixed order. With one part stage 1 writes y. The last lane's columns
+// that would pass the row's end start V before it; the ones another lane owns are summed and not written. The sum over
+// a block's waves quarters the partials that stage 2 reads.
+// MI355X, µs per call with stage 2, FP32 unless said, before (element-wise loads for rows not 16-byte aligned, 1024
+// columns and one partial per block row band) -> now: 6000×1501 23.9 -> 10.2, 6000×1500 15.2 -> 10.0, 40000×333 49.8 ->
+// 15.6, 16384×16383 446 -> 179, FP16 8191×4097 47.7 -> 16; 16384×8192 84.6 -> 82.5.
+template <class T, bool NTL>
 __global__ void __launch_bounds__(NT) gemv_t1_kernel(int M, int N, int rpp, const T *A, ll lda, const T *x, ll ix,
                                                      typename Comp<T>::R *P, int direct, typename Comp<T>::R alpha,
                                                      typename Comp<T>::R beta, T *y, ll iy) {
     using R = typename Comp<T>::R;
-    constexpr int V = VW<T>;
-    const int c0 = (blockIdx.x * NT + threadIdx.x) * V;
-    if (c0 >= N) return;
-    const int part = blockIdx.y, i0 = part * rpp, i1 = min(M, i0 + rpp);
+    constexpr int V = VW<T>, W = NT / 64, U = 8;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b0 = blockIdx.x * 64 * V, cb = b0 + lane * V, c0 = max(min(cb, N - V), 0);
+    const int part = blockIdx.y, i0 = part * rpp, i1 = min(M, i0 + rpp), rw = (i1 - i0 + W - 1) / W;
+    int i = i0 + w * rw;
+    const int a1 = min(i1, i + rw);
     R s[V];
 #pragma unroll
     for (int e = 0; e < V; e++) s[e] = 0;
-    const bool full = VEC && c0 + V <= N;
-    if (full) {
-        // U rows per step: their loads (nontemporal: A is read once) are all issued before the first product
-        constexpr int U = 8;
-        int i = i0;
-        for (; i + U <= i1; i += U) {
+    if (N >= V) {
+        const T *Ac = A + c0;
+        // U rows per step, their loads all issued before the first product
+        for (; i + U <= a1; i += U) {
             Vec<T> av[U];
             R xv[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) av[u] = vload_nt(A + (ll)(i + u) * lda + c0);
+            for (int u = 0; u < U; u++) av[u] = vload_a<NTL>(Ac + (ll)(i + u) * lda);
 #pragma unroll
             for (int u = 0; u < U; u++) xv[u] = (R)x[(ll)(i + u) * ix];
 #pragma unroll
@@ -331,50 +393,59 @@ __global__ void __launch_bounds__(NT) gemv_t1_kernel(int M, int N, int rpp, cons
 #pragma unroll
                 for (int e = 0; e < V; e++) s[e] = fma_r((R)av[u].e[e], xv[u], s[e]);
         }
-        for (; i < i1; i++) {
-            const R xv = (R)x[(ll)i * ix];
-            const Vec<T> av = vload_nt(A + (ll)i * lda + c0);
+        if (i < a1) {   // the last rows, fewer than U
+            Vec<T> av[U - 1];
+            R xv[U - 1];
 #pragma unroll
-            for (int e = 0; e < V; e++) s[e] = fma_r((R)av.e[e], xv, s[e]);
+            for (int u = 0; u < U - 1; u++) av[u] = vload_a<NTL>(Ac + (ll)min(i + u, a1 - 1) * lda);
+#pragma unroll
+            for (int u = 0; u < U - 1; u++) xv[u] = (R)x[(ll)min(i + u, a1 - 1) * ix];
+#pragma unroll
+            for (int u = 0; u < U - 1; u++)
+                if (i + u < a1)
+#pragma unroll
+                    for (int e = 0; e < V; e++) s[e] = fma_r((R)av[u].e[e], xv[u], s[e]);
         }
     } else {
-        for (int i = i0; i < i1; i++) {
+        for (; i < a1; i++) {
             const R xv = (R)x[(ll)i * ix];
 #pragma unroll
-            for (int e = 0; e < V; e++)
-                if (c0 + e < N) s[e] = fma_r((R)A[(ll)i * lda + c0 + e], xv, s[e]);
+            for (int e = 0; e < V; e++) s[e] = fma_r((R)A[(ll)i * lda + min(e, N - 1)], xv, s[e]);
         }
     }
+    __shared__ R red[W][64 * V];
 #pragma unroll
-    for (int e = 0; e < V; e++) {
-        if (c0 + e >= N) break;
+    for (int e = 0; e < V; e++)
+        if (c0 + e >= cb) red[w][c0 + e - b0] = s[e];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 64 * V && b0 + t < N; t += NT) {
+        R sum = red[0][t];
+#pragma unroll
+        for (int q = 1; q < W; q++) sum += red[q][t];
         if (direct) {
-            T *yp = y + (ll)(c0 + e) * iy;
-            *yp = (T)(beta == R(0) ? alpha * s[e] : fma_r(alpha, s[e], beta * (R)*yp));
+            T *yp = y + (ll)(b0 + t) * iy;
+            *yp = (T)(beta == R(0) ? alpha * sum : fma_r(alpha, sum, beta * (R)*yp));
         } else {
-            P[(ll)part * N + c0 + e] = s[e];
+            P[(ll)part * N + b0 + t] = sum;
         }
     }
 }
-template <class T>
-__global__ void __launch_bounds__(NT) gemv_t2_kernel(int N, int parts, const typename Comp<T>::R *P,
+// 64 columns per block; the block's G waves each sum every G-th part (loads issued 8 at a time, added in part order),
+// then wave 0 adds the G sums in wave order: a fixed summation order for every column.
+template <class T, int G>
+__global__ void __launch_bounds__(G * 64) gemv_t2_kernel(int N, int parts, const typename Comp<T>::R *P,
                                                      typename Comp<T>::R alpha, typename Comp<T>::R beta, T *y, ll iy) {
-    // 64 columns per block; the block's 4 waves each sum every 4th part (loads issued 8 at a time, added in part
-    // order), then wave 0 adds the 4 sums in wave order: a fixed summation order for every column.
     using R = typename Comp<T>::R;
-    constexpr int G = NT / 64;
-    const int j = blockIdx.x * 64 + (threadIdx.x & 63), gq = threadIdx.x >> 6;
+    const int j = blockIdx.x * 64 + (threadIdx.x & 63), jc = min(j, N - 1);
+    const int gq = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     R t = 0;
-    if (j < N) {
-        int r = gq;
-        for (; r + 7 * G < parts; r += 8 * G) {
-            R v[8];
+    for (int r = gq; r < parts; r += 8 * G) {
+        R v[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = P[(ll)(r + u * G) * N + j];
+        for (int u = 0; u < 8; u++) v[u] = P[(ll)min(r + u * G, parts - 1) * N + jc];
 #pragma unroll
-            for (int u = 0; u < 8; u++) t += v[u];
-        }
-        for (; r < parts; r += G) t += P[(ll)r * N + j];
+        for (int u = 0; u < 8; u++)
+            if (r + u * G < parts) t += v[u];
     }
     __shared__ R red[G][64];
     red[gq][threadIdx.x & 63] = t;
@@ -441,21 +512,30 @@ int launch_rot(int es, int n, void *x, ll ox, ll ix, void *y, ll oy, ll iy, doub
     return elem<3>(es, n, h11, h12, h21, h22, x, ox, ix, y, oy, iy);
 }
 
+// Reductions of up to one step of one block (1024 chunks) run as that block alone: the second kernel's launch costs more
+// than the other CUs save (nrm2 of 1501 FP32 values, with the wait for the result: 14.8 -> 11.8 µs).
+constexpr ll REDUCE_ONE = 4 * NT;
 int launch_reduce(int es, int mode, int n, const void *x, ll ox, ll ix, const void *y, ll oy, ll iy, double *result) {
     return by_type(es, [&](auto *tag) -> int {
         using T = std::remove_pointer_t<decltype(tag)>;
         const T *xp = (const T *)x + ox, *yp = y ? (const T *)y + oy : xp;
         const bool vec = ix == 1 && (mode != 0 || iy == 1) && al16(xp) && (mode != 0 || al16(yp));
-        const unsigned g = stream_grid(vec ? (n + VW<T> - 1) / VW<T> : n, mode == 0 ? 4 : 8);
-        void *pp;
-        G9_TRY(scratch(SLOT_P, g * sizeof(double), &pp));
-        double *part = (double *)pp;
+        const ll chunks = vec ? (n + VW<T> - 1) / VW<T> : n;
+        const unsigned g = chunks <= REDUCE_ONE ? 1u : stream_grid(chunks, mode == 0 ? 4 : 8);
+        double *part = result;
+        if (g > 1) {
+            void *pp;
+            G9_TRY(scratch(SLOT_P, g * sizeof(double), &pp));
+            part = (double *)pp;
+        }
         if (mode == 0) hipLaunchKernelGGL((reduce_kernel<T, 0>), dim3(g), dim3(NT), 0, stream, n, xp, ix, yp, iy, (int)vec, part);
         else if (mode == 1) hipLaunchKernelGGL((reduce_kernel<T, 1>), dim3(g), dim3(NT), 0, stream, n, xp, ix, yp, iy, (int)vec, part);
         else hipLaunchKernelGGL((reduce_kernel<T, 2>), dim3(g), dim3(NT), 0, stream, n, xp, ix, yp, iy, (int)vec, part);
         G9_HIP(hipGetLastError());
-        hipLaunchKernelGGL(reduce_final, dim3(1), dim3(NT), 0, stream, (int)g, (const double *)part, mode, result);
-        G9_HIP(hipGetLastError());
+        if (g > 1) {
+            hipLaunchKernelGGL(reduce_final, dim3(1), dim3(NT), 0, stream, (int)g, (const double *)part, mode, result);
+            G9_HIP(hipGetLastError());
+        }
         return 0;
     });
 }
@@ -478,6 +558,7 @@ int launch_iamax(int es, int n, const void *x, ll ox, ll ix, long long *result) 
     });
 }
 
+constexpr int GEMV_T_PER_CU = 3;
 int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll lda, const void *x, ll ox, ll ix,
                 double beta, void *y, ll oy, ll iy) {
     return by_type(es, [&](auto *tag) -> int {
@@ -485,26 +566,40 @@ int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll
         using R = typename Comp<T>::R;
         const T *Ap = (const T *)A, *xp = (const T *)x + ox;
         T *yp = (T *)y + oy;
-        const bool avec = al16(Ap) && (lda * (ll)sizeof(T)) % 16 == 0;
+        // A of more than half the 256 MiB last-level cache is read past it (nontemporal); a smaller one, which a
+        // solver's next product with it finds there, is not. FP32, µs, nontemporal against plain loads: 16384² 162
+        // against 174, 16384×8192 100 against 106; 6000×1501 6.2 against 5.8, FP16 1501×11008 6.4 against 5.3.
+        const bool ntl = (double)M * (double)N * sizeof(T) > (double)(128 << 20);
         if (!trans) {
-            const bool vec = avec && ix == 1 && al16(xp);
+            // The four waves of a block share its rows where rows alone would leave CUs with few waves (fewer than 4
+            // blocks per CU), unless a row is so short that they would have nothing to share.
             const unsigned g = (unsigned)((M + RWN * (NT / 64) - 1) / (RWN * (NT / 64)));
-            if (vec) hipLaunchKernelGGL((gemv_n_kernel<T, true>), dim3(g), dim3(NT), 0, stream, M, N, (R)alpha, Ap, lda, xp, ix, (R)beta, yp, iy);
-            else hipLaunchKernelGGL((gemv_n_kernel<T, false>), dim3(g), dim3(NT), 0, stream, M, N, (R)alpha, Ap, lda, xp, ix, (R)beta, yp, iy);
+            const bool share = g < 4u * (unsigned)num_cus && N > 2 * 64 * VW<T>;
+            const auto go = [&](auto xc, auto ks) {
+                constexpr int KS = decltype(ks)::value;
+                constexpr bool XC = decltype(xc)::value;
+                const auto kern = ntl ? gemv_n_kernel<T, XC, true, KS> : gemv_n_kernel<T, XC, false, KS>;
+                hipLaunchKernelGGL(kern, dim3(KS == 1 ? g : (unsigned)((M + RWN - 1) / RWN)),
+                                   dim3(NT), 0, stream, M, N, (R)alpha, Ap, lda, xp, ix, (R)beta, yp, iy);
+            };
+            using One = std::integral_constant<int, 1>;
+            using All = std::integral_constant<int, NT / 64>;
+            if (ix == 1) share ? go(std::true_type(), All()) : go(std::true_type(), One());
+            else share ? go(std::false_type(), All()) : go(std::false_type(), One());
             G9_HIP(hipGetLastError());
             return 0;
         }
-        constexpr int V = VW<T>;
-        const int cblocks = (N + NT * V - 1) / (NT * V);
-        // about 3 blocks per CU, each summing a band of rows into FP32 (FP64) partials: the best HBM rate in a sweep of
-        // 256-8192 blocks at 16384² (fewer, longer bands keep more loads in flight per thread)
-        const int tgt = 3 * (num_cus > 0 ? num_cus : 256);
+        constexpr int V = VW<T>, W = NT / 64;
+        const int cblocks = (N + 64 * V - 1) / (64 * V);
+        // about GEMV_T_PER_CU blocks per CU, each summing a band of rows into FP32 (FP64) partials; whole batches of 8
+        // rows per wave
+        const int tgt = GEMV_T_PER_CU * (num_cus > 0 ? num_cus : 256);
         int parts = (tgt + cblocks - 1) / cblocks;
-        const int maxparts = (M + 15) / 16;
+        const int maxparts = (M + 8 * W - 1) / (8 * W);
         if (parts > maxparts) parts = maxparts;
         if (parts < 1) parts = 1;
-        const int rpp = (M + parts - 1) / parts;
-        parts = (M + rpp - 1) / rpp;
+        const int rpp = (int)(((ll)M + (ll)parts * 8 * W - 1) / ((ll)parts * 8 * W)) * 8 * W;
+        parts = (int)(((ll)M + rpp - 1) / rpp);
         R *P = nullptr;
         if (parts > 1) {
             void *pp;
@@ -512,12 +607,12 @@ int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll
             P = (R *)pp;
         }
         const dim3 grid((unsigned)cblocks, (unsigned)parts);
-        if (avec) hipLaunchKernelGGL((gemv_t1_kernel<T, true>), grid, dim3(NT), 0, stream, M, N, rpp, Ap, lda, xp, ix, P, (int)(parts == 1), (R)alpha, (R)beta, yp, iy);
-        else hipLaunchKernelGGL((gemv_t1_kernel<T, false>), grid, dim3(NT), 0, stream, M, N, rpp, Ap, lda, xp, ix, P, (int)(parts == 1), (R)alpha, (R)beta, yp, iy);
+        hipLaunchKernelGGL((ntl ? gemv_t1_kernel<T, true> : gemv_t1_kernel<T, false>), grid, dim3(NT), 0, stream, M, N, rpp, Ap, lda, xp, ix, P, (int)(parts == 1), (R)alpha, (R)beta, yp, iy);
         G9_HIP(hipGetLastError());
         if (parts > 1) {
-            hipLaunchKernelGGL((gemv_t2_kernel<T>), dim3((unsigned)((N + 63) / 64)), dim3(NT), 0, stream, N, parts,
-                               (const R *)P, (R)alpha, (R)beta, yp, iy);
+            const dim3 g2((unsigned)((N + 63) / 64));
+            if (parts > 32) hipLaunchKernelGGL((gemv_t2_kernel<T, 16>), g2, dim3(1024), 0, stream, N, parts, (const R *)P, (R)alpha, (R)beta, yp, iy);
+            else hipLaunchKernelGGL((gemv_t2_kernel<T, 4>), g2, dim3(256), 0, stream, N, parts, (const R *)P, (R)alpha, (R)beta, yp, iy);
             G9_HIP(hipGetLastError());
         }
         return 0;

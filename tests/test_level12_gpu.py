@@ -118,6 +118,34 @@ def test_gemv_submatrix(g9, orc, dt):
     assert_close("gemv submatrix", g9.gemv(B[10:200, 5:305], B[0, :300]), ref, scale, TOL[dt])
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float16, np.float64])
+@pytest.mark.parametrize("M,N", [(1, 2), (5, 3), (9, 17), (33, 255), (31, 513), (65, 1021), (40, 2049), (700, 4099), (4100, 130),
+                                 (17000, 67)])
+def test_gemv_unaligned_rows(g9, torch_dev, dt, M, N):
+    """Rows aligned to their elements only (a submatrix at column 1 of an odd-width device matrix), at the edges of the
+    16-byte columns, of a wave's steps and of a block's row band: every output against float64, with x contiguous and
+    strided, y accumulated, and the columns and rows around the view and an infinite row kept out of other sums."""
+    torch = torch_dev
+    W = torch.from_numpy(rng.uniform(-1, 1, (M + 2, N + 2 + (N + 1) % 2)).astype(dt)).cuda()
+    W[0], W[-1], W[:, 0], W[:, N + 1:] = (float("nan"),) * 4
+    A = W[1:M + 1, 1:N + 1]
+    Ad = A.cpu().numpy().astype(np.float64)
+    for trans in (False, True):
+        Op = Ad.T if trans else Ad
+        x2 = torch.from_numpy(rng.uniform(-1, 1, 2 * Op.shape[1]).astype(dt)).cuda()
+        for x in (x2[:Op.shape[1]], x2[::2]):
+            y = torch.from_numpy(rng.uniform(-1, 1, Op.shape[0]).astype(dt)).cuda()
+            xd, y0 = x.cpu().numpy().astype(np.float64), y.cpu().numpy().astype(np.float64)
+            got = g9.gemv(A, x, alpha=1.5, beta=-0.5, y=y, trans=trans)
+            scale = 1.5 * (abs(Op) @ abs(xd)) + 0.5 * abs(y0)
+            assert_close(f"gemv trans={trans} {M}x{N}", got.cpu().numpy(), 1.5 * (Op @ xd) - 0.5 * y0, scale, TOL[dt])
+    A[M - 1, N - 1] = float("inf")
+    one = torch.ones(max(M, N), dtype=A.dtype, device="cuda")
+    for trans, n in ((False, M), (True, N)):
+        r = g9.gemv(A, one[:M if trans else N], trans=trans).cpu().numpy()
+        assert np.isposinf(r[n - 1]) and np.isfinite(r[:n - 1]).all(), f"infinity, trans={trans} {M}x{N}"
+
+
 def test_level2_config_device(g9, orc, torch_dev):
     """The benchmarked level 1/2 configuration at full size on device buffers: SAXPY, SDOT (2^26), SGEMV N/T (16384²)."""
     torch = torch_dev
