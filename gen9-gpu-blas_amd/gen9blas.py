@@ -473,6 +473,14 @@ def _square(A, t, uplo):
 def _private_copy(B, t):
     """A new C-contiguous copy of B that a routine may overwrite: on B's device, or in pinned host memory."""
     if _is_tensor(B) and B.is_cuda:
+        n = B.numel()
+        if (B.dtype == _torch_dtype(t) and B.is_contiguous() and 0 < n < 1 << 31 and B.data_ptr() % 16 == 0
+                and not (B.requires_grad or B.is_neg()) and type(B) is _torch_module().Tensor):
+            # Queued on the library's stream like the call that follows. A copy on torch's default stream makes each
+            # stream wait for the other: FP64 trsm of 2000 x 500, 557 us a call queued that way, 378 this way.
+            X = _torch_module().empty_like(B)
+            _call("copy", _TYPE_CODE[t], n, B.data_ptr(), 1, X.data_ptr(), 1)
+            return X
         return B.to(dtype=_torch_dtype(t), copy=True).contiguous()
     b = empty(np.shape(B), t)
     b[...] = B
