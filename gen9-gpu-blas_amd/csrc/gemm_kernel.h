@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     static_assert(TM * MI == WTM && TN * MI == WTN, "wave tile must be a multiple of the MFMA tile");
     static_assert(TRI == 0 || (BM == BN && !SPLIT), "triangle mode: square tiles, no split");
     static_assert(KLIM == 0 || (!SPLIT && TRI == 0), "k-limited tiles: one product, no split");
-    static_assert(KG == 1 || (!SPLIT && TRI == 0 && KLIM == 0), "k groups: plain tiles only");
+    static_assert(KG == 1 || (!SPLIT && TRI == 0), "k groups: no split, no triangle");
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * KG][(BM + BN) * ROWB];
 
     // KG > 1: the workgroup holds KG groups of WM × WN waves; group kh takes the block tiles kh, kh + KG, ... of the

@@ -102,10 +102,28 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     return 0;
 }
 
+// FP64 products of few tiles: 32×32 tiles, four k groups of one wave each (73 KiB of LDS, two workgroups per CU). A
+// wave of a 64×128 or 64×64 tile does 4 to 8 times the MFMAs one after the other while most CUs idle; four k groups hide
+// each other's barrier and load waits, and no second pass adds slices of K.
+// MI355X, µs, the tiles below (two k groups or split K) -> 32×32 (8 groups): 128³ × 7 13.5 -> 5.9 (6.5), 256³ × 3 22.6 ->
+// 7.3 (8.0), 512³ 20.4 -> 10.7 (11.1), 976×500×1024 40.1 -> 26.5 (32.5), 128×4096×128 8.8 -> 7.5, 137×1500×700 23.8 -> 14.6.
+// Beyond two workgroups per CU it loses (700×900×300 16.1 against 20.3, 1024³ 44 against 48), and so it does to split K
+// where that applies (fewer than CUs / 2 tiles of 64×64) with many k-steps: 500×500×5000 57 against 67, 200×200×4000 44
+// against 54; the lines of both cross between K = 1600 and 3500.
+static long long tiles32(int M, int N, int count) { return (long long)((M + 31) / 32) * ((N + 31) / 32) * count; }
+constexpr TileCfg TILE32{32, 32, 1, 1};
+constexpr int TILE32_SPLIT_K = 1536;
+
 template <class T, bool AK, bool BKC>
 static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     using CF = Cfg<T, AK, BKC>;
     if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 1, true>(p, count);
+    if constexpr (sizeof(T) == 8) {
+        const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
+        if (splitk_forced() < 0 && tiles32(p.M, p.N, count) <= 2LL * num_cus &&
+            (count > 1 || t64 * 2 >= num_cus || p.K <= TILE32_SPLIT_K))
+            return launch_t<T, TILE32, AK, BKC, 4>(p, count);
+    }
     const long long big_tiles = (long long)((p.M + CF::big.BM - 1) / CF::big.BM) * ((p.N + CF::big.BN - 1) / CF::big.BN) * count;
     if (big_tiles * CF::small_div < num_cus) {
         // 64×64 tiles with two k groups of 4 waves (8 waves per workgroup, the groups' sums added through LDS), when
@@ -255,15 +273,15 @@ int launch_gemm_tri(const GemmCall &c, bool lower) {
 // range is cut to where the triangle is non-zero (klim as gemm_kernel's KLIM), one launch over every tile of C,
 // longest ranges dispatched first; the small tiles when the big ones are fewer than the CUs. Layout NN only (both
 // operands as stored), one product.
-template <class T, TileCfg C, int KLIM, bool CHECKED = false>
+template <class T, TileCfg C, int KLIM, bool CHECKED = false, int KG = 1>
 static int launch_klim_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     p.tiles_m = (p.M + C.BM - 1) / C.BM;
     p.tiles_n = (p.N + C.BN - 1) / C.BN;
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles)", p.tiles_m, p.tiles_n);
-    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM, 1, CHECKED>;
-    p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(C.WM * C.WN * 64));
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(C.WM * C.WN * 64), 0, stream, p);
+    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM, KG, CHECKED>;
+    p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(C.WM * C.WN * 64 * KG));
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(C.WM * C.WN * 64 * KG), 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
 }
@@ -290,12 +308,18 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     };
     constexpr bool half = sizeof(T) == 2, dbl = sizeof(T) == 8;
     const long long want = half ? num_cus : 2LL * num_cus;
+    // FP64 below that: 32×32 tiles with four k groups up to two workgroups per CU, then 32×64 with two. MI355X, µs,
+    // 64×64 -> these: 1024×500 43.9 -> 20.0, 512×500 22.0 -> 11.2, 1024×16 39.4 -> 15.6; 1024×1000 44.2 -> 26.9 (32×32:
+    // 32.3); 1024×2048 45.4 against 48.0, 512×4096 27.6 against 29.3.
+    constexpr TileCfg half_wide{32, 64, 1, 2};
     const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
     const auto go = [&](auto kc) -> int {
         constexpr int K = decltype(kc)::value;
         if (!unchecked_ok<T>(true, p.lda) || !unchecked_ok<T>(false, p.ldb)) return launch_klim_t<T, tiny, K, true>(p, c.count);
         if (cls == 0) return launch_klim_t<T, CF::big, K>(p, c.count);
         if constexpr (dbl) {
+            if (ntiles(TILE32) <= 2LL * num_cus) return launch_klim_t<T, TILE32, K, false, 4>(p, c.count);
+            if (ntiles(half_wide) <= 2LL * num_cus) return launch_klim_t<T, half_wide, K, false, 2>(p, c.count);
             if (cls == 2) return launch_klim_t<T, tiny, K>(p, c.count);
         }
         return launch_klim_t<T, CF::small, K>(p, c.count);

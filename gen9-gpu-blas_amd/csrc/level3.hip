@@ -137,8 +137,10 @@ __global__ void __launch_bounds__(256) trsm_store_kernel(const T *Y, T *B, ll ld
 constexpr int TRSM_NB = 128;
 // rows of a leaf (an inverted diagonal block applied by one product) of the FP32 and the FP64 solve: one more
 // composition level and half the leaves for FP64 (n = 4096 left lower, MI355X: 1.427 -> 1.412 ms with 1024 rows
-// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured)
-constexpr int TRSM_LEAF_S = 512, TRSM_LEAF_D = 1024;
+// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured). FP64 solves of up to TRSM_LEAF_D_FROM rows take
+// 512 too, as one or two leaves do not repay the level (2000×500 219 -> 209 µs, 1024×2048 142 -> 127, 3000×130 270 ->
+// 261; 4096×500 346 against 378)
+constexpr int TRSM_LEAF_S = 512, TRSM_LEAF_D = 1024, TRSM_LEAF_D_FROM = 3072;
 // Inverse of the diagonal block bi of L (rows and columns r0 .. r0+b-1, b ≤ TRSM_NB, in the leaf p = r0 / lb of lb
 // rows whose element (i, j) is at L[p·bstride + i·ld + j]; the block's entries above the diagonal are read as zeros,
 // and its diagonal as ones when unit),
@@ -553,9 +555,9 @@ int gen9blas_trsm(int type, int side, int uplo, int transA, int diag, int M, int
     // L·Y = alpha·R: op'(A) = left ? op(A) : op(A)ᵀ; lower when the triangle of A, transposed or not, is lower
     const int tr = left ? transA != 0 : transA == 0;
     const int lower = (uplo == GEN9BLAS_LOWER) != (tr != 0), rev = !lower;
-    // Leaves of TRSM_LEAF_S / _D rows for FP32 / FP64: each leaf inverse is composed from the 128-row FP64 inverses (below);
+    // Leaves of TRSM_LEAF_S / _D rows for FP32 / large FP64: each leaf inverse is composed from the 128-row FP64 inverses (below);
     // FP16 keeps 128-row leaves (the composition would round once more in FP16)
-    const int nbl = (n + TRSM_NB - 1) / TRSM_NB, lb = es == 8 ? TRSM_LEAF_D : es == 4 ? TRSM_LEAF_S : TRSM_NB, nleaf = (n + lb - 1) / lb;
+    const int nbl = (n + TRSM_NB - 1) / TRSM_NB, lb = es == 8 && n > TRSM_LEAF_D_FROM ? TRSM_LEAF_D : es >= 4 ? TRSM_LEAF_S : TRSM_NB, nleaf = (n + lb - 1) / lb;
     // A left solve with A lower and not transposed reads both operands where they lie: every product below reads L
     // strictly below its diagonal blocks, the block inversion masks the rest of A itself, B is the right-hand side
     // updated in place (alpha applied by the first product that touches each block of rows), and only the solution

@@ -103,3 +103,13 @@ def test_syrk_ragged_and_long(g9, torch_dev, kind, N, K):
                 g9._call("syrk", code, uplo, trans, N, K, 2.0, x.data_ptr(), ldx, beta, c.data_ptr(), ldc)
                 torch.cuda.synchronize()
                 assert torch.equal(cb, keep), f"{kind} N={N} K={K} trans={trans} uplo={uplo} pad={pad} beta={beta}"
+
+
+@pytest.mark.parametrize("M,N,K,count", [(1, 1, 1, 1), (31, 33, 15, 1), (32, 32, 64, 1), (33, 65, 1536, 1), (33, 65, 1537, 1),
+                                         (500, 513, 200, 1), (520, 520, 70, 1), (65, 31, 129, 20)])
+def test_dgemm_few_tiles(g9, torch_dev, M, N, K, count):
+    """FP64 products of few tiles (32x32, four k groups of 16 k): edges of tiles, groups without a k-step, both sides of the
+    lines in tiles and K that choose them."""
+    for ta, tb in [(0, 0), (1, 0), (0, 1), (1, 1)]:
+        for pad, off, beta in [(0, 0, 0.0), (1, 1, -1.0)]:
+            check(g9, torch_dev, "D", M, N, K, ta, tb, pad, off, beta, count=count, seed=M + K)
