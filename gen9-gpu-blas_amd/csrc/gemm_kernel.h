@@ -218,7 +218,8 @@ template <class T> inline bool unchecked_ok(bool kc, long long ld) {
 constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_WRITE = 0x200;
 
 // TRI (1: lower, 2: upper): C is square and only its lower (upper) triangle is written, alpha·sum + beta·C as
-// elsewhere; the grid holds only the tiles that meet the triangle (square tiles, one product, no split).
+// elsewhere; the grid holds only the tiles that meet the triangle (square tiles, one product). With kper, blockIdx.y is
+// a slice of kper k, its strides those of A, B and the planes of C, which tri_split_sum adds.
 // KLIM: the k range of a tile is cut to where a triangular operand is non-zero (one product, no split):
 //   1: op(A) lower, k < m0 + BM; 2: op(A) upper, k ≥ m0; 3: op(B) lower, k ≥ n0; 4: op(B) upper, k < n0 + BN.
 //   Tiles are dispatched longest range first, spread over the XCDs.
@@ -318,6 +319,8 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         A += z * p.sA;
         B += z * p.sB;
         C += z * p.sC;
+        if constexpr (TRI != 0)
+            if (p.kper) K = min(p.kper, K - (int)z * p.kper);   // slice z of K, into a plane of its own
     }
 
     using SA = Stage<T, BM, NT, AK, (BM < 256)>;
@@ -593,6 +596,31 @@ __global__ void __launch_bounds__(256) splitk_reduce(const S *__restrict__ P, T 
             *c = (T)r;
         }
     }
+}
+
+// Finish of a triangle product in slices: C = alpha·(P[0] + ... + P[slices-1]) + beta·C on the triangle, row blockIdx.y,
+// P[s] an N×N plane; slices added in order (8 loads in flight), rounded once.
+template <class T, class S>
+__global__ void __launch_bounds__(256) tri_split_sum(const S *__restrict__ P, T *C, long long ldc, int N, int slices, int lower,
+                                                     S alpha, S beta) {
+    const int m = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x;
+    if (n >= N || (lower ? n > m : n < m)) return;
+    const long long plane = (long long)N * N;
+    const S *q = P + (long long)m * N + n;
+    S v = 0;
+    int s = 0;
+    for (; s + 8 <= slices; s += 8) {
+        S t[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) t[u] = q[(s + u) * plane];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v += t[u];
+    }
+    for (; s < slices; s++) v += q[s * plane];
+    T *c = C + (long long)m * ldc + n;
+    S r = alpha * v;
+    if (beta != S(0)) r = fma_s(beta, (S)*c, r);
+    *c = (T)r;
 }
 
 }  // namespace g9

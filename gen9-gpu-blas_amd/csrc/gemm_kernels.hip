@@ -219,6 +219,11 @@ static int launch_typed(const GemmCall &c) {
 // element, each C element rounded once; the two layouts those routines use: A and B both k-contiguous, or both
 // mn-contiguous. FP32 and FP64 take 64×64 tiles: at n = 4096 their 2080 tiles keep every CU busy to the end (FP32
 // SYRK 0.71 ms, FP64 1.21), where 128×128 tiles (528) left a nearly empty last round (1.02, 1.58).
+// FP64 triangles of few tiles and a long K: slices of K, as many as keep four workgroups per CU busy, of at least
+// TRI_SLICE_K. A Gram matrix of 1000 features is 136 tiles, half the CUs with one workgroup each.
+// MI355X, µs, N×K, unsliced -> sliced: 1000×20000 1474 -> 399, 128×40000 1662 -> 37, 333×7001 421 -> 40, 600×700 52 -> 22,
+// 1400×15000 1145 -> 511, 2000×9000 1145 -> 816; the shortest it takes, 64×512, 21.6 -> 15.4.
+constexpr int TRI_SLICE_K = 256, TRI_SLICES = 64;
 template <class T, int TRI, bool AK, bool BKC, bool CHECKED = false>
 static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
     constexpr TileCfg C = sizeof(T) == 2 && !CHECKED ? TileCfg{128, 128, 2, 2} : TileCfg{64, 64, 2, 2};
@@ -228,6 +233,31 @@ static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
     p.tiles_m = p.tiles_n = (p.M + C.BM - 1) / C.BM;
     const long long tiles = (long long)p.tiles_m * (p.tiles_m + 1) / 2;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product too large (%d tiles per side)", p.tiles_m);
+    if constexpr (sizeof(T) == 8 && !CHECKED) {
+        constexpr int BK = 128 / (int)sizeof(T);
+        int ns = (int)std::min<long long>({4LL * num_cus / tiles, p.K / TRI_SLICE_K, TRI_SLICES});
+        if (ns > 1 && splitk_forced() < 0) {
+            auto q = p;
+            q.kper = ((p.K + ns - 1) / ns + BK - 1) / BK * BK;
+            ns = (p.K + q.kper - 1) / q.kper;
+            void *P;
+            G9_TRY(scratch(SLOT_P, (size_t)ns * p.M * p.M * sizeof(T), &P));
+            q.C = P;
+            q.ldc = p.M;
+            q.sA = q.kper * (AK ? 1 : p.lda);
+            q.sB = q.kper * (BKC ? 1 : p.ldb);
+            q.sC = (long long)p.M * p.M;
+            q.alpha = 1;
+            q.beta = 0;
+            hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI>), dim3((unsigned)tiles, (unsigned)ns),
+                               dim3(C.WM * C.WN * 64), 0, stream, q);
+            G9_HIP(hipGetLastError());
+            hipLaunchKernelGGL((tri_split_sum<T, T>), dim3((unsigned)((p.M + 255) / 256), (unsigned)p.M), dim3(256), 0, stream,
+                               (const T *)P, (T *)p.C, p.ldc, p.M, ns, TRI == 1, p.alpha, p.beta);
+            G9_HIP(hipGetLastError());
+            return 0;
+        }
+    }
     hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI, 0, 1, CHECKED>), dim3((unsigned)tiles),
                        dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
