@@ -102,7 +102,9 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     return 0;
 }
 
-// FP64 products of few tiles: 32×32 tiles, four k groups of one wave each (73 KiB of LDS, two workgroups per CU). A
+// FP64 products of few tiles: 32×32 tiles, four k groups of one wave each (73 KiB of LDS, two workgroups per CU), or eight
+// for single products of at most a tile per CU, which split K up to 8 ways before: as many partial sums keep the error
+// where it was (500×500×512 against 80-bit sums: split K 2.8e-16, four groups 3.8e-16). A
 // wave of a 64×128 or 64×64 tile does 4 to 8 times the MFMAs one after the other while most CUs idle; four k groups hide
 // each other's barrier and load waits, and no second pass adds slices of K.
 // MI355X, µs, the tiles below (two k groups or split K) -> 32×32 (8 groups): 128³ × 7 13.5 -> 5.9 (6.5), 256³ × 3 22.6 ->
@@ -120,9 +122,10 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 1, true>(p, count);
     if constexpr (sizeof(T) == 8) {
         const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
-        if (splitk_forced() < 0 && tiles32(p.M, p.N, count) <= 2LL * num_cus &&
-            (count > 1 || t64 * 2 >= num_cus || p.K <= TILE32_SPLIT_K))
-            return launch_t<T, TILE32, AK, BKC, 4>(p, count);
+        const long long t32 = tiles32(p.M, p.N, count);
+        if (splitk_forced() < 0 && t32 <= 2LL * num_cus && (count > 1 || t64 * 2 >= num_cus || p.K <= TILE32_SPLIT_K))
+            return count == 1 && t32 <= num_cus ? launch_t<T, TILE32, AK, BKC, 8>(p, count)
+                                                : launch_t<T, TILE32, AK, BKC, 4>(p, count);
     }
     const long long big_tiles = (long long)((p.M + CF::big.BM - 1) / CF::big.BM) * ((p.N + CF::big.BN - 1) / CF::big.BN) * count;
     if (big_tiles * CF::small_div < num_cus) {
