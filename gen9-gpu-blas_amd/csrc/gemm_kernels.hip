@@ -138,7 +138,8 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
         // 54.0 / 45.1, four of one 64×64 wave 41.9 / 34.9, two of 1×2 waves 48.7, four of 2×1 waves 51.1.
         // A batch (count > 1) cannot split K, so it takes these tiles from num_cus / 4 of them: FP64 128³ × 16 (the
         // triangular solve's 256-row compositions) 12.7 → 8.2 µs on 64 workgroups of 8 waves instead of 32 of 64×128,
-        // DTRSM n = 4096 1.458 → 1.443 ms.
+        // DTRSM n = 4096 1.458 → 1.443 ms. (The FP64 figures of at most two 32×32 tiles per CU date from before those tiles,
+        // which take such products now.)
         if constexpr (sizeof(T) >= 4) {
             const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
             const long long need = count > 1 ? (num_cus + 3) / 4 : (num_cus + 1) / 2;
