@@ -117,8 +117,8 @@ template <> __device__ __forceinline__ void transpose<double>(const u32x4 *in, u
 // KC: the operand is stored k-contiguous (element (mn, k) at X[mn·ld + k]); otherwise mn-contiguous
 // (element (mn, k) at X[k·ld + mn]) and transposed in registers on the way to LDS.
 constexpr int ROWB = 144;   // LDS bytes per tile row: 128 of data + 16 of padding
-// SHIFT: as load16 (the 256-row tiles have no registers left for it).
-template <class T, int RT, int NT, bool KC, bool SHIFT>
+// SHIFT: as load16 (the 256-row tiles have no registers left for it). WIDE: 64-bit offsets (see init).
+template <class T, int RT, int NT, bool KC, bool SHIFT, bool WIDE>
 struct Stage {
     static constexpr int V = 16 / (int)sizeof(T);
     // k-contiguous: N16 chunks per thread. Transposed: NB V×V blocks per thread; when the tile has fewer blocks than
@@ -135,10 +135,12 @@ struct Stage {
     // step: bytes per k-step of BK·KG. Rows (starts of chunks) past the matrix's end are moved back onto the last one,
     // whose values no stored element uses; a chunk that straddles the end of an mn-contiguous row reads on into the
     // next row, so a k-step loaded this way must not hold the last k unless the tile lies inside the matrix, and ld
-    // must be at least V - 1. The offsets are 32-bit, which bounds the row stride (unchecked_ok).
+    // must be at least V - 1 (unchecked_ok). The offsets are 32-bit, one register each, where the tile's rows span less
+    // than 4 GiB (narrow_ok), and 64-bit beyond that.
     static constexpr int NOFF = KC ? N16 : NB;
+    using Off = std::conditional_t<WIDE, unsigned long long, unsigned>;
     const char *org;
-    unsigned off[NOFF];
+    Off off[NOFF];
     long long step;
     __device__ __forceinline__ void init(const T *__restrict__ X, long long ld, int MN, int mn0, int k0, int kstep, int tid) {
         org = reinterpret_cast<const char *>(KC ? X + (long long)mn0 * ld + k0 : X + (long long)k0 * ld + mn0);
@@ -147,10 +149,10 @@ struct Stage {
         for (int i = 0; i < NOFF; i++) {
             const int id = i * NT + tid;
             if constexpr (KC) {
-                off[i] = (unsigned)(min(id >> 3, MN - 1 - mn0) * (int)(ld * sizeof(T)) + (id & 7) * 16);
+                off[i] = (Off)min(id >> 3, MN - 1 - mn0) * (Off)(ld * sizeof(T)) + (id & 7) * 16;
             } else {
                 const int lo = id & 31, mb = (lo & 3) + 4 * (id >> 5), kb = lo >> 2;
-                off[i] = (unsigned)(kb * V * (int)(ld * sizeof(T)) + min(mb * V, (MN - 1 - mn0) / V * V) * (int)sizeof(T));
+                off[i] = (Off)(kb * V) * (Off)(ld * sizeof(T)) + min(mb * V, (MN - 1 - mn0) / V * V) * (int)sizeof(T);
             }
         }
     }
@@ -208,10 +210,18 @@ __device__ __forceinline__ float fma_s(float a, float b, float c) { return __bui
 __device__ __forceinline__ double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
 template <class T, class S> __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid);
 
+// How a kernel loads its operands: UNCHECKED with 32-bit offsets inside a tile, the same with 64-bit offsets (WIDE), or
+// CHECKED, every k-step by the checked loads.
+enum Loads { UNCHECKED, WIDE, CHECKED };
 // Whether the unchecked loads take an operand of this row stride: at least one element short of 16 bytes where chunks run
-// along mn, and offsets inside a tile (at most 256 rows) below 2^31 bytes.
-template <class T> inline bool unchecked_ok(bool kc, long long ld) {
-    return (kc || ld >= 16 / (int)sizeof(T) - 1) && ld * 256 * (long long)sizeof(T) < (1LL << 31);
+// along mn.
+template <class T> inline bool unchecked_ok(bool kc, long long ld) { return kc || ld >= 16 / (int)sizeof(T) - 1; }
+// Whether 32-bit offsets reach every row that a tile of RT rows or columns spans, of MN in the matrix: min(RT, MN) of its
+// rows where they run along k, else the first rows of eight V×V blocks of k (the others are a uniform offset away).
+template <class T> inline bool narrow_ok(bool kc, long long ld, int RT, int MN) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const long long rows = kc ? (RT < MN ? RT : MN) - 1 : 7 * V;
+    return rows * ld * (long long)sizeof(T) + (kc ? 128 : RT * (long long)sizeof(T)) <= (1LL << 32);
 }
 
 // Instruction-group masks of __builtin_amdgcn_sched_group_barrier.
@@ -223,9 +233,8 @@ constexpr int SG_MFMA = 0x008, SG_VMEM_READ = 0x020, SG_DS_READ = 0x100, SG_DS_W
 // KLIM: the k range of a tile is cut to where a triangular operand is non-zero (one product, no split):
 //   1: op(A) lower, k < m0 + BM; 2: op(A) upper, k ≥ m0; 3: op(B) lower, k ≥ n0; 4: op(B) upper, k < n0 + BN.
 //   Tiles are dispatched longest range first, spread over the XCDs.
-// CHECKED: every k-step takes the checked loads (row strides that the unchecked ones do not take).
 template <class T, int BM, int BN, int WM, int WN, bool AK, bool BKC, bool SPLIT = false, int TRI = 0, int KLIM = 0,
-          int KG = 1, bool CHECKED = false>
+          int KG = 1, Loads LOADS = UNCHECKED>
 __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typename Mma<T>::Sum> p) {
     using MM = Mma<T>;
     using S = typename MM::Sum;
@@ -323,8 +332,9 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
             if (p.kper) K = min(p.kper, K - (int)z * p.kper);   // slice z of K, into a plane of its own
     }
 
-    using SA = Stage<T, BM, NT, AK, (BM < 256)>;
-    using SB = Stage<T, BN, NT, BKC, (BM < 256)>;
+    constexpr bool SHIFT = BM < 256;
+    using SA = Stage<T, BM, NT, AK, SHIFT, LOADS == WIDE>;
+    using SB = Stage<T, BN, NT, BKC, SHIFT, LOADS == WIDE>;
     SA sa;
     SB sb;
     constexpr int TI = MM::SWAP ? TN : TM, TJ = MM::SWAP ? TM : TN;   // acc[i][j]: D tile of (first, second) operand
@@ -398,7 +408,7 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         sa.store(buf(b), tid);
         sb.store(buf(b) + BM * ROWB, tid);
     };
-    if constexpr (!CHECKED) {
+    if constexpr (LOADS != CHECKED) {
         sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
         sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
         if (m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {

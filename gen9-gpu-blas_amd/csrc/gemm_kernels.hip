@@ -65,26 +65,35 @@ static int splitk_slices(long long tiles, int K, int BK, int count) {
     return s;
 }
 
-template <class T, TileCfg C, bool AK, bool BKC, int KG = 1, bool CHECKED = false>
+// Tiles for operands that the unchecked loads do not take, or not with 32-bit offsets.
+constexpr TileCfg TILE64{64, 64, 2, 2};
+// Operands whose rows under a tile of the chosen size span 4 GiB or more take 64×64 tiles with 64-bit offsets.
+template <class T, TileCfg C, bool AK, bool BKC> static bool narrow(const GemmParams<typename Mma<T>::Sum> &p) {
+    return narrow_ok<T>(AK, p.lda, C.BM, p.M) && narrow_ok<T>(BKC, p.ldb, C.BN, p.N);
+}
+
+template <class T, TileCfg C, bool AK, bool BKC, int KG = 1, Loads LOADS = UNCHECKED>
 static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
     using S = typename Mma<T>::Sum;
+    if constexpr (LOADS == UNCHECKED)
+        if (!narrow<T, C, AK, BKC>(p)) return launch_t<T, TILE64, AK, BKC, 1, WIDE>(p, count);
     constexpr int BK = 128 / (int)sizeof(T);
     p.tiles_m = (p.M + C.BM - 1) / C.BM;
     p.tiles_n = (p.N + C.BN - 1) / C.BN;
     if ((long long)p.tiles_m * p.tiles_n > 0x7fffffffLL || count > 65535)
         G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles, batch %d)", p.tiles_m, p.tiles_n, count);
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
-    const int split = KG > 1 || CHECKED ? 1 : splitk_slices(tiles, p.K, BK, count);
+    const int split = KG > 1 ? 1 : splitk_slices(tiles, p.K, BK, count);
     const dim3 block(C.WM * C.WN * 64 * KG);
-    if constexpr (!CHECKED) if (split > 1) {
+    if (split > 1) {
         static_assert((size_t)C.BM * C.BN * sizeof(S) <= SPLITK_TILE_BYTES_MAX, "split tile beyond the work-space bound");
         p.kper = ((p.K + split - 1) / split + BK - 1) / BK * BK;
         const int ns = (p.K + p.kper - 1) / p.kper;
         void *P;
         G9_TRY(scratch(SLOT_P, (size_t)ns * p.M * p.N * sizeof(S), &P));
         p.P = reinterpret_cast<S *>(P);
-        hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, true>), dim3((unsigned)tiles, (unsigned)ns),
-                           block, 0, stream, p);
+        hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, true, 0, 0, 1, LOADS>),
+                           dim3((unsigned)tiles, (unsigned)ns), block, 0, stream, p);
         G9_HIP(hipGetLastError());
         const long long mn = (long long)p.M * p.N;
         const bool v4 = p.N % 4 == 0;
@@ -97,7 +106,7 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
         return 0;
     }
     const dim3 grid((unsigned)tiles, (unsigned)count);
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, 0, 0, KG, CHECKED>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, 0, 0, KG, LOADS>), grid, block, 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
 }
@@ -119,7 +128,8 @@ constexpr int TILE32_SPLIT_K = 1536;
 template <class T, bool AK, bool BKC>
 static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     using CF = Cfg<T, AK, BKC>;
-    if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 1, true>(p, count);
+    if constexpr (sizeof(T) < 8 && !(AK && BKC))
+        if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_t<T, TILE64, AK, BKC, 1, CHECKED>(p, count);
     if constexpr (sizeof(T) == 8) {
         const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
         const long long t32 = tiles32(p.M, p.N, count);
@@ -144,7 +154,7 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
             const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
             const long long need = count > 1 ? (num_cus + 3) / 4 : (num_cus + 1) / 2;
             if (splitk_forced() < 0 && t64 >= need && (sizeof(T) == 8 || t64 <= num_cus))
-                return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 2>(p, count);
+                return launch_t<T, TILE64, AK, BKC, 2>(p, count);
         }
         return launch_t<T, CF::small, AK, BKC>(p, count);
     }
@@ -163,7 +173,7 @@ static int launch_layout(const GemmParams<typename Mma<T>::Sum> &p, int count) {
     if constexpr (sizeof(T) == 4) {
         const long long t64 = (long long)((p.M + 63) / 64) * ((p.N + 63) / 64) * count;
         if (splitk_forced() < 0 && t64 * 2 >= num_cus && t64 <= num_cus)
-            return launch_t<T, TileCfg{64, 64, 2, 2}, AK, BKC, 2>(p, count);
+            return launch_t<T, TILE64, AK, BKC, 2>(p, count);
     }
     // FP32: 128×128 tiles with two k groups of 2×2 waves (64×64 per wave, 147 KiB of LDS: one workgroup per CU) when
     // their count fills whole rounds of num_cus workgroups (the last round at least 95 % full). Measured (TFLOP/s,
@@ -228,16 +238,18 @@ static int launch_typed(const GemmCall &c) {
 // MI355X, µs, N×K, unsliced -> sliced: 1000×20000 1474 -> 399, 128×40000 1662 -> 37, 333×7001 421 -> 40, 600×700 52 -> 22,
 // 1400×15000 1145 -> 511, 2000×9000 1145 -> 816; the shortest it takes, 64×512, 21.6 -> 15.4.
 constexpr int TRI_SLICE_K = 256, TRI_SLICES = 64;
-template <class T, int TRI, bool AK, bool BKC, bool CHECKED = false>
+template <class T, int TRI, bool AK, bool BKC, Loads LOADS = UNCHECKED>
 static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
-    constexpr TileCfg C = sizeof(T) == 2 && !CHECKED ? TileCfg{128, 128, 2, 2} : TileCfg{64, 64, 2, 2};
-    if constexpr (!CHECKED) {
-        if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_tri_t<T, TRI, AK, BKC, true>(p);
+    constexpr TileCfg C = sizeof(T) == 2 && LOADS == UNCHECKED ? TileCfg{128, 128, 2, 2} : TILE64;
+    if constexpr (LOADS == UNCHECKED) {
+        if constexpr (sizeof(T) < 8 && !(AK && BKC))
+            if (!unchecked_ok<T>(AK, p.lda) || !unchecked_ok<T>(BKC, p.ldb)) return launch_tri_t<T, TRI, AK, BKC, CHECKED>(p);
+        if (!narrow<T, C, AK, BKC>(p)) return launch_tri_t<T, TRI, AK, BKC, WIDE>(p);
     }
     p.tiles_m = p.tiles_n = (p.M + C.BM - 1) / C.BM;
     const long long tiles = (long long)p.tiles_m * (p.tiles_m + 1) / 2;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product too large (%d tiles per side)", p.tiles_m);
-    if constexpr (sizeof(T) == 8 && !CHECKED) {
+    if constexpr (sizeof(T) == 8) {
         constexpr int BK = 128 / (int)sizeof(T);
         int ns = (int)std::min<long long>({4LL * num_cus / tiles, p.K / TRI_SLICE_K, TRI_SLICES});
         if (ns > 1 && splitk_forced() < 0) {
@@ -253,8 +265,8 @@ static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
             q.sC = (long long)p.M * p.M;
             q.alpha = 1;
             q.beta = 0;
-            hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI>), dim3((unsigned)tiles, (unsigned)ns),
-                               dim3(C.WM * C.WN * 64), 0, stream, q);
+            hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI, 0, 1, LOADS>),
+                               dim3((unsigned)tiles, (unsigned)ns), dim3(C.WM * C.WN * 64), 0, stream, q);
             G9_HIP(hipGetLastError());
             hipLaunchKernelGGL((tri_split_sum<T, T>), dim3((unsigned)((p.M + 255) / 256), (unsigned)p.M), dim3(256), 0, stream,
                                (const T *)P, (T *)p.C, p.ldc, p.M, ns, TRI == 1, p.alpha, p.beta);
@@ -262,7 +274,7 @@ static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
             return 0;
         }
     }
-    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI, 0, 1, CHECKED>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, AK, BKC, false, TRI, 0, 1, LOADS>), dim3((unsigned)tiles),
                        dim3(C.WM * C.WN * 64), 0, stream, p);
     G9_HIP(hipGetLastError());
     return 0;
@@ -307,13 +319,15 @@ int launch_gemm_tri(const GemmCall &c, bool lower) {
 // range is cut to where the triangle is non-zero (klim as gemm_kernel's KLIM), one launch over every tile of C,
 // longest ranges dispatched first; the small tiles when the big ones are fewer than the CUs. Layout NN only (both
 // operands as stored), one product.
-template <class T, TileCfg C, int KLIM, bool CHECKED = false, int KG = 1>
+template <class T, TileCfg C, int KLIM, int KG = 1, Loads LOADS = UNCHECKED>
 static int launch_klim_t(GemmParams<typename Mma<T>::Sum> p, int count) {
+    if constexpr (LOADS == UNCHECKED)
+        if (!narrow<T, C, true, false>(p)) return launch_klim_t<T, TILE64, KLIM, 1, WIDE>(p, count);
     p.tiles_m = (p.M + C.BM - 1) / C.BM;
     p.tiles_n = (p.N + C.BN - 1) / C.BN;
     const long long tiles = (long long)p.tiles_m * p.tiles_n;
     if (tiles > 0x7fffffffLL) G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "gemm grid too large (%d × %d tiles)", p.tiles_m, p.tiles_n);
-    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM, KG, CHECKED>;
+    constexpr auto kern = gemm_kernel<T, C.BM, C.BN, C.WM, C.WN, true, false, false, 0, KLIM, KG, LOADS>;
     p.kpair = count == 1 && klim_pair(tiles, wgs_per_cu<kern>(C.WM * C.WN * 64 * KG));
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)count), dim3(C.WM * C.WN * 64 * KG), 0, stream, p);
     G9_HIP(hipGetLastError());
@@ -336,7 +350,6 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     // tile class: FP16 the big tiles when they are at least the CUs; FP32 / FP64 the first of big, small and (FP64)
     // 64×64 that makes two workgroups per CU or more, so that long and short k ranges can share the CUs
     using CF = Cfg<T, true, false>;
-    constexpr TileCfg tiny{64, 64, 2, 2};
     const auto ntiles = [&](TileCfg t) {
         return (long long)((c.M + t.BM - 1) / t.BM) * ((c.N + t.BN - 1) / t.BN) * c.count;
     };
@@ -349,12 +362,13 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
     const auto go = [&](auto kc) -> int {
         constexpr int K = decltype(kc)::value;
-        if (!unchecked_ok<T>(true, p.lda) || !unchecked_ok<T>(false, p.ldb)) return launch_klim_t<T, tiny, K, true>(p, c.count);
+        if constexpr (!dbl)
+            if (!unchecked_ok<T>(false, p.ldb)) return launch_klim_t<T, TILE64, K, 1, CHECKED>(p, c.count);
         if (cls == 0) return launch_klim_t<T, CF::big, K>(p, c.count);
         if constexpr (dbl) {
-            if (ntiles(TILE32) <= 2LL * num_cus) return launch_klim_t<T, TILE32, K, false, 4>(p, c.count);
-            if (ntiles(half_wide) <= 2LL * num_cus) return launch_klim_t<T, half_wide, K, false, 2>(p, c.count);
-            if (cls == 2) return launch_klim_t<T, tiny, K>(p, c.count);
+            if (ntiles(TILE32) <= 2LL * num_cus) return launch_klim_t<T, TILE32, K, 4>(p, c.count);
+            if (ntiles(half_wide) <= 2LL * num_cus) return launch_klim_t<T, half_wide, K, 2>(p, c.count);
+            if (cls == 2) return launch_klim_t<T, TILE64, K>(p, c.count);
         }
         return launch_klim_t<T, CF::small, K>(p, c.count);
     };

@@ -24,6 +24,11 @@
 #include <cmath>
 
 namespace g9 {
+
+// Bytes that the direct copies' lane offsets reach over inside a tile of at most 256 rows: the rows of a k-contiguous
+// operand of MN rows, the k rows of a k-step otherwise (ldb: row stride in bytes). They are 32-bit.
+static long long lane_span(bool kc, long long ldb, int MN, int kb) { return (kc ? std::min(256, MN) : kb) * ldb; }
+
 namespace hgl {
 
 constexpr int KB = 64;   // k per k-step
@@ -132,7 +137,7 @@ static int launch_layout(const hg::Params &p, int count, Choice ch, bool whole) 
 // *rc is the launch's status.
 // The kernel takes operands at 4-byte alignment with even row (and batch) strides, which its direct copies need, and
 // more than one k-step of k (exactly one when no operand row ends inside a 16-byte chunk): the k-step it takes through
-// registers needs a direct one beside it. Lane offsets inside a tile of 256 rows are 32-bit. GEN9BLAS_HGEMM=generic
+// registers needs a direct one beside it. Lane offsets inside a tile are 32-bit (lane_span). GEN9BLAS_HGEMM=generic
 // forces the general kernel; a forced split-K (GEN9BLAS_SPLITK) leaves it the products that are whole 128×128 tiles.
 static bool launch_hgemm_tiles(const GemmCall &c, int *rc) {
     using namespace hgl;
@@ -144,7 +149,7 @@ static bool launch_hgemm_tiles(const GemmCall &c, int *rc) {
     if (generic || c.count > 65535 || c.lda % 2 || c.ldb % 2 || (uintptr_t)c.A % 4 || (uintptr_t)c.B % 4 ||
         (batch && (c.sA % 2 || c.sB % 2)) || std::min(c.lda, c.ldb) < 8)
         return false;
-    if (c.lda * 2 * 256 >= (1LL << 32) || c.ldb * 2 * 256 >= (1LL << 32)) return false;
+    if (lane_span(!c.tA, c.lda * 2, c.M, KB) >= (1LL << 32) || lane_span(c.tB, c.ldb * 2, c.N, KB) >= (1LL << 32)) return false;
     if (c.K < KB || (c.K == KB && ((c.tA && c.M % 8) || (!c.tB && c.N % 8)))) return false;
     // whole: nothing to check or mask, 16-byte stores
     const auto al16 = [&](const void *x, long long ld, long long s) {

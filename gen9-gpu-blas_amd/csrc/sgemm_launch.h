@@ -130,7 +130,7 @@ static sg::Params sg_params(const GemmCall &c) {
     p.beta = (float)c.beta;
     return p;
 }
-// The kernel takes operands at element alignment, lane offsets inside a tile of 256 rows being 32-bit, and more than one
+// The kernel takes operands at element alignment, lane offsets inside a tile being 32-bit (lane_span), and more than one
 // k-step of k (exactly one when no operand row ends inside a 16-byte chunk): the k-step it takes through registers needs a
 // direct one beside it. GEN9BLAS_SGEMM=generic and a forced split-K (GEN9BLAS_SPLITK) ask for the general kernel.
 static bool sgemm_direct_ok(const GemmCall &c) {
@@ -139,7 +139,7 @@ static bool sgemm_direct_ok(const GemmCall &c) {
         return e && !strcmp(e, "generic");
     }();
     if (generic || splitk_forced() >= 0 || c.count > 65535 || std::min(c.lda, c.ldb) < 4) return false;
-    if (c.lda * 4 * 256 >= (1LL << 32) || c.ldb * 4 * 256 >= (1LL << 32)) return false;
+    if (lane_span(!c.tA, c.lda * 4, c.M, sgl::KB) >= (1LL << 32) || lane_span(c.tB, c.ldb * 4, c.N, sgl::KB) >= (1LL << 32)) return false;
     return c.K > sgl::KB || (c.K == sgl::KB && !(c.tA && c.M % 4) && !(!c.tB && c.N % 4));
 }
 // 16-byte aligned operands and row strides, K whole k-steps: what the whole-tile variants take, which check and mask
