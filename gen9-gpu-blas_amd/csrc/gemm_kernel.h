@@ -117,8 +117,8 @@ template <> __device__ __forceinline__ void transpose<double>(const u32x4 *in, u
 // KC: the operand is stored k-contiguous (element (mn, k) at X[mn·ld + k]); otherwise mn-contiguous
 // (element (mn, k) at X[k·ld + mn]) and transposed in registers on the way to LDS.
 constexpr int ROWB = 144;   // LDS bytes per tile row: 128 of data + 16 of padding
-// SHIFT: as load16 (the 256-row tiles have no registers left for it). WIDE: 64-bit offsets (see init).
-template <class T, int RT, int NT, bool KC, bool SHIFT, bool WIDE>
+// WIDE: 64-bit offsets (see init).
+template <class T, int RT, int NT, bool KC, bool WIDE>
 struct Stage {
     static constexpr int V = 16 / (int)sizeof(T);
     // k-contiguous: N16 chunks per thread. Transposed: NB V×V blocks per thread; when the tile has fewer blocks than
@@ -165,23 +165,26 @@ struct Stage {
         }
         org += step;
     }
-    // Checked loads: any tile and k-step, element by element at the edges, zeros outside.
+    // Checked loads: any tile and k-step, zeros outside the matrix.
     __device__ __forceinline__ void load_checked(const T *__restrict__ X, long long ld, int MN, int K, int mn0, int k0, int tid) {
-        if constexpr (KC) {
+        if (PART && tid >= NBLK) return;
+        const int R = KC ? MN : K, Cc = KC ? K : MN;
+        const auto row = [&](int i) {
+            if constexpr (KC) return mn0 + ((i * NT + tid) >> 3);
+            else return k0 + ((((i / V) * NT + tid) & 31) >> 2) * V + i % V;
+        };
+        const auto col = [&](int i) {
+            if constexpr (KC) return k0 + ((i * NT + tid) & 7) * V;
+            else { const int id = (i / V) * NT + tid; return mn0 + ((id & 3) + 4 * (id >> 5)) * V; }
+        };
+        if (Cc >= V) {
 #pragma unroll
-            for (int i = 0; i < N16; i++) {
-                const int id = i * NT + tid;
-                r[i] = load16<T, SHIFT>(X, ld, mn0 + (id >> 3), k0 + (id & 7) * V, MN, K);
-            }
+            for (int i = 0; i < N16; i++) r[i] = load16_raw<T>(X, ld, row(i), col(i), R, Cc);
+#pragma unroll
+            for (int i = 0; i < N16; i++) r[i] = load16_fix<T>(r[i], row(i), col(i), R, Cc);
         } else {
-            if (PART && tid >= NBLK) return;
 #pragma unroll
-            for (int b = 0; b < NB; b++) {
-                const int id = b * NT + tid, lo = id & 31;
-                const int mb = (lo & 3) + 4 * (id >> 5), kb = lo >> 2;
-#pragma unroll
-                for (int i = 0; i < V; i++) r[b * V + i] = load16<T, SHIFT>(X, ld, k0 + kb * V + i, mn0 + mb * V, K, MN);
-            }
+            for (int i = 0; i < N16; i++) r[i] = load16_short<T>(X, ld, row(i), col(i), R, Cc);
         }
     }
     __device__ __forceinline__ void store(unsigned char *rows, int tid) const {
@@ -210,8 +213,8 @@ __device__ __forceinline__ float fma_s(float a, float b, float c) { return __bui
 __device__ __forceinline__ double fma_s(double a, double b, double c) { return __builtin_fma(a, b, c); }
 template <class T, class S> __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int valid);
 
-// How a kernel loads its operands: UNCHECKED with 32-bit offsets inside a tile, the same with 64-bit offsets (WIDE), or
-// CHECKED, every k-step by the checked loads.
+// How a kernel loads its full k-steps: UNCHECKED with 32-bit offsets inside a tile, the same with 64-bit offsets (WIDE), or
+// CHECKED: as WIDE, but mn-contiguous operands by the checked loads.
 enum Loads { UNCHECKED, WIDE, CHECKED };
 // Whether the unchecked loads take an operand of this row stride: at least one element short of 16 bytes where chunks run
 // along mn.
@@ -332,9 +335,8 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
             if (p.kper) K = min(p.kper, K - (int)z * p.kper);   // slice z of K, into a plane of its own
     }
 
-    constexpr bool SHIFT = BM < 256;
-    using SA = Stage<T, BM, NT, AK, SHIFT, LOADS == WIDE>;
-    using SB = Stage<T, BN, NT, BKC, SHIFT, LOADS == WIDE>;
+    using SA = Stage<T, BM, NT, AK, LOADS != UNCHECKED>;
+    using SB = Stage<T, BN, NT, BKC, LOADS != UNCHECKED>;
     SA sa;
     SB sb;
     constexpr int TI = MM::SWAP ? TN : TM, TJ = MM::SWAP ? TM : TN;   // acc[i][j]: D tile of (first, second) operand
@@ -397,9 +399,10 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     // Whole tiles and k-steps load without bounds tests. So do the other shapes, but for their last k-step, which the
     // prologue takes first, with checked loads: the steady-state loop is then one basic block for every shape, whose
     // instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between its
-    // MFMAs. (The checked loop is a variant of its own: beside it, the compiler copies the accumulators in every k-step
-    // of the steady loop.) Before, a ragged tile took the checked loads in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9 µs, 64 × 250³
-    // (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096 140 → 112.
+    // MFMAs. (A second loop beside it makes the compiler copy the accumulators in every k-step of this one.) Before, a
+    // ragged tile took the checked loads in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9
+    // µs, 64 × 250³ (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096
+    // 140 → 112.
     const auto load_checked = [&](int kt) {
         sa.load_checked(A, p.lda, p.M, K, m0, kt * KG * BK + kofs, tid);
         sb.load_checked(B, p.ldb, p.N, K, n0, kt * KG * BK + kofs, tid);
@@ -408,68 +411,58 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
         sa.store(buf(b), tid);
         sb.store(buf(b) + BM * ROWB, tid);
     };
-    if constexpr (LOADS != CHECKED) {
-        sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
-        sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
-        if (m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {
-            sa.load(p.lda);
-            sb.load(p.ldb);
-        } else {
-            load_checked(nk - 1);
-        }
-        store(0);
-        __syncthreads();
-        // what the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes the compiler wait for
-        // every LDS read of a k-step at once (scalar loads and LDS reads share a counter)
-        asm volatile("" : "+s"(C), "+s"(p.P), "+s"(p.ldc), "+s"(p.M), "+s"(p.N));
-        wait_lgkm0();
-        // the accumulators' zeros are hidden from the compiler: as one shared constant they cost FP64 tiles 16-64 register
-        // copies per k-step (the loop's values then rotate through the accumulation registers)
-#pragma unroll
-        for (int i = 0; i < TI; i++)
-#pragma unroll
-            for (int j = 0; j < TJ; j++) asm volatile("" : "+v"(acc[i][j]));
-        for (int kt = 0; kt + 1 < nk; kt++) {
-            const int cur = kt & 1;
-            sa.load(p.lda);
-            sb.load(p.ldb);
-            compute(cur);
-            store(cur ^ 1);
-            constexpr int NRD = TM + TN;                         // LDS fragment reads per group
-            constexpr int NMF = SPG * TI * TJ;                   // MFMAs per group
-            constexpr int NVM = SA::N16 + SB::N16;
-            constexpr int NWR = (AK ? SA::N16 : SA::NB * 8) + (BKC ? SB::N16 : SB::NB * 8);
-            // global loads first, then group 0's fragments; each later group: its MFMAs interleaved with the next
-            // group's reads, and in the last group the LDS writes of the next tile (FP64 n = 4096 NN 70.8 TFLOP/s; over
-            // the last two groups 69.7; without the pinned order 62.8)
-            __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, NVM, 0);
-            __builtin_amdgcn_sched_group_barrier(SG_DS_READ, NRD, 0);
-#pragma unroll
-            for (int q = 0; q < QG; q++) {
-                const int nrd = q + 1 < QG ? NRD : 0;
-                const int nwr = q == QG - 1 ? NWR : 0;
-#pragma unroll
-                for (int t = 0; t < NMF; t++) {
-                    __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                    if (t < nrd) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
-                    else if (t - nrd < nwr) __builtin_amdgcn_sched_group_barrier(SG_DS_WRITE, 1, 0);
-                }
-            }
-            __syncthreads();
-        }
-        compute((nk - 1) & 1);
+    constexpr bool CHECK_A = LOADS == CHECKED && !AK, CHECK_B = LOADS == CHECKED && !BKC;
+    sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
+    sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
+    if (!CHECK_A && !CHECK_B && m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {
+        sa.load(p.lda);
+        sb.load(p.ldb);
     } else {
-        load_checked(0);
-        store(0);
-        __syncthreads();
-        for (int kt = 0; kt < nk; kt++) {
-            const int cur = kt & 1;
-            if (kt + 1 < nk) load_checked(kt + 1);
-            compute(cur);
-            if (kt + 1 < nk) store(cur ^ 1);
-            __syncthreads();
-        }
+        load_checked(nk - 1);
     }
+    store(0);
+    __syncthreads();
+    // what the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes the compiler wait for
+    // every LDS read of a k-step at once (scalar loads and LDS reads share a counter)
+    asm volatile("" : "+s"(C), "+s"(p.P), "+s"(p.ldc), "+s"(p.M), "+s"(p.N));
+    wait_lgkm0();
+    // the accumulators' zeros are hidden from the compiler: as one shared constant they cost FP64 tiles 16-64 register
+    // copies per k-step (the loop's values then rotate through the accumulation registers)
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) asm volatile("" : "+v"(acc[i][j]));
+    for (int kt = 0; kt + 1 < nk; kt++) {
+        const int cur = kt & 1;
+        if constexpr (CHECK_A) sa.load_checked(A, p.lda, p.M, K, m0, kt * KG * BK + kofs, tid);
+        else sa.load(p.lda);
+        if constexpr (CHECK_B) sb.load_checked(B, p.ldb, p.N, K, n0, kt * KG * BK + kofs, tid);
+        else sb.load(p.ldb);
+        compute(cur);
+        store(cur ^ 1);
+        constexpr int NRD = TM + TN;                         // LDS fragment reads per group
+        constexpr int NMF = SPG * TI * TJ;                   // MFMAs per group
+        constexpr int NVM = SA::N16 + SB::N16;
+        constexpr int NWR = (AK ? SA::N16 : SA::NB * 8) + (BKC ? SB::N16 : SB::NB * 8);
+        // global loads first, then group 0's fragments; each later group: its MFMAs interleaved with the next
+        // group's reads, and in the last group the LDS writes of the next tile (FP64 n = 4096 NN 70.8 TFLOP/s; over
+        // the last two groups 69.7; without the pinned order 62.8)
+        __builtin_amdgcn_sched_group_barrier(SG_VMEM_READ, NVM, 0);
+        __builtin_amdgcn_sched_group_barrier(SG_DS_READ, NRD, 0);
+#pragma unroll
+        for (int q = 0; q < QG; q++) {
+            const int nrd = q + 1 < QG ? NRD : 0;
+            const int nwr = q == QG - 1 ? NWR : 0;
+#pragma unroll
+            for (int t = 0; t < NMF; t++) {
+                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                if (t < nrd) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 1, 0);
+                else if (t - nrd < nwr) __builtin_amdgcn_sched_group_barrier(SG_DS_WRITE, 1, 0);
+            }
+        }
+        __syncthreads();
+    }
+    compute((nk - 1) & 1);
 
     if constexpr (KG > 1) {
         // groups 1 .. KG-1 leave their sums in LDS (value-major, so a wave's 64 lanes write 256 consecutive bytes);

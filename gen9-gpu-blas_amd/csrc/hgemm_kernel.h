@@ -154,13 +154,19 @@ struct Loader {
     // stride ld, in elements T), loaded through registers into the tile at `dst`.
     static __device__ __forceinline__ void checked(const T *X, long long ld, int MN, int K, int k0, G9_LDS unsigned char *dst,
                                                    int wave, int lane) {
-        const int c = chunk(wave, lane);
+        const int c = V * chunk(wave, lane), R = KC ? MN : K, Cc = KC ? K : MN, r0 = KC ? 0 : k0, c0 = KC ? k0 + c : c;
+        dma_u32x4 v[NI];
+        if (Cc >= V) {
 #pragma unroll
-        for (int i = 0; i < NI; i++) {
-            const int r = row(i, wave, lane);
-            const dma_u32x4 v = KC ? load16<T>(X, ld, r, k0 + V * c, MN, K) : load16<T>(X, ld, k0 + r, V * c, K, MN);
-            *reinterpret_cast<G9_LDS dma_u32x4 *>(dst + 1024 * (wave + NW * i) + 16 * lane) = v;
+            for (int i = 0; i < NI; i++) v[i] = load16_raw<T>(X, ld, r0 + row(i, wave, lane), c0, R, Cc);
+#pragma unroll
+            for (int i = 0; i < NI; i++) v[i] = load16_fix<T>(v[i], r0 + row(i, wave, lane), c0, R, Cc);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; i++) v[i] = load16_short<T>(X, ld, r0 + row(i, wave, lane), c0, R, Cc);
         }
+#pragma unroll
+        for (int i = 0; i < NI; i++) *reinterpret_cast<G9_LDS dma_u32x4 *>(dst + 1024 * (wave + NW * i) + 16 * lane) = v[i];
     }
 };
 

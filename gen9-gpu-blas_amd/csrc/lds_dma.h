@@ -43,28 +43,31 @@ template <class T> __device__ __forceinline__ dma_u32x4 load16u(const T *p) {
     return __builtin_bit_cast(dma_u32x4, v);
 }
 
-// 16 bytes (V elements) of row r, columns c .. c+V-1 of a row-major matrix X (R valid rows, Cc valid columns, row
-// stride ld); zero outside the valid region. A chunk that crosses the last column is the row's last 16 bytes, shifted:
-// one load as for any other chunk (a load per element there waits for each of them: FP16 1000³, whose K leaves every
-// tile such a k-step, took 9.8 µs against 6.7 for 1024³). SHIFT false: element by element, in fewer registers.
-template <class T, bool SHIFT = true>
-__device__ __forceinline__ dma_u32x4 load16(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
+// 16 bytes (V elements) of row r, columns c .. c+V-1 of a row-major matrix X (R valid rows, Cc valid columns, row stride
+// ld); zero outside the valid region. In two parts where rows hold at least V elements, so that the loads of all of a
+// thread's chunks are on their way before the first is waited for: load16_raw loads the nearest whole chunk inside the
+// matrix, one load wherever (r, c) lies, and load16_fix shifts a chunk that crosses the last column into place and clears
+// what lies outside.
+template <class T> __device__ __forceinline__ dma_u32x4 load16_raw(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
     constexpr int V = 16 / sizeof(T);
-    if (r >= R || c >= Cc) return dma_u32x4{0, 0, 0, 0};
-    const T *row = X + (long long)r * ld;
-    if (SHIFT && Cc >= V) {
-        const int cc = min(c, Cc - V), bytes = (c - cc) * (int)sizeof(T);
-        dma_u32x4 v = load16u(row + cc);
-        if (bytes & 8) v = dma_u32x4{v[2], v[3], 0, 0};
-        if (sizeof(T) < 8 && (bytes & 4)) v = dma_u32x4{v[1], v[2], v[3], 0};
-        if (sizeof(T) < 4 && (bytes & 2))
-            v = dma_u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
-        return v;
-    }
-    if (!SHIFT && c + V <= Cc) return load16u(row + c);
+    return load16u(X + (long long)min(r, R - 1) * ld + min(c, Cc - V));
+}
+template <class T> __device__ __forceinline__ dma_u32x4 load16_fix(dma_u32x4 v, int r, int c, int R, int Cc) {
+    constexpr int V = 16 / sizeof(T);
+    const int bytes = max(c - (Cc - V), 0) * (int)sizeof(T);
+    if (bytes & 8) v = dma_u32x4{v[2], v[3], 0, 0};
+    if (sizeof(T) < 8 && (bytes & 4)) v = dma_u32x4{v[1], v[2], v[3], 0};
+    if (sizeof(T) < 4 && (bytes & 2))
+        v = dma_u32x4{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+    if (r >= R || c >= Cc) v = dma_u32x4{0, 0, 0, 0};
+    return v;
+}
+// The same for rows of fewer than V elements, one by one.
+template <class T> __device__ __forceinline__ dma_u32x4 load16_short(const T *__restrict__ X, long long ld, int r, int c, int R, int Cc) {
+    constexpr int V = 16 / sizeof(T);
     union { dma_u32x4 v; T e[V]; } u;
 #pragma unroll
-    for (int e = 0; e < V; e++) u.e[e] = c + e < Cc ? row[c + e] : T(0);
+    for (int e = 0; e < V; e++) u.e[e] = r < R && c + e < Cc ? X[(long long)r * ld + c + e] : T(0);
     return u.v;
 }
 

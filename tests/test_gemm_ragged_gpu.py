@@ -113,3 +113,21 @@ def test_dgemm_few_tiles(g9, torch_dev, M, N, K, count):
     for ta, tb in [(0, 0), (1, 0), (0, 1), (1, 1)]:
         for pad, off, beta in [(0, 0, 0.0), (1, 1, -1.0)]:
             check(g9, torch_dev, "D", M, N, K, ta, tb, pad, off, beta, count=count, seed=M + K)
+
+
+@pytest.mark.parametrize("kind", ["H", "S", "D"])
+@pytest.mark.parametrize("M,N", [(33, 1), (130, 2), (600, 1), (257, 3), (600, 7), (1025, 2)])
+def test_trmm_narrow(g9, torch_dev, kind, M, N):
+    """Triangular products with rows of B shorter than one 16-byte load (checked loads of B beside unchecked ones of A)."""
+    torch, dt = torch_dev, DT[kind]
+    for uplo in (0, 1):
+        rng = np.random.default_rng(M + N)
+        a, x = rng.integers(-1, 2, (M, M)).astype(np.float64), rng.integers(-2, 3, (M, N)).astype(np.float64)
+        A = torch.from_numpy(a).to("cuda", getattr(torch, dt))
+        bb, b, ldb, _ = _view(torch, rng, dt, (M, N), 0, 1)
+        b[0].copy_(torch.from_numpy(x))
+        g9._call("trmm", {"H": 0, "S": 1, "D": 3}[kind], 0, uplo, 0, 0, M, N, 1.0, A.data_ptr(), M, b.data_ptr(), ldb)
+        torch.cuda.synchronize()
+        want = (np.triu(a) if uplo else np.tril(a)) @ x
+        assert np.array_equal(b[0].double().cpu().numpy(), want), f"{kind} {M}x{N} uplo={uplo}"
+        assert torch.isnan(bb[:1]).all() and torch.isnan(bb[1 + M * N:]).all()
