@@ -41,8 +41,9 @@ template <bool AK, bool BKC> struct Cfg<double, AK, BKC> {
     static constexpr int small_div = 2;
 };
 
-// GEN9BLAS_SPLITK=n forces n split-K slices (0 or 1: none) and turns the two-k-group tiles off, so that the
-// summation order no longer depends on the shape; -1 when unset.
+// GEN9BLAS_SPLITK=n forces n split-K slices (0 or 1: none) and turns the tiles with k groups, the triangle's slices and the
+// direct FP32 kernel off, so that the FP32 / FP64 summation order depends on K alone and not on the other sizes; -1 when
+// unset.
 static int splitk_forced() {
     static int forced = -2;
     if (forced == -2) {
@@ -359,15 +360,18 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     // 64×64 -> these: 1024×500 43.9 -> 20.0, 512×500 22.0 -> 11.2, 1024×16 39.4 -> 15.6; 1024×1000 44.2 -> 26.9 (32×32:
     // 32.3); 1024×2048 45.4 against 48.0, 512×4096 27.6 against 29.3.
     constexpr TileCfg half_wide{32, 64, 1, 2};
-    const int cls = ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
+    // A forced split-K asks for one summation order: 64×64 tiles (FP32's small ones) without k groups, as the k range of
+    // a row, and so its order of k-steps, follows the tile.
+    const bool fixed = !half && splitk_forced() >= 0;
+    const int cls = fixed ? (dbl ? 2 : 1) : ntiles(CF::big) >= want ? 0 : (!dbl || ntiles(CF::small) >= want) ? 1 : 2;
     const auto go = [&](auto kc) -> int {
         constexpr int K = decltype(kc)::value;
         if constexpr (!dbl)
             if (!unchecked_ok<T>(false, p.ldb)) return launch_klim_t<T, TILE64, K, 1, CHECKED>(p, c.count);
         if (cls == 0) return launch_klim_t<T, CF::big, K>(p, c.count);
         if constexpr (dbl) {
-            if (ntiles(TILE32) <= 2LL * num_cus) return launch_klim_t<T, TILE32, K, 4>(p, c.count);
-            if (ntiles(half_wide) <= 2LL * num_cus) return launch_klim_t<T, half_wide, K, 2>(p, c.count);
+            if (!fixed && ntiles(TILE32) <= 2LL * num_cus) return launch_klim_t<T, TILE32, K, 4>(p, c.count);
+            if (!fixed && ntiles(half_wide) <= 2LL * num_cus) return launch_klim_t<T, half_wide, K, 2>(p, c.count);
             if (cls == 2) return launch_klim_t<T, TILE64, K>(p, c.count);
         }
         return launch_klim_t<T, CF::small, K>(p, c.count);

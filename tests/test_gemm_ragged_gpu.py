@@ -131,3 +131,50 @@ def test_trmm_narrow(g9, torch_dev, kind, M, N):
         want = (np.triu(a) if uplo else np.tril(a)) @ x
         assert np.array_equal(b[0].double().cpu().numpy(), want), f"{kind} {M}x{N} uplo={uplo}"
         assert torch.isnan(bb[:1]).all() and torch.isnan(bb[1 + M * N:]).all()
+
+
+ORDER_CHILD = r"""
+import sys, numpy as np, torch
+sys.path.insert(0, sys.argv[1])
+import gen9blas as g
+gen = torch.Generator(device="cuda").manual_seed(1)
+rnd = lambda *s, dt: torch.randn(s, generator=gen, device="cuda", dtype=torch.float64).to(dt)
+for dt in (torch.float32, torch.float64):
+    for K in (64, 96, 700, 704, 2048):
+        for ta in (0, 1):
+            for tb in (0, 1):
+                a, b = rnd(1200, K, dt=dt), rnd(K, 900, dt=dt)
+                A = a.t().contiguous().t() if ta else a
+                B = b.t().contiguous().t() if tb else b
+                C = g.gemm(A, B)
+                for M, N in ((1100, 900), (128, 128), (64, 200), (1200, 70), (257, 129)):
+                    assert torch.equal(g.gemm(A[:M], B[:, :N]), C[:M, :N]), ("gemm", dt, K, ta, tb, M, N)
+        X = rnd(300, K, dt=dt)
+        S = g.syrk(X)
+        for N in (64, 100, 256):
+            assert torch.equal(torch.tril(g.syrk(X[:N])), torch.tril(S[:N, :N])), ("syrk", dt, K, N)
+    for n in (320, 700):
+        T = rnd(n, n, dt=dt) / n ** 0.5 + 2 * torch.eye(n, dtype=dt, device="cuda")
+        B = rnd(n, 4096, dt=dt)
+        for uplo in "LU":
+            for name in ("trmm", "trsm"):
+                want = getattr(g, name)(T, B, uplo=uplo)
+                for N in (16, 64, 500, 1500):
+                    got = getattr(g, name)(T, B[:, :N].contiguous(), uplo=uplo)
+                    assert torch.equal(got, want[:, :N]), (name, dt, n, uplo, N)
+print("ok")
+"""
+
+
+def test_forced_split_fixes_the_order(tmp_path):
+    """With GEN9BLAS_SPLITK set, an element of an FP32 or FP64 product is the same whatever the other sizes of the call: the
+    k groups, slices and tiles that the number of tiles would choose are off, and whole tiles sum in the edge tiles' order."""
+    import os
+    import subprocess
+    import sys
+    script = tmp_path / "order.py"
+    script.write_text(ORDER_CHILD)
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(__file__))), "gen9-gpu-blas_amd")
+    r = subprocess.run([sys.executable, str(script), pkg], env=dict(os.environ, GEN9BLAS_SPLITK="0"), capture_output=True,
+                       text=True, timeout=110)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stderr[-2000:]
