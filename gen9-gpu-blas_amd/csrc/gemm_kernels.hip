@@ -253,12 +253,16 @@ static int launch_tri_t(GemmParams<typename Mma<T>::Sum> p) {
     if constexpr (sizeof(T) == 8) {
         constexpr int BK = 128 / (int)sizeof(T);
         int ns = (int)std::min<long long>({4LL * num_cus / tiles, p.K / TRI_SLICE_K, TRI_SLICES});
-        if (ns > 1 && splitk_forced() < 0) {
+        void *P = nullptr;
+        if (ns > 1 && splitk_forced() < 0) {   // fewer slices, or none, where the work space could not be had
+            size_t work;
+            P = splitk_workspace(&work);
+            ns = (int)std::min<size_t>(ns, work / ((size_t)p.M * p.M * sizeof(T)));
+        }
+        if (ns > 1 && P) {
             auto q = p;
             q.kper = ((p.K + ns - 1) / ns + BK - 1) / BK * BK;
             ns = (p.K + q.kper - 1) / q.kper;
-            void *P;
-            G9_TRY(scratch(SLOT_P, (size_t)ns * p.M * p.M * sizeof(T), &P));
             q.C = P;
             q.ldc = p.M;
             q.sA = q.kper * (AK ? 1 : p.lda);

@@ -51,8 +51,8 @@ struct Choice { int cfg, slices; };
 // them. A few (µs, chosen / others): 48×4096×4096 NT 64×64 in 4 slices 12.9 / unsplit 23.6, in 2 15.6; 600×4096×11008
 // 128×256 in 3 slices 74.9 / 128×128 unsplit 103; 2000×4096×4096 256×128 61.6 / 128×128 77.3, 256×256 98.1;
 // 700×700×6000 TN 128×128 in 6 slices 22.3 / 64×64 in 2 30.3; 1500³ 128×128 16.7 / 64×64 24.0. Slices hold at least 256 k
-// and fit the work space that the split-K bound of the general kernels gives.
-static Choice choose(const GemmCall &c, bool can_split) {
+// and fit the `work` bytes of the split-K work space.
+static Choice choose(const GemmCall &c, size_t work) {
     static constexpr int SLICES[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const double in_bytes = 2.0 * c.count * ((double)c.M * c.K + (double)c.K * c.N);
     Choice best{0, 1};
@@ -63,8 +63,8 @@ static Choice choose(const GemmCall &c, bool can_split) {
         const long long tiles = tiles_of(g, c.M, c.N) * c.count;
         for (const int s : SLICES) {
             const int kper = ((c.K + s - 1) / s + KB - 1) / KB * KB, ns = (c.K + kper - 1) / kper;
-            if (s > 1 && (!can_split || kper < 256 || tiles * s > 3LL * num_cus ||
-                          (size_t)(ns * tiles) * g.BM * g.BN * sizeof(float) > num_cus * SPLITK_TILE_BYTES_MAX)) break;
+            if (s > 1 && (kper < 256 || tiles * s > 3LL * num_cus ||
+                          (size_t)(ns * tiles) * g.BM * g.BN * sizeof(float) > work)) break;
             const bool shared = g.BM == 64;
             const double wgs = (double)(tiles * ns), per_cu = wgs / num_cus, rounds = std::ceil(per_cu);
             const double hbm = in_bytes / std::min(6e6, 2.84e4 * std::min(wgs, (shared ? 3.0 : 1.0) * num_cus));
@@ -159,10 +159,11 @@ static bool launch_hgemm_tiles(const GemmCall &c, int *rc) {
     const bool whole128 = aligned && c.M % 128 == 0 && c.N % 128 == 0 && c.K % KB == 0;
     if (splitk_forced() >= 0 && !whole128) return false;
     // the work space of split products is reserved at its bound with the first product here, so that no later call waits
-    // for queued work to let it grow; without memory for it, products run unsplit
+    // for queued work to let it grow
     void *P = nullptr;
-    if (!batch && splitk_forced() < 0) P = splitk_workspace();
-    const Choice ch = choose(c, P != nullptr);
+    size_t work = 0;
+    if (!batch && splitk_forced() < 0) P = splitk_workspace(&work);
+    const Choice ch = choose(c, work);
     const HgCfg &g = CFG[ch.cfg];
     if (tiles_of(g, c.M, c.N) > 0x7fffffffLL) return false;
     const bool whole = aligned && c.M % g.BM == 0 && c.N % g.BN == 0 && c.K % KB == 0;

@@ -46,13 +46,15 @@ G9_HIDDEN int scratch(int slot, size_t bytes, void **p);
 // placed at `base` if they fit in `bytes`, and every other request (staging of host operands, other work buffers)
 // fails with INVALID_ARG. set_fixed_workspace(nullptr, 0) returns to the growing buffers.
 G9_HIDDEN void set_fixed_workspace(void *base, size_t bytes, const char *who);
-// Largest split-K partial tile, in bytes: the FP16 256×256 tile of FP32 sums and the FP64 256×128 tile of FP64 sums.
-// A split of s > 1 slices is chosen only while tiles · s ≤ CUs, so the slices of one product never exceed
-// CUs × this many bytes (the launch asserts every split tile against it).
+// Bound of the partial sums of one split product, per CU: the largest split tile, the FP16 256×256 one of FP32 sums or the
+// FP64 256×128 one of FP64 sums. The general kernels split into s > 1 slices only while tiles · s ≤ CUs (a launch asserts
+// each split tile against this), the triangle's slices hold four 64×64 FP64 tiles per CU and half of each is off the
+// triangle, and the direct FP16 and FP32 kernels compare the bytes of each split that they consider with the work space.
 constexpr size_t SPLITK_TILE_BYTES_MAX = 256 * 256 * 4;
-// The split-K work space (SLOT_P) at its bound of num_cus × SPLITK_TILE_BYTES_MAX bytes, or null (with no error set) when
-// there is no memory for it.
-G9_HIDDEN void *splitk_workspace();
+// The split-K work space (SLOT_P) and its size: num_cus × SPLITK_TILE_BYTES_MAX bytes (64 MiB), taken with the first call;
+// without memory for that, half of it, a quarter and so on, or what is there already, tried again after some hundreds of
+// calls. *bytes may be 0; no error is set.
+G9_HIDDEN void *splitk_workspace(size_t *bytes);
 // Set-up of the no-allocation entry point on `dev` (called by init with `dev` current): finds the device address of
 // its static work space. A failure is kept and reported by that entry point only.
 G9_HIDDEN void noalloc_setup(int dev);

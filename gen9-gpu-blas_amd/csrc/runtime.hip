@@ -172,13 +172,36 @@ int scratch(int slot, size_t bytes, void **p) {
     return 0;
 }
 
-void *splitk_workspace() {
-    void *p = nullptr;
-    if (scratch(SLOT_P, (size_t)num_cus * SPLITK_TILE_BYTES_MAX, &p)) {
-        gst = 0;
-        return nullptr;
+void *splitk_workspace(size_t *bytes) {
+    const size_t bound = (size_t)num_cus * SPLITK_TILE_BYTES_MAX;
+    if (fixed_base) {
+        *bytes = fixed_bytes < bound ? fixed_bytes : bound;
+        return fixed_base;
     }
-    return p;
+    constexpr int RETRY = 256;   // calls between attempts: an allocation that fails is not cheap either
+    static int wait;
+    if (ssize[SLOT_P] < bound && wait-- <= 0) {
+        // The new buffer comes first: without memory for it the old one stays, and nothing is waited for.
+        void *p = nullptr;
+        size_t nb = bound;
+        for (; nb > ssize[SLOT_P] && nb >= (2u << 20); nb /= 2) {
+            if (hipMalloc(&p, nb) == hipSuccess) break;
+            (void)hipGetLastError();
+            p = nullptr;
+        }
+        if (p && sbuf[SLOT_P] && (hipStreamSynchronize(stream) != hipSuccess || hipFree(sbuf[SLOT_P]) != hipSuccess)) {
+            (void)hipFree(p);
+            *bytes = 0;
+            return nullptr;
+        }
+        if (p) {
+            sbuf[SLOT_P] = p;
+            ssize[SLOT_P] = nb;
+        }
+        wait = ssize[SLOT_P] < bound ? RETRY : 0;
+    }
+    *bytes = ssize[SLOT_P] < bound ? ssize[SLOT_P] : bound;
+    return sbuf[SLOT_P];
 }
 
 // ---------------- operand resolution ----------------

@@ -43,9 +43,9 @@ static double cost(const SgCfg &g, long long tiles, int kper, int ns) {
     if (ns > 1) t += 0.8 + (double)(ns * tiles) * g.BM * g.BN * 8 / 1e7;
     return t;
 }
-// The cheapest configuration and split of K; tri: the tiles of a triangle of side M (square tiles only); big: 128×256 tiles
+// The cheapest configuration and split of K into slices that fit `work` bytes; tri: the tiles of a triangle of side M (square tiles only); big: 128×256 tiles
 // may be taken (their edge-capable variant would need more registers than a wave has).
-static Choice choose(const GemmCall &c, bool can_split, bool tri, bool big) {
+static Choice choose(const GemmCall &c, size_t work, bool tri, bool big) {
     static constexpr int SLICES[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
     Choice best{2, 1, 1e30};
     for (int i = 0; i < NCFG; i++) {
@@ -57,8 +57,8 @@ static Choice choose(const GemmCall &c, bool can_split, bool tri, bool big) {
             int kper;
             const int ns = s == 1 ? 1 : slices_of(c.K, s, kper);
             if (s == 1) kper = (c.K + KB - 1) / KB * KB;
-            if (s > 1 && (!can_split || i == 0 || kper < 4 * KB || tiles * s > 5LL * num_cus ||
-                          (size_t)(ns * tiles) * g.BM * g.BN * sizeof(float) > num_cus * SPLITK_TILE_BYTES_MAX)) break;
+            if (s > 1 && (i == 0 || kper < 4 * KB || tiles * s > 5LL * num_cus ||
+                          (size_t)(ns * tiles) * g.BM * g.BN * sizeof(float) > work)) break;
             const double t = cost(g, tiles, kper, ns);
             if (t < best.us) best = Choice{i, ns, t};
         }
@@ -164,11 +164,12 @@ static int whole_block(const GemmCall &c) {
     }
     return 0;
 }
-static sg::Params sg_work(const GemmCall &c, bool batch) {   // parameters, with the work space of split products
+static sg::Params sg_work(const GemmCall &c, bool batch, size_t &work) {   // parameters, with the work space of split products
     sg::Params p = sg_params(c);
+    work = 0;
     if (batch) return p;
     p.sA = p.sB = p.sC = 0;
-    p.P = reinterpret_cast<float *>(splitk_workspace());
+    p.P = reinterpret_cast<float *>(splitk_workspace(&work));
     return p;
 }
 
@@ -176,8 +177,9 @@ static sg::Params sg_work(const GemmCall &c, bool batch) {   // parameters, with
 // 220 µs (1137 on 136 unsplit tiles of 64×64), of 13321×896 95 (466).
 static bool sg_tri(const GemmCall &c, bool lower, int *rc) {
     if (c.M != c.N || c.count != 1 || !sgemm_direct_ok(c) || c.tA == c.tB) return false;
-    const sg::Params p = sg_work(c, false);
-    const sgl::Choice ch = sgl::choose(c, p.P != nullptr, true, false);
+    size_t work;
+    const sg::Params p = sg_work(c, false, work);
+    const sgl::Choice ch = sgl::choose(c, work, true, false);
     // whole tiles (sums blocked per 128 or 256 k, as whole_block) where they fill the CUs, 64×64 ones unless 128×128 fill
     // their last round as well
     const long long s64 = c.M / 64, s128 = c.M / 128, t64 = s64 * (s64 + 1) / 2, t128 = s128 * (s128 + 1) / 2;
@@ -270,10 +272,11 @@ static bool sg_strip(const GemmCall &c, const sg::Params &p0, double us, int *rc
 static bool launch_sgemm_direct(const GemmCall &c, int *rc) {
     if (!sgemm_direct_ok(c)) return false;
     const bool batch = c.count > 1;
-    const sg::Params p = sg_work(c, batch);
+    size_t work;
+    const sg::Params p = sg_work(c, batch, work);
     const bool tiles_ok = sgemm_tiles_ok(c);
     const int block = tiles_ok ? whole_block(c) : 0;
-    const sgl::Choice ch = sgl::choose(c, p.P != nullptr, false, block >= sgl::CFG[0].BLK && c.M % 128 == 0 && c.N % 256 == 0);
+    const sgl::Choice ch = sgl::choose(c, work, false, block >= sgl::CFG[0].BLK && c.M % 128 == 0 && c.N % 256 == 0);
     const sgl::SgCfg &g = sgl::CFG[ch.cfg];
     if ((long long)((c.M + g.BM - 1) / g.BM) * ((c.N + g.BN - 1) / g.BN) > 0x7fffffffLL) return false;
     if (sg_strip(c, p, ch.us, rc)) return true;
