@@ -42,6 +42,9 @@ enum Slot { SLOT_A = 0, SLOT_B, SLOT_C, SLOT_P, SLOT_Q, SLOT_T, SLOT_X, SLOT_Y, 
 // Device scratch owned by the library, grown on demand and kept between calls (the reference's work buffers,
 // reference: lib/src/core.c:272-277). Growing waits for queued work first.
 G9_HIDDEN int scratch(int slot, size_t bytes, void **p);
+// The same for callers that can do without: null, with no error set, when there is no memory for it or a fixed work space
+// is set.
+G9_HIDDEN void *try_scratch(int slot, size_t bytes);
 // While a fixed work space is set (base != nullptr), scratch() allocates nothing: the split-K slices (SLOT_P) are
 // placed at `base` if they fit in `bytes`, and every other request (staging of host operands, other work buffers)
 // fails with INVALID_ARG. set_fixed_workspace(nullptr, 0) returns to the growing buffers.

@@ -248,33 +248,21 @@ template <bool NTL, class T> __device__ __forceinline__ Vec<T> vload_a(const T *
     else v.u = *q;
     return v;
 }
-// Elements j .. j + V - 1 of x; XC: contiguous.
-template <class T, bool XC> __device__ __forceinline__ Vec<T> vload_x(const T *x, ll j, ll ix) {
-    Vec<T> v;
-    if constexpr (XC) {
-        v.u = *reinterpret_cast<const typename Unaligned<(int)sizeof(T)>::type *>(x + j);
-    } else {
-#pragma unroll
-        for (int e = 0; e < VW<T>; e++) v.e[e] = x[(j + e) * ix];
-    }
-    return v;
-}
-
 // No-trans, y = alpha·A·x + beta·y: RWN rows per group of KS waves, whose lanes stream 16 bytes of each row per step
 // (1 KiB per row and wave, steps dealt to the waves in turn) and reuse each chunk of x for the RWN rows. The RWN sums
-// are reduced across the wave by the transposing butterfly, the KS waves' sums added in LDS in wave order. Two steps
-// per batch: 4 take 101 registers and halve the waves of a SIMD (40000×200 FP32 7.8 µs against 5.6), 1 leaves too few
-// bytes in flight on long rows (1000×8192 7.5 against 5.8).
-// MI355X, µs per call, FP32 unless said, before (element-wise loads for rows not 16-byte aligned, a block of 16 rows
-// throughout) -> now: 6000×1501 10.3 -> 5.8, 6000×1500 6.5 -> 5.8, 1000×8192 13.5 -> 5.3, 300×40000 75 -> 12,
-// 16384×16383 188 -> 168, FP16 8191×4097 23.2 -> 11.3.
+// are reduced across the wave by the transposing butterfly, the KS waves' sums added in LDS in wave order. U steps per
+// batch. VEC false: an element per lane and step, for short rows, which would leave most lanes of a 16-byte step idle, and
+// for an x with a stride, whose elements the lanes then load side by side.
+// MI355X, µs per call, FP32 unless said; before the 16-byte loads at element alignment (element-wise loads for rows not
+// 16-byte aligned, 16 rows per block throughout) -> now: 6000×1501 10.3 -> 5.8, 6000×1500 6.5 -> 5.8, 1000×8192 13.5 -> 5.3,
+// 300×40000 75 -> 12, 16384×16383 188 -> 168, FP16 8191×4097 23.2 -> 11.3.
 constexpr int RWN = 4;
-template <class T, bool XC, bool NTL, int KS>
+template <class T, bool VEC, bool NTL, int KS, int U>
 __global__ void __launch_bounds__(NT) gemv_n_kernel(int M, int N, typename Comp<T>::R alpha, const T *A, ll lda, const T *x,
                                                     ll ix, typename Comp<T>::R beta, T *y, ll iy) {
     static_assert(KS == 1 || KS == NT / 64, "rows of a wave, or of a block");
     using R = typename Comp<T>::R;
-    constexpr int V = VW<T>, U = 2, SW = KS * 64 * V;
+    constexpr int V = VEC ? VW<T> : 1, SW = KS * 64 * V;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r0 = (KS == 1 ? (int)blockIdx.x * (NT / 64) + w : (int)blockIdx.x) * RWN, kw = KS == 1 ? 0 : w;
     if (KS == 1 && r0 >= M) return;
@@ -284,54 +272,82 @@ __global__ void __launch_bounds__(NT) gemv_n_kernel(int M, int N, typename Comp<
     R s[RWN];
 #pragma unroll
     for (int r = 0; r < RWN; r++) s[r] = 0;
-    const int nvec = N - N % V;
-    // US steps from column j0 of this wave; LAST: columns past nvec count as zeros (both factors, so that an infinity
-    // beside them stays out)
-    auto batch = [&](int j0, auto us, auto last) {
-        constexpr int US = decltype(us)::value;
-        constexpr bool LAST = decltype(last)::value;
-        Vec<T> xv[US], av[US][RWN];
+    if constexpr (VEC) {
+        const int nvec = N - N % V;
+        // US steps from column j0 of this wave; LAST: lanes past nvec in the last of them load nothing and add zeros
+        auto batch = [&](int j0, auto us, auto last) {
+            constexpr int US = decltype(us)::value;
+            constexpr bool LAST = decltype(last)::value;
+            Vec<T> xv[US], av[US][RWN];
 #pragma unroll
-        for (int u = 0; u < US; u++) {
-            const unsigned j = (unsigned)j0 + u * SW + lane * V, jc = LAST ? min(j, (unsigned)(nvec - V)) : j;
-            xv[u] = vload_x<T, XC>(x, jc, ix);
+            for (int u = 0; u < US; u++) {
+                const unsigned j = (unsigned)j0 + u * SW + lane * V;
+                const auto load = [&] {
+                    xv[u].u = *reinterpret_cast<const typename Unaligned<(int)sizeof(T)>::type *>(x + j);
 #pragma unroll
-            for (int r = 0; r < RWN; r++) av[u][r] = vload_a<NTL>(ar[r] + jc);
-        }
-        if constexpr (LAST) {
-            const u32x4 z = {0u, 0u, 0u, 0u};
-            if ((unsigned)j0 + (US - 1) * SW + lane * V >= (unsigned)nvec) {   // only the last step can be partial
-                xv[US - 1].u = z;
+                    for (int r = 0; r < RWN; r++) av[u][r] = vload_a<NTL>(ar[r] + j);
+                };
+                if (LAST && u == US - 1) {
+                    xv[u].u = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int r = 0; r < RWN; r++) av[US - 1][r].u = z;
+                    for (int r = 0; r < RWN; r++) av[u][r].u = u32x4{0u, 0u, 0u, 0u};
+                    if (j < (unsigned)nvec) load();
+                } else {
+                    load();
+                }
             }
+#pragma unroll
+            for (int u = 0; u < US; u++)
+#pragma unroll
+                for (int r = 0; r < RWN; r++)
+#pragma unroll
+                    for (int e = 0; e < V; e++) s[r] = fma_r((R)av[u][r].e[e], (R)xv[u].e[e], s[r]);
+        };
+        using No = std::false_type;
+        using Yes = std::true_type;
+        int j0 = kw * 64 * V;
+        for (; nvec - j0 >= U * SW; j0 += U * SW) batch(j0, std::integral_constant<int, U>(), No());
+        // the columns past the last whole 16 bytes, one per lane of the first wave, loaded ahead of the last batch
+        const bool tail = kw == 0 && nvec + lane < N;
+        R at[RWN], xt = 0;
+#pragma unroll
+        for (int r = 0; r < RWN; r++) at[r] = 0;
+        if (tail) {
+            xt = (R)x[nvec + lane];
+#pragma unroll
+            for (int r = 0; r < RWN; r++) at[r] = (R)ar[r][nvec + lane];
         }
+        const int left = j0 < nvec ? (nvec - j0 + SW - 1) / SW : 0;   // steps of this wave still to do, 0 .. U
+        if constexpr (U > 2) {
+            if (left == 4) batch(j0, std::integral_constant<int, 4>(), Yes());
+            else if (left == 3) batch(j0, std::integral_constant<int, 3>(), Yes());
+        }
+        if (left == 2) batch(j0, std::integral_constant<int, 2>(), Yes());
+        else if (left == 1) batch(j0, std::integral_constant<int, 1>(), Yes());
+        if (tail)
 #pragma unroll
-        for (int u = 0; u < US; u++)
+            for (int r = 0; r < RWN; r++) s[r] = fma_r(at[r], xt, s[r]);
+    } else {
+        ll j = kw * 64 + lane;
+        for (; j + (U - 1) * SW < N; j += U * SW) {
+            T xv[U], av[U][RWN];
 #pragma unroll
-            for (int r = 0; r < RWN; r++)
+            for (int u = 0; u < U; u++) {
+                xv[u] = x[(j + u * SW) * ix];
 #pragma unroll
-                for (int e = 0; e < V; e++) s[r] = fma_r((R)av[u][r].e[e], (R)xv[u].e[e], s[r]);
-    };
-    using No = std::false_type;
-    using Yes = std::true_type;
-    int j0 = kw * 64 * V;
-    for (; nvec - j0 >= U * SW; j0 += U * SW) batch(j0, std::integral_constant<int, U>(), No());
-    // the columns past the last whole 16 bytes, one per lane of the first wave, loaded ahead of the last batch
-    const bool tail = kw == 0 && nvec < N;
-    R at[RWN], xt = 0;
-    if (tail) {
-        const int jt = min(nvec + lane, N - 1);
-        xt = (R)x[(ll)jt * ix];
+                for (int r = 0; r < RWN; r++) av[u][r] = ar[r][j + u * SW];
+            }
 #pragma unroll
-        for (int r = 0; r < RWN; r++) at[r] = (R)ar[r][jt];
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int r = 0; r < RWN; r++) s[r] = fma_r((R)av[u][r], (R)xv[u], s[r]);
+        }
+        for (; j < N; j += SW) {
+            const R xj = (R)x[j * ix];
+#pragma unroll
+            for (int r = 0; r < RWN; r++) s[r] = fma_r((R)ar[r][j], xj, s[r]);
+        }
     }
-    const int left = j0 < nvec ? (nvec - j0 + SW - 1) / SW : 0;   // steps of this wave still to do, 0 .. U
-    if (left == 2) batch(j0, std::integral_constant<int, 2>(), Yes());
-    else if (left == 1) batch(j0, std::integral_constant<int, 1>(), Yes());
-    if (tail && nvec + lane < N)
-#pragma unroll
-        for (int r = 0; r < RWN; r++) s[r] = fma_r(at[r], xt, s[r]);
     // butterfly over the RWN row sums: two halving exchanges, then plain sums
     int base = 0;
     butterfly<0, RWN>(s, lane, base);
@@ -354,6 +370,56 @@ __global__ void __launch_bounds__(NT) gemv_n_kernel(int M, int N, typename Comp<
         T *yp = y + (ll)row * iy;
         *yp = (T)(beta == R(0) ? alpha * sum : fma_r(alpha, sum, beta * (R)*yp));
     }
+}
+
+// Trans, y = alpha·Aᵀ·x + beta·y, at most FEW rows: a thread owns V columns (16 bytes per lane) and all the rows, in four
+// groups whose sums are added in order, as the waves of the kernel below would. Those would have a row or two each, and a
+// pass through LDS after it: MI355X, µs, FP64 × 1000000 columns, 1 row 7.6 -> 5.8, 4 rows 12.5 -> 6.1, FP32 4 rows 7.7 -> 4.7
+// (16 rows: FP16 8.6 against 6.9).
+constexpr int FEW = 8;
+template <class T>
+__global__ void __launch_bounds__(NT) gemv_t_few_kernel(int M, int N, const T *A, ll lda, const T *x, ll ix,
+                                                        typename Comp<T>::R alpha, typename Comp<T>::R beta, T *y, ll iy) {
+    using R = typename Comp<T>::R;
+    constexpr int V = VW<T>, G = FEW / 4;   // rows of a group
+    const ll cb = ((ll)blockIdx.x * NT + threadIdx.x) * V;
+    if (cb >= N) return;
+    const int c0 = (int)max(min(cb, (ll)N - V), 0ll);   // as below: the last thread's columns end with the row
+    const int rw = (M + 3) / 4;
+    Vec<T> av[FEW];
+    R xv[FEW];
+    const auto row = [&](int u) { return min(u / G * rw + min(u % G, rw - 1), M - 1); };
+    if (N >= V) {
+#pragma unroll
+        for (int u = 0; u < FEW; u++) av[u] = vload_a<false>(A + row(u) * lda + c0);
+    } else {
+#pragma unroll
+        for (int u = 0; u < FEW; u++)
+#pragma unroll
+            for (int e = 0; e < V; e++) av[u].e[e] = A[row(u) * lda + min(e, N - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < FEW; u++) xv[u] = (R)x[row(u) * ix];
+    R s[V];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        R t[V];
+#pragma unroll
+        for (int e = 0; e < V; e++) t[e] = 0;
+#pragma unroll
+        for (int u = 0; u < G; u++)
+            if (u < rw && q * rw + u < M)
+#pragma unroll
+                for (int e = 0; e < V; e++) t[e] = fma_r((R)av[q * G + u].e[e], xv[q * G + u], t[e]);
+#pragma unroll
+        for (int e = 0; e < V; e++) s[e] = q == 0 ? t[e] : s[e] + t[e];
+    }
+#pragma unroll
+    for (int e = 0; e < V; e++)
+        if (c0 + e >= cb && c0 + e < N) {
+            T *yp = y + (c0 + e) * iy;
+            *yp = (T)(beta == R(0) ? alpha * s[e] : fma_r(alpha, s[e], beta * (R)*yp));
+        }
 }
 
 // Trans, y = alpha·Aᵀ·x + beta·y. Stage 1: a block owns 64·V columns (16 bytes per lane) and a band of rpp rows, a
@@ -566,26 +632,54 @@ int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll
         using R = typename Comp<T>::R;
         const T *Ap = (const T *)A, *xp = (const T *)x + ox;
         T *yp = (T *)y + oy;
-        // A of more than half the 256 MiB last-level cache is read past it (nontemporal); a smaller one, which a
-        // solver's next product with it finds there, is not. FP32, µs, nontemporal against plain loads: 16384² 162
-        // against 174, 16384×8192 100 against 106; 6000×1501 6.2 against 5.8, FP16 1501×11008 6.4 against 5.3.
-        const bool ntl = (double)M * (double)N * sizeof(T) > (double)(128 << 20);
+        // A of more than the 256 MiB last-level cache is read past it (nontemporal); a smaller one, which a solver's next
+        // product with it finds there, is not. No-trans, µs, nontemporal against plain loads: FP32 16384×8192 (512 MiB) 104 against 122, 32768×4096 92 against 113; FP64 16384×2048 (256 MiB)
+        // 47 against 40.
+        const bool ntl = (double)M * (double)N * sizeof(T) > (double)(256 << 20);
         if (!trans) {
+            // An element per lane: rows of at most 64 of them (FP16: 128), FP32 100000×32 5.4 against 6.2, FP16 ×100 6.1
+            // against 7.9 (×200: 10.2 against 8.1), FP64 1000000×8 47 against 54; and an x with a stride, where rows are
+            // not long nor A large: those have x gathered first. FP16 16384×4096 25 µs (loads of x inside each lane's 16 bytes
+            // instead 39), 8192² gathered 23 (36).
+            bool vec = N > (sizeof(T) == 2 ? 128 : 64);
+            if (vec && ix != 1) {
+                void *g = nullptr;
+                vec = (ntl || N > 2048 * (int)sizeof(T)) && (g = try_scratch(SLOT_P, (size_t)N * sizeof(T)));
+                if (vec) {
+                    G9_TRY(launch_copy(es, N, x, ox, ix, g, 0, 1));
+                    xp = (const T *)g;
+                    ix = 1;
+                }
+            }
             // The four waves of a block share its rows where rows alone would leave CUs with few waves (fewer than 4
             // blocks per CU), unless a row is so short that they would have nothing to share.
             const unsigned g = (unsigned)((M + RWN * (NT / 64) - 1) / (RWN * (NT / 64)));
-            const bool share = g < 4u * (unsigned)num_cus && N > 2 * 64 * VW<T>;
-            const auto go = [&](auto xc, auto ks) {
-                constexpr int KS = decltype(ks)::value;
-                constexpr bool XC = decltype(xc)::value;
-                const auto kern = ntl ? gemv_n_kernel<T, XC, true, KS> : gemv_n_kernel<T, XC, false, KS>;
-                hipLaunchKernelGGL(kern, dim3(KS == 1 ? g : (unsigned)((M + RWN - 1) / RWN)),
-                                   dim3(NT), 0, stream, M, N, (R)alpha, Ap, lda, xp, ix, (R)beta, yp, iy);
+            const bool share = g < 4u * (unsigned)num_cus && N > 2 * 64 * (vec ? VW<T> : 1);
+            // Batches of four steps where a row holds four of them, else of two, whose registers leave more waves: FP16
+            // 16384×2048 11.5 against 13.8, FP32 32768×4096 92 against 101, FP64 40000×3000 137 against 146; FP32 100000×200
+            // (one step) 14.8 against 12.7, 4096² (shared rows, from the cache) 12.4 against 11.2.
+            const bool four = (!share || ntl) && N >= 4 * 64 * VW<T> * (share ? NT / 64 : 1);
+            const auto go = [&](auto vc, auto nt, auto us) {
+                constexpr bool VEC = decltype(vc)::value, NTL = decltype(nt)::value;
+                constexpr int U = decltype(us)::value;
+                const auto kern = share ? gemv_n_kernel<T, VEC, NTL, NT / 64, U> : gemv_n_kernel<T, VEC, NTL, 1, U>;
+                hipLaunchKernelGGL(kern, dim3(share ? (unsigned)((M + RWN - 1) / RWN) : g), dim3(NT), 0, stream, M, N, (R)alpha,
+                                   Ap, lda, xp, ix, (R)beta, yp, iy);
             };
-            using One = std::integral_constant<int, 1>;
-            using All = std::integral_constant<int, NT / 64>;
-            if (ix == 1) share ? go(std::true_type(), All()) : go(std::true_type(), One());
-            else share ? go(std::false_type(), All()) : go(std::false_type(), One());
+            using Yes = std::true_type;
+            using No = std::false_type;
+            using One = std::integral_constant<int, 1>;   // element-wise: waves enough hide a step's loads
+            using Two = std::integral_constant<int, 2>;
+            using Four = std::integral_constant<int, 4>;
+            if (!vec) share ? go(No(), No(), Four()) : go(No(), No(), One());
+            else if (four) ntl ? go(Yes(), Yes(), Four()) : go(Yes(), No(), Four());
+            else ntl ? go(Yes(), Yes(), Two()) : go(Yes(), No(), Two());
+            G9_HIP(hipGetLastError());
+            return 0;
+        }
+        if (M <= FEW) {
+            hipLaunchKernelGGL((gemv_t_few_kernel<T>), dim3((unsigned)(((ll)N + NT * VW<T> - 1) / (NT * VW<T>))), dim3(NT), 0,
+                               stream, M, N, Ap, lda, xp, ix, (R)alpha, (R)beta, yp, iy);
             G9_HIP(hipGetLastError());
             return 0;
         }

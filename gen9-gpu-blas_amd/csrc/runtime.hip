@@ -140,6 +140,8 @@ void set_fixed_workspace(void *base, size_t bytes, const char *who) {
     fixed_who = who;
 }
 
+static size_t scratch_round(size_t bytes) { return (bytes + (1u << 21) - 1) & ~(size_t)((1u << 21) - 1); }
+
 int scratch(int slot, size_t bytes, void **p) {
     if (fixed_base) {
         if (slot != SLOT_P)
@@ -159,7 +161,7 @@ int scratch(int slot, size_t bytes, void **p) {
             sbuf[slot] = nullptr;
             ssize[slot] = 0;
         }
-        size_t nb = (bytes + (1u << 21) - 1) & ~(size_t)((1u << 21) - 1);
+        const size_t nb = scratch_round(bytes);
         hipError_t e = hipMalloc(&sbuf[slot], nb);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -172,6 +174,28 @@ int scratch(int slot, size_t bytes, void **p) {
     return 0;
 }
 
+// A buffer of nb bytes for the slot in place of its smaller one, allocated first, so that without memory for it the old one
+// stays and nothing is waited for; false then.
+static bool replace_scratch(int slot, size_t nb) {
+    void *p = nullptr;
+    if (hipMalloc(&p, nb) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (sbuf[slot] && (hipStreamSynchronize(stream) != hipSuccess || hipFree(sbuf[slot]) != hipSuccess)) {
+        (void)hipFree(p);
+        return false;
+    }
+    sbuf[slot] = p;
+    ssize[slot] = nb;
+    return true;
+}
+
+void *try_scratch(int slot, size_t bytes) {
+    if (fixed_base) return nullptr;
+    return ssize[slot] >= bytes || replace_scratch(slot, scratch_round(bytes)) ? sbuf[slot] : nullptr;
+}
+
 void *splitk_workspace(size_t *bytes) {
     const size_t bound = (size_t)num_cus * SPLITK_TILE_BYTES_MAX;
     if (fixed_base) {
@@ -181,23 +205,8 @@ void *splitk_workspace(size_t *bytes) {
     constexpr int RETRY = 256;   // calls between attempts: an allocation that fails is not cheap either
     static int wait;
     if (ssize[SLOT_P] < bound && wait-- <= 0) {
-        // The new buffer comes first: without memory for it the old one stays, and nothing is waited for.
-        void *p = nullptr;
-        size_t nb = bound;
-        for (; nb > ssize[SLOT_P] && nb >= (2u << 20); nb /= 2) {
-            if (hipMalloc(&p, nb) == hipSuccess) break;
-            (void)hipGetLastError();
-            p = nullptr;
-        }
-        if (p && sbuf[SLOT_P] && (hipStreamSynchronize(stream) != hipSuccess || hipFree(sbuf[SLOT_P]) != hipSuccess)) {
-            (void)hipFree(p);
-            *bytes = 0;
-            return nullptr;
-        }
-        if (p) {
-            sbuf[SLOT_P] = p;
-            ssize[SLOT_P] = nb;
-        }
+        for (size_t nb = bound; nb > ssize[SLOT_P] && nb >= (2u << 20); nb /= 2)
+            if (replace_scratch(SLOT_P, nb)) break;
         wait = ssize[SLOT_P] < bound ? RETRY : 0;
     }
     *bytes = ssize[SLOT_P] < bound ? ssize[SLOT_P] : bound;

@@ -146,6 +146,37 @@ def test_gemv_unaligned_rows(g9, torch_dev, dt, M, N):
         assert np.isposinf(r[n - 1]) and np.isfinite(r[:n - 1]).all(), f"infinity, trans={trans} {M}x{N}"
 
 
+@pytest.mark.parametrize("dt", ["float32", "float16", "float64"])
+@pytest.mark.parametrize("M,N", [(3, 64), (70, 65), (1030, 64), (5, 128), (1030, 129), (50, 4096), (9, 4097), (1, 6000), (2, 1), (4, 7),
+                                 (5, 511), (8, 1025), (13, 2047), (16, 3001), (17, 3000), (33, 40000), ("over", 8191), (8191, "over")])
+def test_gemv_rules(g9, torch_dev, dt, M, N):
+    """Both sides of each line between the GEMV kernels, bit-exact on small integers: rows of 64 and 128 elements, x with a
+    stride at 4096 columns, 16 rows of a transposed product, and a matrix just over 256 MiB. Around the view: NaN."""
+    torch, d = torch_dev, getattr(torch_dev, dt)
+    es = torch.tensor([], dtype=d).element_size()
+    if "over" in (M, N):
+        n = 2 ** 28 // es // 8191 + 9
+        M, N = (n, N) if M == "over" else (M, n)
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    ints = lambda *s: torch.randint(-1, 2, s, generator=gen, device="cuda", dtype=torch.int8).to(d)
+    for pad in (0, 1):
+        W = torch.full((M * (N + pad) + 2 * pad,), float("nan"), dtype=d, device="cuda")
+        A = torch.as_strided(W, (M, N), (N + pad, 1), pad)
+        A.copy_(ints(M, N))
+        for trans in (False, True):
+            Op = A.t() if trans else A
+            X = torch.full((3 * Op.shape[1],), float("nan"), dtype=d, device="cuda")
+            for inc in (1, 3):
+                x, y = X[:inc * Op.shape[1]:inc], ints(2 * Op.shape[0])[::2]
+                # values in a few places, so that FP16 sums stay exact; 1 elsewhere in the matrix must not matter
+                x.zero_()
+                x[torch.randint(0, x.numel(), (200,), generator=gen, device="cuda")] = 1
+                x[-1], x[0] = 1, -1
+                want = 2.0 * (Op.double() * x.double()).sum(1) - y.double()
+                got = g9.gemv(A, x, alpha=2.0, beta=-1.0, y=y, trans=trans)
+                assert torch.equal(got.double(), want), f"{M}x{N} pad={pad} trans={trans} inc={inc}"
+
+
 def test_level2_config_device(g9, orc, torch_dev):
     """The benchmarked level 1/2 configuration at full size on device buffers: SAXPY, SDOT (2^26), SGEMV N/T (16384²)."""
     torch = torch_dev
