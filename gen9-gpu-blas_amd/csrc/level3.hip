@@ -137,10 +137,16 @@ __global__ void __launch_bounds__(256) trsm_store_kernel(const T *Y, T *B, ll ld
 constexpr int TRSM_NB = 128;
 // rows of a leaf (an inverted diagonal block applied by one product) of the FP32 and the FP64 solve: one more
 // composition level and half the leaves for FP64 (n = 4096 left lower, MI355X: 1.427 -> 1.412 ms with 1024 rows
-// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured). FP64 solves of up to TRSM_LEAF_D_FROM rows take
-// 512 too, as one or two leaves do not repay the level (2000×500 219 -> 209 µs, 1024×2048 142 -> 127, 3000×130 270 ->
-// 261; 4096×500 346 against 378)
-constexpr int TRSM_LEAF_S = 512, TRSM_LEAF_D = 1024, TRSM_LEAF_D_FROM = 3072;
+// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured). FP64 solves of up to TRSM_LEAF_D_FROM rows with fewer
+// than TRSM_LEAF_D_WORK elements of B take 512 too, as one or two leaves do not repay the level (µs, 512 against 1024 rows:
+// 1024×16 91 against 109, 2048×512 165 against 168, 2800×512 273 against 265, 3072×2000 473 against 485); with more the
+// products on whole leaves do (2800×4096 842 against 755, 3000² 874 against 753, 3072×8192 1713 against 1526, 2300×8192 1164
+// against 1134).
+constexpr int TRSM_LEAF_S = 512, TRSM_LEAF_D = 1024, TRSM_LEAF_D_FROM = 3072, TRSM_LEAF_D_WORK = 9000000;
+static int trsm_leaf(int es, int n, int m) {
+    if (es == 8 && (n > TRSM_LEAF_D_FROM || (n > 2 * TRSM_LEAF_D && (ll)n * m >= TRSM_LEAF_D_WORK))) return TRSM_LEAF_D;
+    return es >= 4 ? TRSM_LEAF_S : TRSM_NB;
+}
 // Inverse of the diagonal block bi of L (rows and columns r0 .. r0+b-1, b ≤ TRSM_NB, in the leaf p = r0 / lb of lb
 // rows whose element (i, j) is at L[p·bstride + i·ld + j]; the block's entries above the diagonal are read as zeros,
 // and its diagonal as ones when unit),
@@ -557,7 +563,7 @@ int gen9blas_trsm(int type, int side, int uplo, int transA, int diag, int M, int
     const int lower = (uplo == GEN9BLAS_LOWER) != (tr != 0), rev = !lower;
     // Leaves of TRSM_LEAF_S / _D rows for FP32 / large FP64: each leaf inverse is composed from the 128-row FP64 inverses (below);
     // FP16 keeps 128-row leaves (the composition would round once more in FP16)
-    const int nbl = (n + TRSM_NB - 1) / TRSM_NB, lb = es == 8 && n > TRSM_LEAF_D_FROM ? TRSM_LEAF_D : es >= 4 ? TRSM_LEAF_S : TRSM_NB, nleaf = (n + lb - 1) / lb;
+    const int nbl = (n + TRSM_NB - 1) / TRSM_NB, lb = trsm_leaf(es, n, m), nleaf = (n + lb - 1) / lb;
     // A left solve with A lower and not transposed reads both operands where they lie: every product below reads L
     // strictly below its diagonal blocks, the block inversion masks the rest of A itself, B is the right-hand side
     // updated in place (alpha applied by the first product that touches each block of rows), and only the solution

@@ -295,6 +295,31 @@ def test_trsm_paired_leaf_products(g9, kind, dt, tol):
         assert e <= tol, f"trsm {kind} L{uplo} {n}x{m}: {e:.1e}"
 
 
+@pytest.mark.parametrize("n,m", [(3073, 5), (3700, 40), (4096, 17), (2300, 3913), (2300, 3914)])
+def test_trsm_fp64_leaves_of_1024(g9, torch_dev, n, m):
+    """FP64 solves on leaves of 1024 rows: a last leaf of one row, of 628 rows (composed from 512 and 116, 128-row blocks
+    before that) and whole ones; both sides of the line in n·m below 3073 rows. In place with huge values in A's other
+    triangle (and unit diagonal), then the upper triangle, transposed, and the right side, against float64 (n eps = 4.5e-13)."""
+    import scipy.linalg
+    torch = torch_dev
+    rng = np.random.default_rng(n + m)
+    A = rng.uniform(-1, 1, (n, n)) / n
+    A[np.diag_indices(n)] = 1.0 + rng.uniform(0, 1, n)
+    B = rng.uniform(-1, 1, (n, m))
+    calls = [("L", "L", False, False), ("L", "L", False, True), ("L", "U", True, False), ("R", "L", False, False)]
+    for side, uplo, ta, dg in calls if n > 3072 else calls[:1]:
+        G = A.copy()
+        G[np.triu_indices(n, 1) if uplo == "L" else np.tril_indices(n, -1)] = 1e300
+        if dg:
+            G[np.diag_indices(n)] = 1e300
+        Gd, Bd = torch.from_numpy(G).cuda(), torch.from_numpy(B if side == "L" else np.ascontiguousarray(B.T)).cuda()
+        X = g9.trsm(Gd, Bd, side, uplo, ta, dg, 0.5).cpu().numpy()
+        trans = ta if side == "L" else not ta
+        Xr = scipy.linalg.solve_triangular(A, 0.5 * B, trans=int(trans), lower=uplo == "L", unit_diagonal=dg)
+        e = np.abs((X if side == "L" else X.T) - Xr).max() / np.abs(Xr).max()
+        assert e <= 1e-12, f"trsm D {side}{uplo} tA={ta} diag={dg} {n}x{m}: {e:.1e}"
+
+
 def _l3_cases(seed, count):
     """Seeded random level-3 calls: operation, type, side / triangle / transpose / unit diagonal, and dimensions that
     are small (1-79), multiples of 64 (the whole-tile classes of the GEMMs underneath), within 3 of one, or 80-599."""
