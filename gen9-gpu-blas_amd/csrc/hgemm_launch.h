@@ -32,29 +32,32 @@ static long long lane_span(bool kc, long long ldb, int MN, int kb) { return (kc 
 namespace hgl {
 
 constexpr int KB = 64;   // k per k-step
-// ns: time per k of a round of one tile per CU on the whole chip, for choose()
-struct HgCfg { int BM, BN, WM, WN, NS; bool RA; double ns; };
-constexpr HgCfg CFG[] = {{256, 256, 2, 4, 2, false, 27.8}, {128, 128, 2, 4, 3, false, 8.42}, {64, 64, 2, 2, 3, true, 5.04},
-                         {256, 192, 4, 2, 2, false, 22.8}, {192, 256, 2, 4, 2, false, 22.8},
-                         {256, 128, 4, 2, 3, false, 14.3}, {128, 256, 2, 4, 3, false, 14.3}};
+// For choose(): ns, time per k of a round of one tile per CU on the whole chip; fix, the rest of a round (µs); st, µs per MB
+// of C stored
+struct HgCfg { int BM, BN, WM, WN, NS; bool RA; double ns, fix, st; };
+constexpr HgCfg CFG[] = {{256, 256, 2, 4, 2, false, 25, 3.1, 0.062}, {128, 128, 2, 4, 3, false, 8.1, 1.8, 0.037},
+                         {64, 64, 2, 2, 3, true, 3.3, 1.8, 0}, {256, 192, 4, 2, 2, false, 22, 2.1, 0.064},
+                         {192, 256, 2, 4, 2, false, 22, 2.1, 0.064}, {256, 128, 4, 2, 3, false, 13.07, 3, 0.044},
+                         {128, 256, 2, 4, 3, false, 13, 3, 0.044}};
 constexpr int NCFG = sizeof CFG / sizeof CFG[0];
 
 static long long tiles_of(const HgCfg &g, int M, int N) { return (long long)((M + g.BM - 1) / g.BM) * ((N + g.BN - 1) / g.BN); }
 
 struct Choice { int cfg, slices; };
-// The configuration and number of K slices with the smallest estimated time (µs): a launch, then rounds of one tile per
-// CU (64×64: three share a CU), each a fixed part and the tile's time per k (less where part of the chip idles: the
-// board's power limit leaves the rest a higher clock), and no less than the operands take from HBM with what the
-// workgroups in flight can draw; for slices, the second kernel and the FP32 sums written and read. The constants are a
-// fit to 34 products (K 146 to 11008, 20 to 8192 rows, whole and ragged, NN / NT / TN / TT, operands rotated beyond the
-// last-level cache) timed with every configuration and 1-16 slices: the choice is within 10 % of the fastest for each of
-// them. A few (µs, chosen / others): 48×4096×4096 NT 64×64 in 4 slices 12.9 / unsplit 23.6, in 2 15.6; 600×4096×11008
-// 128×256 in 3 slices 74.9 / 128×128 unsplit 103; 2000×4096×4096 256×128 61.6 / 128×128 77.3, 256×256 98.1;
-// 700×700×6000 TN 128×128 in 6 slices 22.3 / 64×64 in 2 30.3; 1500³ 128×128 16.7 / 64×64 24.0. Slices hold at least 256 k
-// and fit the `work` bytes of the split-K work space.
+// The configuration and number of K slices with the smallest estimated time (µs): a launch; rounds of one tile per CU
+// (64×64: two share a CU, one alone takes two thirds of their time), each a fixed part and the tile's time per k, less where
+// part of the chip idles (the board's power limit leaves the rest a higher clock); C written by the larger tiles, which most costs where its rows are
+// not whole 128-byte lines; for slices, the second kernel, its pass over each slice, and the FP32 sums written and read.
+// The constants are a fit to the order of 392 products (K 64 to 11008, 17 to 20000 rows, batches, whole and ragged, NN /
+// NT / TN), each timed with every configuration and 1-16 slices on operands in the last-level cache and rotated beyond it:
+// by the geometric mean of both the choice is 0.6 % from the fastest on average, and within 22 % for all. A few (µs,
+// in the cache and beyond it, chosen / others): 48×4096×4096 NT 64×64 in 4 slices 10.7 and 12.7 / unsplit 21 and 23;
+// 600×4096×11008 128×256 in 3 slices 74 / 128×128 unsplit 103; 256×1024×1024 64×64 5.4 and 8.2 / in 3 slices 7.5 and 8.5;
+// 1280³ 64×64 9.1 and 11.7 / 128×128 11.3 and 14.4; 5000×5000×64 64×64 or 128×128 27 and 31 / 256×256 41 and 48. Slices hold
+// at least 256 k and fit the `work` bytes of the split-K work space.
 static Choice choose(const GemmCall &c, size_t work) {
     static constexpr int SLICES[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    const double in_bytes = 2.0 * c.count * ((double)c.M * c.K + (double)c.K * c.N);
+    const double mn = (double)c.M * c.N, c_mb = 2e-6 * c.count * mn * (c.ldc % 64 ? 7 : 1);
     Choice best{0, 1};
     double t_best = 1e30;
     for (int i = 0; i < NCFG; i++) {
@@ -66,11 +69,11 @@ static Choice choose(const GemmCall &c, size_t work) {
             if (s > 1 && (kper < 256 || tiles * s > 3LL * num_cus ||
                           (size_t)(ns * tiles) * g.BM * g.BN * sizeof(float) > work)) break;
             const bool shared = g.BM == 64;
-            const double wgs = (double)(tiles * ns), per_cu = wgs / num_cus, rounds = std::ceil(per_cu);
-            const double hbm = in_bytes / std::min(6e6, 2.84e4 * std::min(wgs, (shared ? 3.0 : 1.0) * num_cus));
-            const double body = g.ns * 1e-3 * kper * (shared ? std::max(0.78, per_cu) : 0.86 * rounds + 0.14 * per_cu);
-            double t = 3.2 + std::max(body, hbm) + 2.6 * (shared ? std::max(1.0, rounds / 3) : rounds);
-            if (ns > 1) t += 1.3 + (double)ns * c.M * c.N * 8 / 5.85e6;
+            const double per_cu = (double)(tiles * ns) / num_cus, rounds = std::ceil(per_cu);
+            const double load = 0.8 * rounds + 0.2 * per_cu;
+            const double t = 2.8 + g.ns * 1e-3 * kper * (shared ? std::max(1.3, load) : load) +
+                             g.fix * (shared ? std::max(1.0, per_cu / 2) : rounds) +
+                             (ns > 1 ? 1.8 + 0.46 * ns + ns * mn * 8 / 9.2e6 : g.st * c_mb);
             if (t < t_best) {
                 t_best = t;
                 best = Choice{i, ns};
