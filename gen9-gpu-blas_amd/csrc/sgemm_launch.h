@@ -50,7 +50,9 @@ static Choice choose(const GemmCall &c, size_t work, bool tri, bool big) {
     Choice best{2, 1, 1e30};
     for (int i = 0; i < NCFG; i++) {
         const SgCfg &g = CFG[i];
-        if ((tri && g.BM != g.BN) || (i == 0 && !big)) continue;
+        // a triangle that no whole tiles fill: 128×128 tiles lose half of each on the diagonal, and on this kernel they
+        // were slower throughout (2000×200 22.1 µs against 20.0, 5000×160 50.8 against 40.3)
+        if ((tri && (g.BM != g.BN || (g.BM == 128 && c.M % 64))) || (i == 0 && !big)) continue;
         const long long tm = (c.M + g.BM - 1) / g.BM, tn = (c.N + g.BN - 1) / g.BN;
         const long long tiles = (tri ? tm * (tm + 1) / 2 : tm * tn) * c.count;
         for (const int s : SLICES) {
@@ -175,8 +177,12 @@ static sg::Params sg_work(const GemmCall &c, bool batch, size_t &work) {   // pa
 
 // Triangle of an FP32 square product (NT or TN). K is split where the triangle leaves CUs idle: XᵀX of 20000×1000 takes
 // 220 µs (1137 on 136 unsplit tiles of 64×64), of 13321×896 95 (466).
+// A rank-K update with a short K of a triangle that fills the chip is bound by C, which the general kernel's four workgroups
+// per CU write faster: 2000×64 8.0 against 11.7, 5000×128 38 against 51, at β = 0.5 46 against 62 (1500×128 9.9 either way).
 static bool sg_tri(const GemmCall &c, bool lower, int *rc) {
     if (c.M != c.N || c.count != 1 || !sgemm_direct_ok(c) || c.tA == c.tB) return false;
+    const long long side = (c.M + 63) / 64;
+    if (c.K <= 128 && side * (side + 1) / 2 > 2LL * num_cus) return false;
     size_t work;
     const sg::Params p = sg_work(c, false, work);
     const sgl::Choice ch = sgl::choose(c, work, true, false);
@@ -269,8 +275,11 @@ static bool sg_strip(const GemmCall &c, const sg::Params &p0, double us, int *rc
 }
 
 // FP32 products on this kernel. False, with nothing launched, for those it does not take.
+// Not NT with a short K whose rows of C are not whole 64-byte sectors: C bounds it, and the general kernel writes it
+// faster (β = 0.5, K = 33: 1500² 9.7 against 12.9, 3000² 23 against 32, 5000² 52 against 72, 1000² 5 % less; with whole
+// sectors, 2000² or 4096², 12 % more). From K = 128 on its one running sum would round more than the two here.
 static bool launch_sgemm_direct(const GemmCall &c, int *rc) {
-    if (!sgemm_direct_ok(c)) return false;
+    if (!sgemm_direct_ok(c) || (!c.tA && c.tB && c.K < 128 && c.ldc % 16)) return false;
     const bool batch = c.count > 1;
     size_t work;
     const sg::Params p = sg_work(c, batch, work);

@@ -178,3 +178,17 @@ def test_forced_split_fixes_the_order(tmp_path):
     r = subprocess.run([sys.executable, str(script), pkg], env=dict(os.environ, GEN9BLAS_SPLITK="0"), capture_output=True,
                        text=True, timeout=110)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("N,K", [(2050, 128), (2050, 129), (2049, 40), (1984, 33)])
+def test_ssyrk_short_k(g9, torch_dev, N, K):
+    """FP32 rank-K updates on both sides of the lines in K and in tiles between the kernels."""
+    test_syrk_ragged_and_long(g9, torch_dev, "S", N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 333, 127), (300, 333, 128), (300, 336, 127), (129, 1001, 33)])
+def test_sgemm_short_k(g9, torch_dev, M, N, K):
+    """FP32 NT products with a short K, rows of C of whole 64-byte sectors or not."""
+    for pad, off, beta in [(0, 0, 0.5), (1, 1, 0.0), (2, 2, -1.0)]:
+        check(g9, torch_dev, "S", M, N, K, 0, 1, pad, off, beta, seed=N + K)
+        check(g9, torch_dev, "S", M, N, K, 0, 1, pad, off, beta, count=3, seed=N + K)
