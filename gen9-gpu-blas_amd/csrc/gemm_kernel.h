@@ -89,6 +89,7 @@ template <class S> struct GemmParams {
     S *P;
     int kper;
     int kpair = 0;   // KLIM: the second half of the dispatch order reversed (see the tile mapping)
+    int lastk = 0;   // whole tiles take their last k-step first, as edge tiles do: one order for all elements
 };
 
 // Transpose of a V×V block held as V rows of 16 bytes: out[j] element i = in[i] element j.
@@ -399,8 +400,9 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     // Whole tiles and k-steps load without bounds tests. So do the other shapes, but for their last k-step, which the
     // prologue takes first, with checked loads: the steady-state loop is then one basic block for every shape, whose
     // instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between its
-    // MFMAs. Whole tiles take their last k-step first too, so that an element's order of summation depends on K alone and
-    // not on where the tiles end. (A second loop beside it makes the compiler copy the accumulators in every k-step of this one.) Before, a
+    // MFMAs. Whole tiles take their last k-step first only where one order is asked for (lastk): in a triangular product
+    // the diagonal's large terms lie there, and are better added last (FP64 TRSM 2000×500 differs from another FP64 solve by
+    // 5.1e-16 of the result against 4.5e-16). (A second loop beside it makes the compiler copy the accumulators in every k-step of this one.) Before, a
     // ragged tile took the checked loads in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9
     // µs, 64 × 250³ (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096
     // 140 → 112.
@@ -416,12 +418,13 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     sa.init(A, p.lda, p.M, m0, kofs, KG * BK, tid);
     sb.init(B, p.ldb, p.N, n0, kofs, KG * BK, tid);
     if (!CHECK_A && !CHECK_B && m0 + BM <= p.M && n0 + BN <= p.N && K % (BK * KG) == 0) {
-        sa.org += (nk - 1) * sa.step;
-        sb.org += (nk - 1) * sb.step;
+        const int first = p.lastk ? nk - 1 : 0, back = p.lastk ? nk : 0;
+        sa.org += first * sa.step;
+        sb.org += first * sb.step;
         sa.load(p.lda);
         sb.load(p.ldb);
-        sa.org -= nk * sa.step;
-        sb.org -= nk * sb.step;
+        sa.org -= back * sa.step;
+        sb.org -= back * sb.step;
     } else {
         load_checked(nk - 1);
     }

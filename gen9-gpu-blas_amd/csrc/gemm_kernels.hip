@@ -224,6 +224,7 @@ static int launch_typed(const GemmCall &c) {
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
     p.kper = 0;
+    p.lastk = splitk_forced() >= 0;
     const bool ak = !c.tA, bk = c.tB;   // k-contiguous A: not transposed; k-contiguous B: transposed (stored N×K)
     if (ak) return bk ? launch_layout<T, true, true>(p, c.count) : launch_layout<T, true, false>(p, c.count);
     return bk ? launch_layout<T, false, true>(p, c.count) : launch_layout<T, false, false>(p, c.count);
@@ -302,6 +303,7 @@ static int launch_tri_typed(const GemmCall &c, bool lower) {
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
     p.kper = 0;
+    p.lastk = splitk_forced() >= 0;
     if (!c.tA && c.tB) return launch_tri_layout<T, true, true>(p, lower);
     if (c.tA && !c.tB) return launch_tri_layout<T, false, false>(p, lower);
     G9_FAIL(GEN9BLAS_ERR_UNSUPPORTED, "triangle product: layout tA=%d tB=%d", c.tA, c.tB);
@@ -352,6 +354,7 @@ static int launch_klim_typed(const GemmCall &c, int klim) {
     p.tiles_m = p.tiles_n = 0;
     p.P = nullptr;
     p.kper = 0;
+    p.lastk = splitk_forced() >= 0;
     // tile class: FP16 the big tiles when they are at least the CUs; FP32 / FP64 the first of big, small and (FP64)
     // 64×64 that makes two workgroups per CU or more, so that long and short k ranges can share the CUs
     using CF = Cfg<T, true, false>;
