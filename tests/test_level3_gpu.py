@@ -320,6 +320,21 @@ def test_trsm_fp64_leaves_of_1024(g9, torch_dev, n, m):
         assert e <= 1e-12, f"trsm D {side}{uplo} tA={ta} diag={dg} {n}x{m}: {e:.1e}"
 
 
+@pytest.mark.parametrize("kind,dt,bound", [("S", np.float32, 9.5e-8), ("D", np.float64, 3.5e-16)])
+@pytest.mark.parametrize("n,m", [(1300, 50), (700, 96)])
+def test_trmm_adds_the_diagonal_last(g9, torch_dev, kind, dt, bound, n, m):
+    """A lower triangular product with a diagonal of 1 to 2 and small values off it, on shapes that no tiles fill: rows sum
+    their small terms first and the diagonal's last, so that all but one rounding are of small sums. Against 80-bit sums;
+    the bound lies between that order (8.3e-8 and 2.5e-16) and the opposite one (1.09e-7 and 5.0e-16)."""
+    torch, rng = torch_dev, np.random.default_rng(n)
+    A = (np.tril(rng.normal(0, n ** -0.5, (n, n)), -1) + np.diag(rng.uniform(1, 2, n))).astype(dt)
+    B = rng.normal(0, 1, (n, m)).astype(dt)
+    ref = A.astype(np.longdouble) @ B.astype(np.longdouble)
+    X = g9.trmm(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy().astype(np.longdouble)
+    e = float(np.sqrt(((X - ref) ** 2).sum() / (ref ** 2).sum()))
+    assert e <= bound, f"trmm {kind} {n}x{m}: {e:.2e}"
+
+
 def _l3_cases(seed, count):
     """Seeded random level-3 calls: operation, type, side / triangle / transpose / unit diagonal, and dimensions that
     are small (1-79), multiples of 64 (the whole-tile classes of the GEMMs underneath), within 3 of one, or 80-599."""
