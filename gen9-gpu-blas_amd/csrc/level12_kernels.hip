@@ -251,7 +251,7 @@ template <bool NTL, class T> __device__ __forceinline__ Vec<T> vload_a(const T *
 // No-trans, y = alpha·A·x + beta·y: RWN rows per group of KS waves, whose lanes stream 16 bytes of each row per step
 // (1 KiB per row and wave, steps dealt to the waves in turn) and reuse each chunk of x for the RWN rows. The RWN sums
 // are reduced across the wave by the transposing butterfly, the KS waves' sums added in LDS in wave order. U steps per
-// batch. VEC false: an element per lane and step, for short rows, which would leave most lanes of a 16-byte step idle, and
+// batch. VEC false: an element per lane and step, for short FP16 rows, which would leave most lanes of a 16-byte step idle, and
 // for an x with a stride, whose elements the lanes then load side by side.
 // MI355X, µs per call, FP32 unless said; before the 16-byte loads at element alignment (element-wise loads for rows not
 // 16-byte aligned, 16 rows per block throughout) -> now: 6000×1501 10.3 -> 5.8, 6000×1500 6.5 -> 5.8, 1000×8192 13.5 -> 5.3,
@@ -637,11 +637,11 @@ int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll
         // 47 against 40.
         const bool ntl = (double)M * (double)N * sizeof(T) > (double)(256 << 20);
         if (!trans) {
-            // An element per lane: rows of at most 64 of them (FP16: 128), FP32 100000×32 5.4 against 6.2, FP16 ×100 6.1
-            // against 7.9 (×200: 10.2 against 8.1), FP64 1000000×8 47 against 54; and an x with a stride, where rows are
-            // not long nor A large: those have x gathered first. FP16 16384×4096 25 µs (loads of x inside each lane's 16 bytes
-            // instead 39), 8192² gathered 23 (36).
-            bool vec = N > (sizeof(T) == 2 ? 128 : 64);
+            // An element per lane: FP16 rows of at most 128 of them (100000×100 6.1 µs against 7.9, ×200 10.2 against 8.1; FP32
+            // and FP64 rows of up to 64 take 5.4 against 6.2, but their products then round before they are added: 1000×50
+            // 7.1e-8 of the result against 6.2e-8), and an x with a stride, where rows are not long nor A large: those have x
+            // gathered first. FP16 16384×4096 25 µs (loads of x inside each lane's 16 bytes instead 39), 8192² gathered 23 (36).
+            bool vec = sizeof(T) > 2 || N > 128;
             if (vec && ix != 1) {
                 void *g = nullptr;
                 vec = (ntl || N > 2048 * (int)sizeof(T)) && (g = try_scratch(SLOT_P, (size_t)N * sizeof(T)));
