@@ -402,10 +402,10 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     // instruction order is pinned below so the LDS reads, global loads and LDS writes of a k-step run between its
     // MFMAs. Whole tiles take their last k-step first only where one order is asked for (lastk): in a triangular product
     // the diagonal's large terms lie there, and are better added last (FP64 TRSM 2000×500 differs from another FP64 solve by
-    // 5.1e-16 of the result against 4.5e-16). (A second loop beside it makes the compiler copy the accumulators in every k-step of this one.) Before, a
-    // ragged tile took the checked loads in every k-step (element-wise where rows were unaligned): FP32 1000³ 37.4 → 24.9
-    // µs, 64 × 250³ (rows of 1000 bytes) 46.0 → 28.4, FP64 TN 1500×1300×1700 135.7 → 115.4, FP16 NT 1000×11008×4096
-    // 140 → 112.
+    // 5.1e-16 of the result against 4.5e-16). (A second loop beside it makes the compiler copy the accumulators in every
+    // k-step of this one.) Before, a ragged tile took the checked loads in every k-step (element-wise where rows were
+    // unaligned): FP64 TN 1500×1300×1700 135.7 → 115.4 µs; and, on this kernel, which no longer serves them by default, FP32
+    // 1000³ 37.4 → 24.9, 64 × 250³ (rows of 1000 bytes) 46.0 → 28.4, FP16 NT 1000×11008×4096 140 → 112.
     const auto load_checked = [&](int kt) {
         sa.load_checked(A, p.lda, p.M, K, m0, kt * KG * BK + kofs, tid);
         sb.load_checked(B, p.ldb, p.N, K, n0, kt * KG * BK + kofs, tid);
@@ -435,8 +435,8 @@ __global__ void __launch_bounds__(WM *WN * 64 * KG) gemm_kernel(GemmParams<typen
     }
     store(0);
     __syncthreads();
-    // what the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes the compiler wait for
-    // every LDS read of a k-step at once (scalar loads and LDS reads share a counter)
+    // what the epilogue takes from the kernel arguments is loaded here: one still on its way when the loop begins makes the
+    // compiler wait for every LDS read of a k-step at once (scalar loads and LDS reads share a counter)
     asm volatile("" : "+s"(C), "+s"(p.P), "+s"(p.ldc), "+s"(p.M), "+s"(p.N));
     wait_lgkm0();
     // the accumulators' zeros are hidden from the compiler: as one shared constant they cost FP64 tiles 16-64 register
@@ -585,7 +585,7 @@ __device__ __forceinline__ void store4(T *c, const S *v, S alpha, S beta, int va
 }
 
 // Split-K finish: C = alpha·(P[0] + ... + P[splits-1]) + beta·C (C not read when beta = 0), summed in slice order
-// and rounded once to T. One thread per 4 consecutive elements of a row (N % 4 == 0 and aligned C), else per element.
+// and rounded once to T. One thread per 4 consecutive elements of a row (N % 4 == 0), else per element.
 template <class T, class S, bool VEC4>
 __global__ void __launch_bounds__(256) splitk_reduce(const S *__restrict__ P, T *C, long long ldc, int M, int N, int splits,
                                                      S alpha, S beta) {

@@ -12,6 +12,10 @@ namespace g9 {
 // Tile configurations, per element type and layout, from a sweep on MI355X at n = 4096 (every variant checked against
 // a float64 reference). Big: the steady-state configuration. Small: smaller tiles for products whose big tiles
 // would leave most of the 256 CUs idle.
+// FP64 products come here. By default the FP16 ones that do are those with odd strides or unaligned operands and those of
+// at most a k-step of 64, the FP32 ones those of at most a k-step of 32 and short-K NT products and triangles, in both types
+// also rows too far apart for the direct kernels' 32-bit offsets; the rates below are of larger products, as
+// GEN9BLAS_HGEMM / GEN9BLAS_SGEMM=generic and a forced split send them here.
 //   FP16 256×256, 8 waves (4×2): NN 794, NT 950 TFLOP/s. FP64 256×128, 8 waves (4×2): 70.6 TFLOP/s.
 //   FP32 with A k-contiguous: small tiles with 4 waves, many workgroups per CU. NN 64×128: 123 TFLOP/s at n = 4096,
 //   117 at n = 2048 (256×128: 117 / 105; 128×128, 64×64, 128×64, 64×256 and 2- or 8-wave variants: 74-118). NT
@@ -22,7 +26,7 @@ namespace g9 {
 //   FP64 64×128 split two ways 43, 64×64 41. Both are beaten by 64×64 tiles with two k groups (launch_layout).
 struct TileCfg { int BM, BN, WM, WN; };
 // Transposed A, whose staging needs more registers than a wave has at 2 waves per SIMD, keeps FP16 at 4 waves (512
-// registers per wave), which compiles without spills.
+// registers per wave), which still spills 68 (B k-contiguous: 144) bytes per lane.
 template <class T, bool AK, bool BKC> struct Cfg;
 // small_div: the small tile is taken when the big tiles times small_div are fewer than the CUs.
 template <bool AK, bool BKC> struct Cfg<f16, AK, BKC> {
@@ -54,7 +58,8 @@ static int splitk_forced() {
 }
 
 // Split-K slices for a single product of `tiles` tiles: doubled while the slices still leave at most one workgroup
-// per CU and each slice keeps at least 4 k-steps, up to 8. Without a forced split, s > 1 implies tiles · s ≤ CUs.
+// per CU and each slice keeps at least 4 k-steps, up to 8. Without a forced split, s > 1 implies tiles · s ≤ CUs here; the
+// direct kernels split further (choose() in hgemm_launch.h and sgemm_launch.h, by the bytes of the slices).
 // Splitting changes only the FP32 (FP64) summation order: each slice sums its k-range, the slices are then added in
 // order, and alpha/beta and the rounding to the element type are applied once.
 static int splitk_slices(long long tiles, int K, int BK, int count) {
@@ -113,7 +118,7 @@ static int launch_t(GemmParams<typename Mma<T>::Sum> p, int count) {
 }
 
 // FP64 products of few tiles: 32×32 tiles, four k groups of one wave each (73 KiB of LDS, two workgroups per CU), or eight
-// for single products of at most a tile per CU, which split K up to 8 ways before: as many partial sums keep the error
+// (which spill 36 bytes per lane) for single products of at most a tile per CU, which split K up to 8 ways before: as many partial sums keep the error
 // where it was (500×500×512 against 80-bit sums: split K 2.8e-16, four groups 3.8e-16). A
 // wave of a 64×128 or 64×64 tile does 4 to 8 times the MFMAs one after the other while most CUs idle; four k groups hide
 // each other's barrier and load waits, and no second pass adds slices of K.

@@ -6,8 +6,10 @@
 // alpha·sum + beta·C in FP32 (C not read when beta = 0), rounded once to FP16. The MFMA accumulates in FP32, which
 // gives both reference modes (FP16 chains, or FP32 partial sums every 32 products) at least their accuracy.
 //
-// This kernel serves products whose tiles are all full (M % BM = N % BN = K % KB = 0) with 16-byte aligned
-// operands; the general FP16 kernel in gemm_kernel.h takes every other shape. Design:
+// Whole tiles (EDGE false: M % BM = N % BN = K % KB = 0, 16-byte aligned operands) and, with EDGE, tiles that cross the
+// last row or column, any K beyond one k-step and operands at 4-byte alignment with even strides; SPLIT: slices of K whose
+// unscaled sums go to P for split_sum. The general kernel in gemm_kernel.h takes what is left (odd strides, K of at most a
+// k-step, rows too far apart for 32-bit lane offsets). Design:
 // - the matrix-core instruction is v_mfma_f32_16x16x32_f16. It moves a quarter of the accumulator bytes per flop of
 //   v_mfma_f32_32x32x16_f16 (4 instead of 16 FP32 per lane per instruction), and large FP16 products on random data
 //   run at the board's power limit, so the energy per flop sets the rate: a loop of it sustains 1627 TFLOP/s on

@@ -46,8 +46,9 @@ static long long tiles_of(const HgCfg &g, int M, int N) { return (long long)((M 
 struct Choice { int cfg, slices; };
 // The configuration and number of K slices with the smallest estimated time (µs): a launch; rounds of one tile per CU
 // (64×64: two share a CU, one alone takes two thirds of their time), each a fixed part and the tile's time per k, less where
-// part of the chip idles (the board's power limit leaves the rest a higher clock); C written by the larger tiles, which most costs where its rows are
-// not whole 128-byte lines; for slices, the second kernel, its pass over each slice, and the FP32 sums written and read.
+// part of the chip idles (the board's power limit leaves the rest a higher clock); C written by the larger tiles, which
+// costs most where its rows are not whole 128-byte lines; for slices, the second kernel, its pass over each slice, and the
+// FP32 sums written and read.
 // The constants are a fit to the order of 392 products (K 64 to 11008, 17 to 20000 rows, batches, whole and ragged, NN /
 // NT / TN), each timed with every configuration and 1-16 slices on operands in the last-level cache and rotated beyond it:
 // by the geometric mean of both the choice is 0.6 % from the fastest on average, and within 22 % for all. A few (µs,

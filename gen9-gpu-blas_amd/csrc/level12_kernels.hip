@@ -251,8 +251,8 @@ template <bool NTL, class T> __device__ __forceinline__ Vec<T> vload_a(const T *
 // No-trans, y = alpha·A·x + beta·y: RWN rows per group of KS waves, whose lanes stream 16 bytes of each row per step
 // (1 KiB per row and wave, steps dealt to the waves in turn) and reuse each chunk of x for the RWN rows. The RWN sums
 // are reduced across the wave by the transposing butterfly, the KS waves' sums added in LDS in wave order. U steps per
-// batch. VEC false: an element per lane and step, for short FP16 rows, which would leave most lanes of a 16-byte step idle, and
-// for an x with a stride, whose elements the lanes then load side by side.
+// batch. VEC false: an element per lane and step, for short FP16 rows, which would leave most lanes of a 16-byte step idle,
+// and for an x with a stride, whose elements the lanes then load side by side.
 // MI355X, µs per call, FP32 unless said; before the 16-byte loads at element alignment (element-wise loads for rows not
 // 16-byte aligned, 16 rows per block throughout) -> now: 6000×1501 10.3 -> 5.8, 6000×1500 6.5 -> 5.8, 1000×8192 13.5 -> 5.3,
 // 300×40000 75 -> 12, 16384×16383 188 -> 168, FP16 8191×4097 23.2 -> 11.3.
@@ -633,14 +633,15 @@ int launch_gemv(int es, int trans, int M, int N, double alpha, const void *A, ll
         const T *Ap = (const T *)A, *xp = (const T *)x + ox;
         T *yp = (T *)y + oy;
         // A of more than the 256 MiB last-level cache is read past it (nontemporal); a smaller one, which a solver's next
-        // product with it finds there, is not. No-trans, µs, nontemporal against plain loads: FP32 16384×8192 (512 MiB) 104 against 122, 32768×4096 92 against 113; FP64 16384×2048 (256 MiB)
-        // 47 against 40.
+        // product with it finds there, is not. No-trans, µs, nontemporal against plain loads: FP32 16384×8192 (512 MiB) 104
+        // against 122, 32768×4096 92 against 113; FP64 16384×2048 (256 MiB) 47 against 40.
         const bool ntl = (double)M * (double)N * sizeof(T) > (double)(256 << 20);
         if (!trans) {
-            // An element per lane: FP16 rows of at most 128 of them (100000×100 6.1 µs against 7.9, ×200 10.2 against 8.1; FP32
-            // and FP64 rows of up to 64 take 5.4 against 6.2, but their products then round before they are added: 1000×50
-            // 7.1e-8 of the result against 6.2e-8), and an x with a stride, where rows are not long nor A large: those have x
-            // gathered first. FP16 16384×4096 25 µs (loads of x inside each lane's 16 bytes instead 39), 8192² gathered 23 (36).
+            // An element per lane: FP16 rows of at most 128 of them (100000×100 6.1 µs against 7.9, ×200 10.2 against 8.1;
+            // FP32 and FP64 rows of up to 64 take 5.4 against 6.2, but their products then round before they are added:
+            // 1000×50 7.1e-8 of the result against 6.2e-8), and an x with a stride, where rows are not long nor A large:
+            // those have x gathered first. FP16 16384×4096 25 µs (loads of x inside each lane's 16 bytes instead 39), 8192²
+            // gathered 23 (36).
             bool vec = sizeof(T) > 2 || N > 128;
             if (vec && ix != 1) {
                 void *g = nullptr;

@@ -137,11 +137,11 @@ __global__ void __launch_bounds__(256) trsm_store_kernel(const T *Y, T *B, ll ld
 constexpr int TRSM_NB = 128;
 // rows of a leaf (an inverted diagonal block applied by one product) of the FP32 and the FP64 solve: one more
 // composition level and half the leaves for FP64 (n = 4096 left lower, MI355X: 1.427 -> 1.412 ms with 1024 rows
-// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured). FP64 solves of up to TRSM_LEAF_D_FROM rows with fewer
-// than TRSM_LEAF_D_WORK elements of B take 512 too, as one or two leaves do not repay the level (µs, 512 against 1024 rows:
-// 1024×16 91 against 109, 2048×512 165 against 168, 2800×512 273 against 265, 3072×2000 473 against 485); with more the
-// products on whole leaves do (2800×4096 842 against 755, 3000² 874 against 753, 3072×8192 1713 against 1526, 2300×8192 1164
-// against 1134).
+// against 512; FP32 stays at 512: 0.729 against 0.823 ms when measured). FP64 solves of up to TRSM_LEAF_D_FROM rows with
+// fewer than TRSM_LEAF_D_WORK elements of B take 512 too, as one or two leaves do not repay the level (µs, 512 against 1024
+// rows: 1024×16 91 against 109, 2048×512 165 against 168, 2800×512 273 against 265, 3072×2000 473 against 485); with more
+// the products on whole leaves do (2800×4096 842 against 755, 3000² 874 against 753, 3072×8192 1713 against 1526,
+// 2300×8192 1164 against 1134).
 constexpr int TRSM_LEAF_S = 512, TRSM_LEAF_D = 1024, TRSM_LEAF_D_FROM = 3072, TRSM_LEAF_D_WORK = 9000000;
 static int trsm_leaf(int es, int n, int m) {
     if (es == 8 && (n > TRSM_LEAF_D_FROM || (n > 2 * TRSM_LEAF_D && (ll)n * m >= TRSM_LEAF_D_WORK))) return TRSM_LEAF_D;

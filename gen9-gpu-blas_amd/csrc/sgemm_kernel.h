@@ -5,7 +5,8 @@
 // gen9blas_epilog_fb): every C element is the sum over k of the A·B products in FP32, then alpha·sum + beta·C (C not
 // read when beta = 0).
 //
-// This kernel serves products of more than one k-step of 32; the general kernel in gemm_kernel.h takes the others.
+// This kernel serves products of more than one k-step of 32, but for the short-K NT products and triangles that C bounds;
+// those, the shorter ones and rows too far apart for 32-bit lane offsets stay on the general kernel in gemm_kernel.h.
 // Design (the FP16 kernel's of hgemm_kernel.h, for FP32):
 // - operand tiles go from global memory straight into LDS with global_load_lds_dwordx4, through the FP16 kernel's
 //   loaders (an FP32 tile seen as FP16 pairs: a k-contiguous row of 32 FP32 is one of 64 FP16); NS LDS stages of

@@ -1,7 +1,8 @@
 // Host side of the FP32 GEMM on direct global→LDS loads (sgemm_kernel.h): which products it takes, their tiles and their
 // split of K, the triangle and k-limited modes of the level-3 routines. Part of gemm_kernels.hip.
-// Against the general kernel (µs): 1000³ 37.4 → 25.0, 64 × 250³ 46.1 → 27.7, 141×3840×3712 TN 205 → 60, 6192×192×5910 NT
-// 413 → 143, 1512×362×738 43.4 → 19.5.
+// Against the general kernel that served ragged products before, with checked loads in every k-step and whole-tile interiors
+// (µs): 1000³ 37.4 → 25.0, 64 × 250³ 46.1 → 27.7, 141×3840×3712 TN 205 → 60, 6192×192×5910 NT 413 → 143, 1512×362×738
+// 43.4 → 19.5.
 //
 // Tile configurations, with rates on MI355X (TFLOP/s, sustained): 128×256, 8 waves of 64×64, two stages, sums blocked per
 // 128 k: n = 4096 NN 144.9, NT 144.3, 8192×8192×2048 144.1 (three stages 142.6; blocks of 32 k 134.3, 64 k 140.3, 256 k
@@ -43,8 +44,9 @@ static double cost(const SgCfg &g, long long tiles, int kper, int ns) {
     if (ns > 1) t += 0.8 + (double)(ns * tiles) * g.BM * g.BN * 8 / 1e7;
     return t;
 }
-// The cheapest configuration and split of K into slices that fit `work` bytes; tri: the tiles of a triangle of side M (square tiles only); big: 128×256 tiles
-// may be taken (their edge-capable variant would need more registers than a wave has).
+// The cheapest configuration and split of K into slices that fit `work` bytes; tri: the tiles of a triangle of side M
+// (square tiles only); big: 128×256 tiles may be taken (their edge-capable variant would need more registers than a wave
+// has).
 static Choice choose(const GemmCall &c, size_t work, bool tri, bool big) {
     static constexpr int SLICES[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
     Choice best{2, 1, 1e30};
@@ -166,7 +168,8 @@ static int whole_block(const GemmCall &c) {
     }
     return 0;
 }
-static sg::Params sg_work(const GemmCall &c, bool batch, size_t &work) {   // parameters, with the work space of split products
+// Parameters, with the work space of split products.
+static sg::Params sg_work(const GemmCall &c, bool batch, size_t &work) {
     sg::Params p = sg_params(c);
     work = 0;
     if (batch) return p;

@@ -33,7 +33,7 @@ GEN9BLAS_API int gen9blas_flush(void);
 // device memory (tight serving loops, harnesses that forbid hipMalloc). Same arguments, kernels and results as
 // gen9blas_gemm, but A, B and C must be device memory (an operand in host memory would need staging buffers:
 // INVALID_ARG before anything runs), and the work space is a static 64 MiB device array per GPU: enough for the
-// split-K slices of every default dispatch on MI355X (CUs × the largest split tile) and for the skinny products
+// split-K slices of every default dispatch on MI355X (no split is chosen that needs more) and for the skinny products
 // (min(M, N) ≤ 16: a transposed small operand gathered, M·K elements; the K-split partial sums of weights stored
 // K×N, at most 4 MiB). A product that would need more (a split forced by GEN9BLAS_SPLITK, or a skinny product whose
 // M·K·element size passes about 60 MiB) gives INVALID_ARG before any launch. It runs on the library stream like every call and
