@@ -4,9 +4,9 @@ Same kernels and dispatch as gen9blas_gemm, so on the same device operands the r
 bit: products that take split-K (whose slices then live in the entry point's static work space), the two-k-group
 tiles and the whole-tile FP16 kernel, in every type, two calls in a row with the second smaller (the work space
 keeps the last call's contents; a split-K slice writes every element it is later read at). The largest default
-splits are included: FP16 2048×4096×1000 (128 general-kernel tiles of 256×256 split two ways: the whole 64 MiB),
-FP64 640×640×1024 (split four ways) and FP16
-1280×1280×1000 on the general kernel. Skinny products whose gathered operand and partial sums live in that work
+splits are included: FP16 and FP32 1280×4352 (256×256 tiles, K = 8192, and 128×128 tiles, K = 4096, in three slices:
+63.75 MiB), beside products of a few hundred tiles that no longer split or split less (FP16 2048×4096×1000, FP64
+640×640×1024, FP16 1280×1280×1000). Skinny products whose gathered operand and partial sums live in that work
 space are included too. Both are also held to the GEMM bounds against float64. Host operands (checked
 before any dispatch, so the staging paths never run) and a work space beyond the fixed maximum give INVALID_ARG
 before any launch (the latter needs a split forced with GEN9BLAS_SPLITK, read once per process: a child process).
@@ -63,8 +63,8 @@ CASES = [((200, 136, 1000, 0, 0), (100, 72, 500, 1, 1)),
 # sums in the work space) and a transposed small operand (gathered into the work space), the second call smaller
 SKINNY = [((4, 4096, 4096, 0, 0), (16, 2048, 1024, 1, 0)),
           ((4096, 8, 2048, 0, 0), (1000, 3, 512, 1, 1))]
-# the largest default work spaces: 64 MiB (FP16 2048×4096×1000), then 12.5 MiB (FP64 640×640×1024, FP16
-# 1280×1280×1000); FP64 2048³, whose big tiles are half the CUs, takes the small tiles instead of a split
+# products of many tiles: FP64 2048³, whose big tiles are half the CUs, takes the small tiles instead of a split, FP64
+# 640×640×1024 32×32 tiles with k groups; the FP16 ones take the direct kernel, at most a few slices
 LARGE = {"D": ((2048, 2048, 2048, 0, 0), (640, 640, 1024, 1, 0)),
          "H": ((2048, 4096, 1000, 0, 0), (1280, 1280, 1000, 0, 1)),
          "HS": ((1280, 1280, 1000, 1, 1), (1000, 600, 1000, 0, 0))}
@@ -101,6 +101,16 @@ def test_noalloc_skinny(g9, torch_dev, kind, pair):
 @pytest.mark.parametrize("kind", sorted(LARGE))
 def test_noalloc_largest_work_space(g9, torch_dev, kind):
     _compare(g9, torch_dev, kind, LARGE[kind], 50)
+
+
+# the largest default splits: three slices of 85 tiles of 256×256 (FP16), of 340 tiles of 128×128 (FP32), 63.75 MiB
+SPLIT = {"H": ((1280, 4352, 8192, 0, 1), (200, 136, 1000, 0, 0)),
+         "S": ((1280, 4352, 4096, 0, 0), (200, 136, 1000, 1, 0))}
+
+
+@pytest.mark.parametrize("kind", sorted(SPLIT))
+def test_noalloc_largest_split(g9, torch_dev, kind):
+    _compare(g9, torch_dev, kind, SPLIT[kind], 51)
 
 
 def test_noalloc_rejects_host_operands(g9):
